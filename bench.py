@@ -443,7 +443,7 @@ def fit_bench(dev, chunks=3, rows=65536, d=4096, targets=16, lams=(1e-4, 1e-3, 1
         del x, ys
     steady = sum(times[1:]) / max(1, len(times) - 1)
     flop = 2.0 * rows * d * d * (1 + targets)
-    tiles = -(-(d + 2 * stats.cen_x.s) // 256)
+    tiles = d // 256
     flop_exec = 2.0 * rows * d * d * targets + 2.0 * rows * 256 * 256 * (tiles * tiles - tiles * (tiles - 1) // 2)
     t0 = time.perf_counter()
     fit = ridge.RidgeFit(stats.state(device=dev), device=dev)

@@ -438,6 +438,43 @@ int rf_gram_accumulate_upper(const uint16_t* a, int64_t lda, int64_t M, int64_t 
 /* Workspace bytes of rf_gram_accumulate_upper's run-split schedule for this shape (0: it uses none). */
 int rf_gram_upper_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t fold_rows, size_t* bytes);
 
+/* The Gram of centred operands (rf_transpose_centred): A [da + ea, K] and B [db + eb, K], da / db main rows
+ * (multiples of 256) and ea / eb extra rows (the mid and lo parts of centred channels; even, at most 256):
+ * C[i, j] += sum_k A[i, k] B[j, k] for i < da + ea, j < db + eb (code/kva/ridge.py:47, :62). The main product runs
+ * as rf_gram_accumulate's (upper: rf_gram_accumulate_upper's, with b == a: main block-upper tiles, and the extra
+ * columns of every row; the extra rows' main columns are their mirror and are not written); the extra rows run as
+ * products of few rows over split K ranges of at most fold_rows, each split's fp32 sums added into C in fp64.
+ * init: C's old values count as zeros and need not be initialised. Other columns of C are not touched. Needs the
+ * workspace of rf_gram_centred_workspace_bytes; limits as rf_gram_accumulate. */
+int rf_gram_centred(const uint16_t* a, int64_t lda, int64_t da, int64_t ea, const uint16_t* b, int64_t ldb, int64_t db,
+                    int64_t eb, int64_t K, int64_t fold_rows, double* c, int64_t ldc, int upper, int init,
+                    void* workspace, size_t ws_bytes, hipStream_t stream);
+int rf_gram_centred_workspace_bytes(int64_t da, int64_t ea, int64_t db, int64_t eb, int64_t K, int64_t fold_rows,
+                                    int upper, size_t* bytes);
+
+/* One product of RidgeStats.state() (code/kva/ridge.py:70-74) from the augmented Gram G [ca + 2 sa, >= cb + 2 sb] of
+ * rf_gram_centred, in one pass: out[r, c] = the sum of channel r's and c's parts (main, mid, lo; lo_a / lo_b: int32
+ * rows among the centred channels or -1, as rf_transpose_centred's lo_row) - da[r] s1b[c] - s1a[r] db[c]
+ * + n da[r] db[c]: the sums moved from the stored shifts by da / db. upper (ca == cb, sa == sb): G holds its
+ * block-upper 256 x 256 tiles only and is symmetric. */
+int rf_gram_state(const double* g, int64_t ldg, int64_t ca, int64_t sa, const int32_t* lo_a, int64_t cb, int64_t sb,
+                  const int32_t* lo_b, int upper, const double* s1a, const double* s1b, const double* da,
+                  const double* db, double n, double* out, int64_t ldo, hipStream_t stream);
+
+/* Per-64-row sums and sums of squares of src [rows, cols] bf16 (both [ceil(rows / 64), cols] fp32): the partials
+ * that rf_transpose_centred without a shift gives, without the transpose. */
+int rf_col_moments(const uint16_t* src, int64_t ld_src, int64_t rows, int64_t cols, float* partial, float* partial_sq,
+                   hipStream_t stream);
+
+/* The centring of an operand from its sums s1 / sums of squares s2 over n rows (the shifts of
+ * code/kva/ridge.py:37-38): c [cols] = the mean rounded to fp32, or `given`; centred are the channels with c^2 >
+ * variance, at most cap of them (largest ratio first, lower channel first among equals). shift [cols] fp32 = c of a
+ * centred channel, else 0; lo_row [cols] = its index among the centred ones in channel order, else -1; delta =
+ * c - shift; idx [cap] = the centred channels in order, count = their number. scratch: [cols] fp64. */
+int rf_centre_select(const double* s1, const double* s2, double n, const double* given, int64_t cols, int64_t cap,
+                     double* c, float* shift, int32_t* lo_row, double* delta, int64_t* idx, int32_t* count,
+                     double* scratch, hipStream_t stream);
+
 /* Held-out read cosine of one late layer for one document (code/scripts/fit_sweep.py:307-313): pred and
  * truth are [rows, >= (na + nb) d] bf16 reads, each row na vectors of group a then nb vectors of group b,
  * each d wide. An attention layer's reads are its pre-RoPE K and V (code/kva/model.py:282-287, one

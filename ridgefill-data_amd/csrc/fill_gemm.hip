@@ -341,7 +341,7 @@ __device__ __forceinline__ void wait_steps(int n) {
 template <int RT>
 __device__ __forceinline__ void rows_partial(const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ W,
                                              int64_t ldw, int M, int N, int K, int kper, int rblocks,
-                                             float* __restrict__ part, uint4* lds) {
+                                             float* __restrict__ part, uint4* lds, int bid, int nblocks, int wrows) {
   using C = RowsCfg<RT>;
   static_assert(C::S >= 3 && (C::S - 2) * C::L < 64, "ring depth");
   const int t = threadIdx.x, lane = t & 63;
@@ -350,7 +350,7 @@ __device__ __forceinline__ void rows_partial(const uint16_t* __restrict__ X, int
   // per XCD: the row blocks of one column block run together on one XCD, so its weight rows are read
   // from memory once and meet in that XCD's L2
   const int cblocks = N / RN;
-  const int u = xcd_tile(blockIdx.x, gridDim.x);
+  const int u = xcd_tile(bid, nblocks);
   const int rbk = u % rblocks, rest = u / rblocks;
   const int cb = rest % cblocks, sp = rest / cblocks;
   // row blocks of about equal size, each a whole number of row tiles
@@ -362,7 +362,7 @@ __device__ __forceinline__ void rows_partial(const uint16_t* __restrict__ X, int
   const __amdgpu_buffer_rsrc_t rx = buffer_rsrc(X + static_cast<int64_t>(m0) * ldx + kbeg,
                                                 static_cast<uint32_t>(rows_x * ldx * 2));
   const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(W + static_cast<int64_t>(n0) * ldw + kbeg,
-                                                static_cast<uint32_t>(RN * ldw * 2));
+                                                static_cast<uint32_t>(min(wrows - n0, RN) * ldw * 2));
   // load i of this wave: stage rows 8 (4 i + w) .. + 7 (activation rows below MT, then weight rows);
   // lane L fetches row + L / 8, logical chunk (L % 8) ^ slot_swz(row) into physical chunk L % 8
   uint32_t voff[C::L];
@@ -463,7 +463,7 @@ __global__ __launch_bounds__(NTHR) void k_rows_partial(const uint16_t* __restric
                                                        const uint16_t* __restrict__ W, int64_t ldw, int M, int N,
                                                        int K, int kper, int rblocks, float* __restrict__ part) {
   __shared__ uint4 lds[RowsCfg<RT>::S * RowsCfg<RT>::STAGE_U4];
-  rows_partial<RT>(X, ldx, W, ldw, M, N, K, kper, rblocks, part, lds);
+  rows_partial<RT>(X, ldx, W, ldw, M, N, K, kper, rblocks, part, lds, blockIdx.x, gridDim.x, N);
 }
 
 // The split sums of 8 consecutive columns col .. col + 7 of row gm: 8 fp32 values, splits added in order.
@@ -981,9 +981,10 @@ __global__ __launch_bounds__(256) void k_norm_kv_reduce(const float* __restrict_
 // through LDS, half the tile (128 rows) at a time, as a row-major fp32 image (row r's 16-byte chunk c at
 // r * 64 + (c ^ (r & 15)): the accumulator writes and the row reads both hit 16 distinct bank groups per
 // 16 lanes), so that each wave instruction of the read-modify-write of C covers 2 KB of one row of C instead
-// of 16 bytes in each of 32 rows. Needs the LDS free on entry; leaves it free.
+// of 16 bytes in each of 32 rows. With `init` (block-uniform) C's old values count as zeros and are not
+// read. Needs the LDS free on entry; leaves it free.
 __device__ __forceinline__ void fold_tile(const f32x16 (&acc)[4][4], uint4* lds, double* __restrict__ C,
-                                          int64_t ldc, int M, int m0, int n0) {
+                                          int64_t ldc, int M, int m0, int n0, bool init) {
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wm = w >> 1, wn = w & 1, lr = lane & 31, lk = lane >> 5;
@@ -1013,8 +1014,8 @@ __device__ __forceinline__ void fold_tile(const f32x16 (&acc)[4][4], uint4* lds,
       for (int i = 0; i < 8; ++i) {
         const int gm = min(m0 + h * 128 + w * 32 + b * 8 + i, M - 1);
         const double* p = C + static_cast<int64_t>(gm) * ldc + n0 + 4 * lane;
-        d[i][0] = *reinterpret_cast<const double2*>(p);
-        d[i][1] = *reinterpret_cast<const double2*>(p + 2);
+        d[i][0] = init ? make_double2(0.0, 0.0) : *reinterpret_cast<const double2*>(p);
+        d[i][1] = init ? make_double2(0.0, 0.0) : *reinterpret_cast<const double2*>(p + 2);
       }
     };
     load_batch(0, v[0]);
@@ -1086,6 +1087,7 @@ struct GramPlan {
   int ptiles, runs;
   float* part;
   int upper;              // the logical tiles are C's block-upper tiles only (gram_coords)
+  int init;               // C's old values count as zeros: the first run's sums are stored, not added
 };
 
 // Logical tile -> (tile row, tile column) of a Gram launch: tile_coords over every tile, or with `upper` the
@@ -1130,14 +1132,15 @@ __global__ __launch_bounds__(NTHR) void k_gram(const uint16_t* __restrict__ A, i
   for (int k0 = 0; k0 < K; k0 += fold) {
     const int k1 = min(k0 + fold, K);
     mainloop(A + k0, lda, B + k0, ldb, M, k1 - k0, m0, n0, lds, acc);
-    fold_tile(acc, lds, C, ldc, M, m0, n0);
+    fold_tile(acc, lds, C, ldc, M, m0, n0, pl.init && k0 == 0);
   }
 }
 
 // C += the stored runs of the last ptiles logical tiles (GramPlan), each tile's runs in run order: block =
 // 4 rows of one tile, thread = 4 consecutive columns (whole 1 KB rows of the planes, 2 KB rows of C).
 __global__ __launch_bounds__(256) void k_gram_fold(const float* __restrict__ part, int ptiles, int runs, int whole,
-                                                   int M, int N, double* __restrict__ C, int64_t ldc, int upper) {
+                                                   int M, int N, double* __restrict__ C, int64_t ldc, int upper,
+                                                   int init) {
   const int t = blockIdx.x >> 6, row = (blockIdx.x & 63) * 4 + (threadIdx.x >> 6), c4 = threadIdx.x & 63;
   if (t >= ptiles) return;
   int tm, tn;
@@ -1145,7 +1148,11 @@ __global__ __launch_bounds__(256) void k_gram_fold(const float* __restrict__ par
   const int gm = tm * BM + row;
   if (gm >= M) return;
   double* p = C + static_cast<int64_t>(gm) * ldc + tn * BN + 4 * c4;
-  double2 v0 = *reinterpret_cast<const double2*>(p), v1 = *reinterpret_cast<const double2*>(p + 2);
+  double2 v0 = make_double2(0.0, 0.0), v1 = v0;
+  if (!init) {
+    v0 = *reinterpret_cast<const double2*>(p);
+    v1 = *reinterpret_cast<const double2*>(p + 2);
+  }
   const float* q = part + (static_cast<int64_t>(t) * runs * BM + row) * BN + 4 * c4;
   for (int r = 0; r < runs; ++r) {
     const float4 a = *reinterpret_cast<const float4*>(q + static_cast<int64_t>(r) * BM * BN);
@@ -1156,6 +1163,58 @@ __global__ __launch_bounds__(256) void k_gram_fold(const float* __restrict__ par
   }
   *reinterpret_cast<double2*>(p) = v0;
   *reinterpret_cast<double2*>(p + 2) = v1;
+}
+
+// The extra rows of a centred Gram (rf_gram_centred). A main product of 4096 x 4096 is 256 tiles, exactly one
+// round of the CUs; the few mid and lo rows of centred channels (2 per channel, usually 8 or 16) would add a
+// tile row and a tile column that are nearly all padding, i.e. a second round. They run here instead, as two
+// products with few rows (rows_partial): the row strip, A's ea extra rows against every B row, and the column
+// strip, B's eb extra rows against A's main rows (its planes are the transposed strip). Their K range is
+// split over the CUs; k_strip_fold adds the splits' fp32 sums into C in fp64, in split order. Measured at
+// 4096 x 4096 main, 16 extra rows each over K = 8190: main product 254 us, strips 21 us (the operands read once
+// more, 138 MB) and their fold 7 us, against 383 us for the augmented product as 289 tiles.
+struct StripJob {
+  const uint16_t* x;      // few rows
+  const uint16_t* w;      // wrows rows, N = wrows rounded up to 256
+  int64_t ldx, ldw;
+  int m, n, wrows, rblocks, blocks;
+  float* part;            // [splits][m][n]
+};
+template <int RT>
+__global__ __launch_bounds__(NTHR) void k_gram_strips(StripJob j0, StripJob j1, int K, int kper) {
+#ifdef __HIP_DEVICE_COMPILE__   // (the host pass rejects a second instantiation of rows_partial's buffer builtins)
+  __shared__ uint4 lds[RowsCfg<RT>::S * RowsCfg<RT>::STAGE_U4];
+  const bool second = static_cast<int>(blockIdx.x) >= j0.blocks;   // block-uniform
+  const StripJob j = second ? j1 : j0;
+  const int bid = static_cast<int>(blockIdx.x) - (second ? j0.blocks : 0);
+  rows_partial<RT>(j.x, j.ldx, j.w, j.ldw, j.m, j.n, K, kper, j.rblocks, j.part, lds, bid, j.blocks, j.wrows);
+#endif
+}
+
+// C[da + r, c] += sum_s p0[s][r][c] (r < ea, c < nb) and C[m, db + j] += sum_s p1[s][j][m] (j < eb, m < da),
+// each in split order; with init C's old values count as zeros. Blocks [0, b0) take 256 columns of a row of
+// the row strip each, the rest 64 rows x 4 interleaved column groups of the column strip.
+__global__ __launch_bounds__(256) void k_strip_fold(const float* __restrict__ p0, int n0, int ea, int nb,
+                                                    const float* __restrict__ p1, int n1, int eb, int da, int db,
+                                                    int splits, int b0, double* __restrict__ C, int64_t ldc, int init) {
+  const int t = threadIdx.x;
+  if (static_cast<int>(blockIdx.x) < b0) {
+    const int per = n0 / 256, r = blockIdx.x / per, c = (blockIdx.x - r * per) * 256 + t;
+    if (c >= nb) return;
+    double* p = C + static_cast<int64_t>(da + r) * ldc + c;
+    double v = init ? 0.0 : *p;
+    for (int s = 0; s < splits; ++s) v += static_cast<double>(p0[(static_cast<int64_t>(s) * ea + r) * n0 + c]);
+    *p = v;
+    return;
+  }
+  const int m = (blockIdx.x - b0) * 64 + (t & 63);
+  if (m >= da) return;
+  for (int j = t >> 6; j < eb; j += 4) {
+    double* p = C + static_cast<int64_t>(m) * ldc + db + j;
+    double v = init ? 0.0 : *p;
+    for (int s = 0; s < splits; ++s) v += static_cast<double>(p1[(static_cast<int64_t>(s) * eb + j) * n1 + m]);
+    *p = v;
+  }
 }
 
 // The MFMA throughput the power budget allows: back-to-back v_mfma_f32_32x32x16_bf16 on register operands,
@@ -2346,7 +2405,7 @@ static int gram_workspace(const char* who, int64_t M, int64_t N, int64_t K, int6
 
 static int gram_launch(const char* who, const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb, int64_t M,
                        int64_t N, int64_t K, int64_t fold_rows, double* c, int64_t ldc, void* workspace,
-                       size_t workspace_bytes, bool upper, hipStream_t stream) {
+                       size_t workspace_bytes, bool upper, bool init, hipStream_t stream) {
   if (!a || !b || !c) return fail(RF_EINVAL_ARG, "%s: null pointer", who);
   if (M < 0 || M > (1 << 30) || N <= 0 || N % BN || K <= 0 || K % 64 || (upper && M > N))
     return fail(RF_EINVAL_SHAPE, "%s: M %lld, N %lld (multiple of 256%s), K %lld (multiple of 64)", who,
@@ -2362,11 +2421,11 @@ static int gram_launch(const char* who, const uint16_t* a, int64_t lda, const ui
   const int64_t fold = (fold_rows == 0 || fold_rows > K) ? K : fold_rows;
   const GramShape g = gram_shape(M, N, K, fold_rows, upper);
   const size_t need = static_cast<size_t>(g.ptiles * g.runs) * BM * BN * sizeof(float);
-  GramPlan pl{0, 0, 1, nullptr, upper ? 1 : 0};
+  GramPlan pl{0, 0, 1, nullptr, upper ? 1 : 0, init ? 1 : 0};
   if (g.ptiles > 0 && workspace && workspace_bytes >= need) {     // else every tile whole (same bits)
     if (!aligned16(workspace)) return fail(RF_EINVAL_ARG, "%s: workspace must be 16-byte aligned", who);
     pl = GramPlan{static_cast<int>((g.ptiles * g.runs + 7) / 8 * 8), static_cast<int>(g.ptiles),
-                  static_cast<int>(g.runs), static_cast<float*>(workspace), upper ? 1 : 0};
+                  static_cast<int>(g.runs), static_cast<float*>(workspace), upper ? 1 : 0, init ? 1 : 0};
   }
   const int grid = static_cast<int>(g.tiles - pl.ptiles) + pl.pieces;
   hipLaunchKernelGGL(k_gram, dim3(grid), dim3(NTHR), 0, stream, a, lda, b, ldb, static_cast<int>(M),
@@ -2376,7 +2435,7 @@ static int gram_launch(const char* who, const uint16_t* a, int64_t lda, const ui
     if (rc != RF_OK) return rc;
     hipLaunchKernelGGL(k_gram_fold, dim3(pl.ptiles * 64), dim3(256), 0, stream, pl.part, pl.ptiles, pl.runs,
                        static_cast<int>(g.tiles - pl.ptiles), static_cast<int>(M), static_cast<int>(N), c, ldc,
-                       pl.upper);
+                       pl.upper, pl.init);
   }
   return check_launch(who);
 }
@@ -2389,7 +2448,7 @@ extern "C" int rf_gram_accumulate(const uint16_t* a, int64_t lda, const uint16_t
                                   int64_t N, int64_t K, int64_t fold_rows, double* c, int64_t ldc, void* workspace,
                                   size_t workspace_bytes, hipStream_t stream) {
   return gram_launch("rf_gram_accumulate", a, lda, b, ldb, M, N, K, fold_rows, c, ldc, workspace, workspace_bytes,
-                     false, stream);
+                     false, false, stream);
 }
 
 extern "C" int rf_gram_upper_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t fold_rows, size_t* bytes) {
@@ -2400,7 +2459,98 @@ extern "C" int rf_gram_accumulate_upper(const uint16_t* a, int64_t lda, int64_t 
                                         int64_t fold_rows, double* c, int64_t ldc, void* workspace,
                                         size_t workspace_bytes, hipStream_t stream) {
   return gram_launch("rf_gram_accumulate_upper", a, lda, a, lda, M, N, K, fold_rows, c, ldc, workspace,
-                     workspace_bytes, true, stream);
+                     workspace_bytes, true, false, stream);
+}
+
+// The strips of rf_gram_centred: row blocks of at most 160 rows, K split so that about one block runs per CU,
+// no split longer than a fold run.
+struct StripPlan {
+  int rt, rb0, rb1, kper, splits;
+  int64_t n0, n1;
+  size_t bytes;
+};
+static StripPlan strip_plan(int64_t da, int64_t ea, int64_t db, int64_t eb, int64_t K, int64_t fold, bool upper) {
+  StripPlan p{};
+  const int64_t rows0 = upper ? 0 : ea;             // upper: the row strip but its corner is the column strip's mirror
+  p.n0 = rows0 ? (db + eb + 255) / 256 * 256 : 0;
+  p.n1 = eb ? (upper ? (da + ea + 255) / 256 * 256 : da) : 0;
+  p.rb0 = static_cast<int>((rows0 + 159) / 160);
+  p.rb1 = static_cast<int>((eb + 159) / 160);
+  const int64_t per0 = p.rb0 ? (rows0 + p.rb0 - 1) / p.rb0 : 0, per1 = p.rb1 ? (eb + p.rb1 - 1) / p.rb1 : 0;
+  p.rt = static_cast<int>((std::max(per0, per1) + 31) / 32);
+  const int64_t blocks = p.rb0 * (p.n0 / RN) + p.rb1 * (p.n1 / RN);
+  if (blocks == 0) return p;
+  const int64_t want = std::max<int64_t>(std::min<int64_t>(std::min<int64_t>(256 / blocks, K / 512), 16), 1);
+  p.kper = static_cast<int>(std::min<int64_t>(((K + want - 1) / want + BK - 1) / BK * BK, fold));
+  p.splits = static_cast<int>((K + p.kper - 1) / p.kper);
+  p.bytes = static_cast<size_t>(p.splits) * (rows0 * p.n0 + eb * p.n1) * 4;
+  return p;
+}
+
+static int gram_centred_check(const char* who, int64_t da, int64_t ea, int64_t db, int64_t eb, int64_t K,
+                              int64_t fold_rows, int upper) {
+  if (da <= 0 || da % BM || db <= 0 || db % BN || ea < 0 || ea > 256 || eb < 0 || eb > 256 || ea % 2 || eb % 2 ||
+      da > (1 << 24) || db > (1 << 24) || K <= 0 || K % 64 || fold_rows < 0 || fold_rows % 64 ||
+      (upper && (da != db || ea != eb)))
+    return fail(RF_EINVAL_SHAPE, "%s: main rows %lld / %lld (multiples of 256), extra rows %lld / %lld (even, <= 256), "
+                "K %lld and fold_rows %lld (multiples of 64)%s", who, (long long)da, (long long)db, (long long)ea,
+                (long long)eb, (long long)K, (long long)fold_rows, upper ? ", equal sides" : "");
+  return RF_OK;
+}
+
+extern "C" int rf_gram_centred_workspace_bytes(int64_t da, int64_t ea, int64_t db, int64_t eb, int64_t K,
+                                               int64_t fold_rows, int upper, size_t* bytes) {
+  const char* who = "rf_gram_centred_workspace_bytes";
+  if (!bytes) return fail(RF_EINVAL_ARG, "%s: null pointer", who);
+  if (int rc = gram_centred_check(who, da, ea, db, eb, K, fold_rows, upper)) return rc;
+  const int64_t fold = (fold_rows == 0 || fold_rows > K) ? K : fold_rows;
+  size_t main = 0;
+  if (int rc = gram_workspace(who, da, db, K, fold_rows, upper != 0, &main)) return rc;
+  *bytes = std::max(main, strip_plan(da, ea, db, eb, K, fold, upper != 0).bytes);
+  return RF_OK;
+}
+
+extern "C" int rf_gram_centred(const uint16_t* a, int64_t lda, int64_t da, int64_t ea, const uint16_t* b, int64_t ldb,
+                               int64_t db, int64_t eb, int64_t K, int64_t fold_rows, double* c, int64_t ldc, int upper,
+                               int init, void* workspace, size_t ws_bytes, hipStream_t stream) {
+  const char* who = "rf_gram_centred";
+  if (!a || !b || !c) return fail(RF_EINVAL_ARG, "%s: null pointer", who);
+  if (int rc = gram_centred_check(who, da, ea, db, eb, K, fold_rows, upper)) return rc;
+  if (upper && (a != b || lda != ldb)) return fail(RF_EINVAL_ARG, "%s: upper needs b == a", who);
+  if (ldc < db + eb) return fail(RF_EINVAL_SHAPE, "%s: ldc %lld", who, (long long)ldc);
+  const int64_t fold = (fold_rows == 0 || fold_rows > K) ? K : fold_rows;
+  const StripPlan sp = strip_plan(da, ea, db, eb, K, fold, upper != 0);
+  if (sp.bytes && (!workspace || !aligned16(workspace) || ws_bytes < sp.bytes))
+    return fail(RF_EINVAL_ARG, "%s: workspace %zu bytes (16-byte aligned), needs %zu", who, ws_bytes, sp.bytes);
+  if (int rc = gram_launch(who, a, lda, b, ldb, da, db, K, fold_rows, c, ldc, workspace, ws_bytes, upper != 0,
+                           init != 0, stream))
+    return rc;
+  if (!sp.bytes) return RF_OK;
+  // (the strips reuse the workspace after the main launch's fold, in stream order)
+  const int64_t rows0 = upper ? 0 : ea;
+  float* part0 = static_cast<float*>(workspace);
+  float* part1 = part0 + static_cast<int64_t>(sp.splits) * rows0 * sp.n0;
+  const int64_t arows = upper ? da + ea : da;       // rows of A the column strip covers
+  const StripJob j0{a + da * lda, b, lda, ldb, static_cast<int>(rows0), static_cast<int>(sp.n0),
+                    static_cast<int>(db + eb), sp.rb0, static_cast<int>(sp.rb0 * (sp.n0 / RN) * sp.splits), part0};
+  const StripJob j1{b + db * ldb, a, ldb, lda, static_cast<int>(eb), static_cast<int>(sp.n1), static_cast<int>(arows),
+                    sp.rb1, static_cast<int>(sp.rb1 * (sp.n1 / RN) * sp.splits), part1};
+  const dim3 grid(static_cast<unsigned>(j0.blocks + j1.blocks));
+  const int k = static_cast<int>(K);
+  switch (sp.rt) {
+    case 1: hipLaunchKernelGGL(k_gram_strips<1>, grid, dim3(NTHR), 0, stream, j0, j1, k, sp.kper); break;
+    case 2: hipLaunchKernelGGL(k_gram_strips<2>, grid, dim3(NTHR), 0, stream, j0, j1, k, sp.kper); break;
+    case 3: hipLaunchKernelGGL(k_gram_strips<3>, grid, dim3(NTHR), 0, stream, j0, j1, k, sp.kper); break;
+    case 4: hipLaunchKernelGGL(k_gram_strips<4>, grid, dim3(NTHR), 0, stream, j0, j1, k, sp.kper); break;
+    default: hipLaunchKernelGGL(k_gram_strips<5>, grid, dim3(NTHR), 0, stream, j0, j1, k, sp.kper); break;
+  }
+  if (int rc = check_launch(who)) return rc;
+  const int b0 = static_cast<int>(rows0 * (sp.n0 / 256)), b1 = eb ? static_cast<int>((arows + 63) / 64) : 0;
+  hipLaunchKernelGGL(k_strip_fold, dim3(b0 + b1), dim3(256), 0, stream, part0, static_cast<int>(sp.n0),
+                     static_cast<int>(rows0), static_cast<int>(db + eb), part1, static_cast<int>(sp.n1),
+                     static_cast<int>(eb), static_cast<int>(arows), static_cast<int>(db), sp.splits, b0, c, ldc,
+                     init != 0 ? 1 : 0);
+  return check_launch(who);
 }
 
 extern "C" int rf_norm_linear(const uint16_t* x, int64_t ldx, const float* ssq, int64_t P, int64_t H, float eps,

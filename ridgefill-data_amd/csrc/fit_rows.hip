@@ -35,7 +35,8 @@ struct TransposeArgs {
 // lo rows] gives the products of the centred fp32 values. The sums (and squares) of d over a 64-row tile:
 // each 16-row group in row order (lane 8 (2g + 1) + j continues the chain lane 8 (2g) + j began), then the
 // four groups pairwise, ((g0 + g1) + (g2 + g3)).
-template <bool SHIFT>
+// STORE false: the column sums only, nothing is written to dst (rf_col_moments).
+template <bool SHIFT, bool STORE = true>
 __global__ __launch_bounds__(256) void k_transpose(TransposeArgs a) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = lane >> 3, j = lane & 7;
   const int64_t r0 = static_cast<int64_t>(blockIdx.x) * TT;
@@ -99,6 +100,7 @@ __global__ __launch_bounds__(256) void k_transpose(TransposeArgs a) {
       }
     }
   }
+  if constexpr (!STORE) return;
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
     const int64_t orow = cb + c;
@@ -133,6 +135,161 @@ __global__ __launch_bounds__(256) void k_colsum_fold(const float* __restrict__ p
     __syncthreads();
   }
   if (i == 0 && c < cols) sums[c] += red[0][cl];
+}
+
+// The centring of one operand from its rows' sums s1 and sums of squares s2 over n rows: the shift c (the mean
+// rounded to fp32, or `given`), the channels with c^2 > variance (at most cap of them, largest c^2 / variance
+// first, lower index first among equals) with their fp32 shift, their row among the centred channels in
+// channel order, and what is left of c for the others. One block: thread t takes the per = ceil(cols / 1024)
+// channels from t * per on, so a block scan of the threads' counts gives the channel order; when more than cap
+// channels qualify, each one's rank is counted against every ratio, staged 1024 at a time in LDS. It takes 16 us
+// at 4096 channels and replaces about twenty launches of sorts and index operations (their gaps: 150 us).
+constexpr int SEL_THREADS = 1024;
+struct CentreArgs {
+  const double *s1, *s2, *given;
+  double n;
+  int cols, cap;
+  double* c;
+  float* shift;
+  int* lo_row;
+  double* delta;
+  int64_t* idx;
+  int* count;
+  double* ratio;          // [cols] scratch: c^2 / variance of a qualifying channel, else -1
+};
+__global__ __launch_bounds__(SEL_THREADS) void k_centre_select(CentreArgs a) {
+#pragma clang fp contract(off)
+  __shared__ double stage[SEL_THREADS];
+  __shared__ int scan[SEL_THREADS];
+  const int t = threadIdx.x, per = (a.cols + SEL_THREADS - 1) / SEL_THREADS;
+  const int lo = min(t * per, a.cols), hi = min(lo + per, a.cols);
+  int mine = 0;
+  for (int k = lo; k < hi; ++k) {
+    const double mean = a.s1[k] / a.n;
+    double var = a.s2[k] / a.n - mean * mean;
+    var = var < 0.0 ? 0.0 : var;                    // (a NaN stays one and qualifies nothing)
+    const double c = a.given ? a.given[k] : static_cast<double>(static_cast<float>(mean));
+    const double c2 = c * c;
+    const bool big = c2 > var;
+    a.c[k] = c;
+    a.ratio[k] = big ? c2 / fmax(var, 1e-300) : -1.0;
+    mine += big ? 1 : 0;
+  }
+  scan[t] = mine;
+  __syncthreads();
+  for (int h = SEL_THREADS / 2; h >= 1; h >>= 1) {
+    if (t < h) scan[t] += scan[t + h];
+    __syncthreads();
+  }
+  const int nbig = scan[0];
+  __syncthreads();
+  // selected channels of this thread: a.lo_row holds the rank until the row is known
+  for (int k = lo; k < hi; ++k) a.lo_row[k] = 0;
+  if (nbig > a.cap) {
+    for (int j0 = 0; j0 < a.cols; j0 += SEL_THREADS) {
+      __syncthreads();
+      stage[t] = j0 + t < a.cols ? a.ratio[j0 + t] : -1.0;
+      __syncthreads();
+      for (int k = lo; k < hi; ++k) {
+        const double r = a.ratio[k];
+        if (r < 0.0) continue;
+        int above = 0;
+        for (int j = 0; j < SEL_THREADS; ++j) above += (stage[j] > r || (stage[j] == r && j0 + j < k)) ? 1 : 0;
+        a.lo_row[k] += above;
+      }
+    }
+  }
+  mine = 0;
+  for (int k = lo; k < hi; ++k) mine += (a.ratio[k] >= 0.0 && a.lo_row[k] < a.cap) ? 1 : 0;
+  __syncthreads();
+  scan[t] = mine;
+  __syncthreads();
+  for (int h = 1; h < SEL_THREADS; h <<= 1) {       // inclusive scan
+    const int v = t >= h ? scan[t - h] : 0;
+    __syncthreads();
+    scan[t] += v;
+    __syncthreads();
+  }
+  int row = scan[t] - mine;
+  for (int k = lo; k < hi; ++k) {
+    const bool sel = a.ratio[k] >= 0.0 && a.lo_row[k] < a.cap;
+    const float sh = sel ? static_cast<float>(a.c[k]) : 0.f;
+    a.shift[k] = sh;
+    a.delta[k] = a.c[k] - static_cast<double>(sh);
+    a.lo_row[k] = sel ? row : -1;
+    if (sel) a.idx[row++] = k;
+  }
+  if (t == SEL_THREADS - 1) *a.count = scan[t];
+}
+
+// One product of the fit's state from its augmented Gram G: D[r, c] = the sum of the parts of the centred
+// products (main, mid and lo rows and columns, added in that order) moved onto the reference's shifts,
+// D = parts - da s1b^T - s1a db^T + n da db^T, in one pass: G read once, D written once (bound by that traffic: 268
+// MB at 4096 x 4096, 90 us = 3.0 TB/s), where separate index, clone and rank-1 operations passed over D ten times
+// in some twenty launches (about 330 us). upper: G
+// holds its block-upper 256 x 256 tiles only and is symmetric (G[r, c] = G[c, r] for a block-lower (r, c)); such
+// a tile is read transposed through LDS.
+struct GramStateArgs {
+  const double* g;
+  int64_t ldg;
+  int ca, sa, cb, sb;
+  const int *lo_a, *lo_b;
+  int upper;
+  const double *s1a, *s1b, *da, *db;
+  double n;
+  double* out;
+  int64_t ldo;
+};
+constexpr int ST = 64;                            // 64 x 64 values a block
+__global__ __launch_bounds__(256) void k_gram_state(GramStateArgs a) {
+  __shared__ double tile[ST][ST + 1];
+  const int t = threadIdx.x, r0 = blockIdx.y * ST, c0 = blockIdx.x * ST;
+  const bool mirror = a.upper && (r0 >> 8) > (c0 >> 8);             // block-uniform: 64 divides 256
+  if (mirror) {
+    for (int k = t; k < ST * ST; k += 256) {
+      const int i = k >> 6, j = k & 63;                             // G row c0 + i, column r0 + j
+      tile[j][i] = (c0 + i < a.cb && r0 + j < a.ca) ? a.g[static_cast<int64_t>(c0 + i) * a.ldg + r0 + j] : 0.0;
+    }
+    __syncthreads();
+  }
+  auto at = [&](int r, int c) {
+    return a.upper && (r >> 8) > (c >> 8) ? a.g[static_cast<int64_t>(c) * a.ldg + r]
+                                          : a.g[static_cast<int64_t>(r) * a.ldg + c];
+  };
+  const int c = c0 + (t & 63);
+  if (c >= a.cb) return;
+  const int lb = a.sb ? a.lo_b[c] : -1;
+  const double s1b = a.s1b[c], db = a.db[c];
+  auto parts = [&](int r, double v) {
+    if (lb >= 0) {
+      v += at(r, a.cb + lb);
+      v += at(r, a.cb + a.sb + lb);
+    }
+    return v;
+  };
+  // the thread's 16 values first, all their loads in flight (rows past ca read row ca - 1, not stored)
+  double main[ST / 4];
+#pragma unroll
+  for (int k = 0; k < ST / 4; ++k) {
+    const int i = (t >> 6) + 4 * k;
+    main[k] = mirror ? tile[i][t & 63] : a.g[static_cast<int64_t>(min(r0 + i, a.ca - 1)) * a.ldg + c];
+  }
+#pragma unroll
+  for (int k = 0; k < ST / 4; ++k) {
+    const int r = r0 + (t >> 6) + 4 * k;
+    if (r >= a.ca) break;
+    double v = parts(r, main[k]);
+    const int la = a.sa ? a.lo_a[r] : -1;           // uniform over the row's 64 lanes
+    if (la >= 0) {
+      v += parts(a.ca + la, at(a.ca + la, c));
+      v += parts(a.ca + a.sa + la, at(a.ca + a.sa + la, c));
+    }
+    const double da = a.da[r];
+    v -= da * s1b;
+    v -= a.s1a[r] * db;
+    v += a.n * (da * db);
+    a.out[static_cast<int64_t>(r) * a.ldo + c] = v;
+  }
 }
 
 // Read cosines of one late layer for one held-out document (code/scripts/fit_sweep.py:307-313). A work
@@ -265,6 +422,55 @@ extern "C" int rf_transpose_centred(const uint16_t* src, int64_t ld_src, int64_t
   const TransposeArgs a{src, ld_src, rows, static_cast<int>(cols), dst, ld_dst, shift, lo_row, dst_lo, n_centred,
                         partial, partial_sq};
   return launch_transpose("rf_transpose_centred", a, rows, cols, ld_src, ld_dst, stream);
+}
+
+extern "C" int rf_col_moments(const uint16_t* src, int64_t ld_src, int64_t rows, int64_t cols, float* partial,
+                              float* partial_sq, hipStream_t stream) {
+  const char* fn = "rf_col_moments";
+  if (!src || !partial || !partial_sq) return fail(RF_EINVAL_ARG, "%s: null pointer", fn);
+  const int64_t tiles = (rows + TT - 1) / TT;
+  if (rows < 0 || cols <= 0 || cols % TT || cols > (1 << 24) || ld_src < cols || ld_src % 8 || tiles > (1ll << 31) - 1 ||
+      !aligned16(src))
+    return fail(RF_EINVAL_SHAPE, "%s: rows %lld, cols %lld (multiple of 64), ld_src %lld (multiple of 8), 16-byte aligned",
+                fn, (long long)rows, (long long)cols, (long long)ld_src);
+  if (rows == 0) return RF_OK;
+  const TransposeArgs a{src, ld_src, rows, static_cast<int>(cols), nullptr, 0, nullptr, nullptr, nullptr, 0,
+                        partial, partial_sq};
+  const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>((cols + 4 * TT - 1) / (4 * TT)));
+  hipLaunchKernelGGL((k_transpose<false, false>), grid, dim3(256), 0, stream, a);
+  return check_launch(fn);
+}
+
+extern "C" int rf_centre_select(const double* s1, const double* s2, double n, const double* given, int64_t cols,
+                                int64_t cap, double* c, float* shift, int32_t* lo_row, double* delta, int64_t* idx,
+                                int32_t* count, double* scratch, hipStream_t stream) {
+  const char* fn = "rf_centre_select";
+  if (!s1 || !s2 || !c || !shift || !lo_row || !delta || !count || !scratch || (!idx && cap > 0))
+    return fail(RF_EINVAL_ARG, "%s: null pointer", fn);
+  if (cols <= 0 || cols > (1 << 24) || cap < 0 || !(n > 0.0))
+    return fail(RF_EINVAL_SHAPE, "%s: cols %lld, cap %lld, n %g", fn, (long long)cols, (long long)cap, n);
+  const CentreArgs a{s1, s2, given, n, static_cast<int>(cols), static_cast<int>(cap < cols ? cap : cols), c, shift,
+                     lo_row, delta, idx, count, scratch};
+  hipLaunchKernelGGL(k_centre_select, dim3(1), dim3(SEL_THREADS), 0, stream, a);
+  return check_launch(fn);
+}
+
+extern "C" int rf_gram_state(const double* g, int64_t ldg, int64_t ca, int64_t sa, const int32_t* lo_a, int64_t cb,
+                             int64_t sb, const int32_t* lo_b, int upper, const double* s1a, const double* s1b,
+                             const double* da, const double* db, double n, double* out, int64_t ldo,
+                             hipStream_t stream) {
+  const char* fn = "rf_gram_state";
+  if (!g || !s1a || !s1b || !da || !db || !out || (sa > 0 && !lo_a) || (sb > 0 && !lo_b))
+    return fail(RF_EINVAL_ARG, "%s: null pointer", fn);
+  if (ca <= 0 || cb <= 0 || sa < 0 || sb < 0 || ca + 2 * sa > (1 << 24) || cb + 2 * sb > (1 << 24) || ldg < cb + 2 * sb ||
+      ldo < cb || (upper && (ca != cb || sa != sb)) || (ca + ST - 1) / ST > 65535)
+    return fail(RF_EINVAL_SHAPE, "%s: %lld + 2 x %lld by %lld + 2 x %lld, ldg %lld, ldo %lld", fn, (long long)ca,
+                (long long)sa, (long long)cb, (long long)sb, (long long)ldg, (long long)ldo);
+  const GramStateArgs a{g, ldg, static_cast<int>(ca), static_cast<int>(sa), static_cast<int>(cb), static_cast<int>(sb),
+                        lo_a, lo_b, upper ? 1 : 0, s1a, s1b, da, db, n, out, ldo};
+  const dim3 grid(static_cast<unsigned>((cb + ST - 1) / ST), static_cast<unsigned>((ca + ST - 1) / ST));
+  hipLaunchKernelGGL(k_gram_state, grid, dim3(256), 0, stream, a);
+  return check_launch(fn);
 }
 
 extern "C" int rf_colsum_fold(const float* partial, int64_t ntiles, int64_t cols, double* sums, hipStream_t stream) {

@@ -85,7 +85,7 @@ class Capture:
         main, lo = self.T[r:r + self.H, self.off:self.off + kp], self.T[r + self.H:r + self.R, self.off:self.off + kp]
         part = ridge.tiles_view(self.part, kp // 64, self.H)
         if self.cen[j] is None:                           # the first document: its means are the shifts
-            self.cen[j] = ridge.Centring.of_rows(h, self.T[r:r + self.H, self.off:], self.part, self.part_sq)
+            self.cen[j] = ridge.Centring.of_rows(h, self.part, self.part_sq)
         c = self.cen[j]
         ridge.transpose_centred(h, main, lo, c.shift, c.lo_row, part, n_centred=c.s)
         ridge._colsum_fold(part, self.s1[j])
@@ -132,7 +132,7 @@ class Capture:
             blk = G[:, (i - S) * R:(i - S + 1) * R]
             cy[i] = c.c.to(device)
             sy[i] = (s1y - n * c.delta).to(device)
-            sxy[i] = ridge.recentre(ridge.centred_products(blk, H, cx, H, c), s1x, s1y, cx.delta, c.delta, n).to(device)
+            sxy[i] = ridge.centred_state(blk, H, cx, H, c, s1x, s1y, n).to(device)
         return dict(split=S, layers=late, dim=H, n=self.n, cx=cx.c.to(device), cy=cy,
                     sx=(s1x - n * cx.delta).to(device), sxx=sxy[S].clone(), sy=sy, sxy=sxy)
 

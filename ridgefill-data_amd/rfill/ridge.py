@@ -136,6 +136,35 @@ def gram_accumulate(a, b, c, fold_rows=0, workspace=None):
     return c
 
 
+def gram_centred_workspace_bytes(da, ea, db, eb, K, fold_rows=0, upper=False):
+    """Bytes of rf_gram_centred's workspace for this shape."""
+    nb = ctypes.c_size_t(0)
+    _lib.call("rf_gram_centred_workspace_bytes", da, ea, db, eb, K, int(fold_rows), int(upper), ctypes.byref(nb))
+    return nb.value
+
+
+def gram_centred(a, da, ea, b, db, eb, c, fold_rows=0, upper=False, init=False, workspace=None):
+    """The augmented Gram of centred operands: c [:da + ea, :db + eb] += a[:da + ea] b[:db + eb]^T (a, b bf16
+    K-contiguous; c fp64), the da x db main product as gram_accumulate (or, upper, gram_accumulate_upper) runs
+    it and the few extra rows (mid and lo parts) as products of few rows with their K range split, each split
+    added in fp64. upper (b is a): the main block-upper tiles and the extra columns only. init: c's old values
+    count as zeros (c may be uninitialised); its columns past db + eb are never touched."""
+    _need(a, "a", torch.bfloat16, 2)
+    _need(b, "b", torch.bfloat16, 2)
+    _need(c, "c", torch.float64, 2)
+    K = a.shape[1]
+    if b.shape[1] != K or a.shape[0] < da + ea or b.shape[0] < db + eb or c.shape[0] < da + ea or c.shape[1] < db + eb:
+        raise ValueError(f"gram_centred shapes a {tuple(a.shape)}, b {tuple(b.shape)}, c {tuple(c.shape)} for "
+                         f"{da} + {ea} by {db} + {eb} rows")
+    need = gram_centred_workspace_bytes(da, ea, db, eb, K, fold_rows, upper)
+    if need and (workspace is None or workspace.numel() < need):
+        workspace = torch.empty(need, dtype=torch.uint8, device=c.device)
+    _lib.call("rf_gram_centred", _ptr(a), a.stride(0), da, ea, _ptr(b), b.stride(0), db, eb, K, int(fold_rows), _ptr(c),
+              c.stride(0), int(upper), int(init), _ptr(workspace), workspace.numel() if workspace is not None else 0,
+              _stream(a))
+    return c
+
+
 class Centring:
     """One operand's centring: the reference's shift c [cols] (fp64 of an fp32 mean), the centred channels idx
     (sorted) with their shift (fp32, 0 elsewhere) and mid rows (int32, -1 elsewhere; the lo row is s rows
@@ -144,9 +173,13 @@ class Centring:
     square exceeds the rows' variance, largest ratio first, at most cap of them."""
 
     def __init__(self, s1, s2, n, c=None, cap=SHIFT_MAX):
+        c = None if c is None else c.to(s1.device, torch.float64).contiguous()
+        if s1.is_cuda:
+            self._select(s1, s2, n, c, cap)
+            return
         mean = s1 / n
         var = (s2 / n - mean * mean).clamp_min(0)
-        self.c = mean.float().double() if c is None else c.to(s1.device, torch.float64)
+        self.c = mean.float().double() if c is None else c
         c2 = self.c * self.c
         big = (c2 > var).nonzero().flatten()
         ratio = c2[big] / var[big].clamp_min(1e-300)
@@ -160,15 +193,31 @@ class Centring:
         self.lo_rows = LO_ROWS if self.s else 0
         self.delta = self.c - self.shift.double()       # the stored sums' shift -> the reference's shift
 
+    def _select(self, s1, s2, n, c, cap):
+        """The same choice on the GPU in one launch (rf_centre_select); the count is read back once."""
+        cols, dev = s1.numel(), s1.device
+        cap = max(0, min(cap, cols))
+        f64 = torch.empty(3, cols, dtype=torch.float64, device=dev)
+        self.c, self.delta, scratch = f64
+        self.shift = torch.empty(cols, dtype=torch.float32, device=dev)
+        self.lo_row = torch.empty(cols, dtype=torch.int32, device=dev)
+        idx = torch.empty(cap, dtype=torch.int64, device=dev)
+        count = torch.empty(1, dtype=torch.int32, device=dev)
+        _lib.call("rf_centre_select", _ptr(s1), _ptr(s2), float(n), _ptr(c), cols, cap, _ptr(self.c), _ptr(self.shift),
+                  _ptr(self.lo_row), _ptr(self.delta), _ptr(idx) if cap else None, _ptr(count), _ptr(scratch),
+                  _stream(s1))
+        self.s = int(count.item())
+        self.idx = idx[:self.s]
+        self.lo_rows = LO_ROWS if self.s else 0
+
     @classmethod
-    def of_rows(cls, x, work, part, part_sq, c=None, cap=SHIFT_MAX):
-        """The centring chosen from rows x [n, cols] (their sums, via a plain transpose into work)."""
+    def of_rows(cls, x, part, part_sq, c=None, cap=SHIFT_MAX):
+        """The centring chosen from rows x [n, cols] (part / part_sq: room for their per-64-row sums)."""
         n, cols = x.shape
-        kp = (n + 63) // 64 * 64
-        s1 = torch.zeros(cols, dtype=torch.float64, device=x.device)
-        s2 = torch.zeros_like(s1)
-        p1, p2 = tiles_view(part, kp // 64, cols), tiles_view(part_sq, kp // 64, cols)
-        transpose_centred(x, work[:cols, :kp], None, None, None, p1, p2)
+        tiles = (n + 63) // 64
+        s1, s2 = torch.zeros(2, cols, dtype=torch.float64, device=x.device)
+        p1, p2 = tiles_view(part, tiles, cols), tiles_view(part_sq, tiles, cols)
+        _lib.call("rf_col_moments", _ptr(x), x.stride(0), n, cols, _ptr(p1), _ptr(p2), _stream(x))
         _colsum_fold(p1, s1)
         _colsum_fold(p2, s2)
         return cls(s1, s2, n, c, cap)
@@ -199,6 +248,21 @@ def recentre(D, s1a, s1b, da, db, n):
     D.addr_(s1a, db, alpha=-1.0)
     D.addr_(da, db, alpha=float(n))
     return D
+
+
+def centred_state(G, ca, A, cb, B, s1a, s1b, n, upper=False):
+    """The [ca, cb] product of an augmented Gram G about the reference's shifts: centred_products, then
+    recentre by A.delta / B.delta over n rows. upper: G (symmetric, A is B) holds its block-upper 256 x 256 tiles
+    only. On the GPU one pass over G (rf_gram_state)."""
+    if not G.is_cuda:
+        return recentre(centred_products(mirror_block_upper(G) if upper else G, ca, A, cb, B), s1a, s1b, A.delta,
+                        B.delta, n)
+    if G.stride(1) != 1:
+        raise ValueError("centred_state: G must be row-major")
+    out = torch.empty(ca, cb, dtype=torch.float64, device=G.device)
+    _lib.call("rf_gram_state", _ptr(G), G.stride(0), ca, A.s, _ptr(A.lo_row), cb, B.s, _ptr(B.lo_row), int(upper),
+              _ptr(s1a), _ptr(s1b), _ptr(A.delta), _ptr(B.delta), float(n), _ptr(out), out.stride(0), _stream(G))
+    return out
 
 
 class RidgeStats:
@@ -243,21 +307,16 @@ class RidgeStats:
         extra rows, and the per-64-row column-sum partials."""
         if self._xt is None or self._xt.shape[1] - ROW_PAD < kp:
             d, o, lo = self.dim, self.out_dim, LO_ROWS
-            self._xt = torch.zeros(d + lo, kp + ROW_PAD, dtype=torch.bfloat16, device=self.device)
-            self._yt = torch.zeros(o + lo, kp + ROW_PAD, dtype=torch.bfloat16, device=self.device)
+            self._xt = torch.empty(d + lo, kp + ROW_PAD, dtype=torch.bfloat16, device=self.device)
+            self._yt = torch.empty(o + lo, kp + ROW_PAD, dtype=torch.bfloat16, device=self.device)
             self._part = torch.empty(kp // 64 * max(d, o), dtype=torch.float32, device=self.device)
             self._sq = torch.empty_like(self._part)
         return self._xt, self._yt, self._part
 
-    def _gram(self, a, b, c, block):
-        """gram_accumulate with a workspace kept between calls (grown as needed)."""
-        need = gram_workspace_bytes(a.shape[0], b.shape[0], a.shape[1], block)
-        gram_accumulate(a, b, c, block, self._workspace(need))
-
-    def _gram_upper(self, a, M, c, block):
-        """gram_accumulate_upper with the same kept workspace."""
-        need = gram_upper_workspace_bytes(M, a.shape[0], a.shape[1], block)
-        gram_accumulate_upper(a, M, c, block, self._workspace(need))
+    def _gram(self, a, ea, b, db, eb, c, block, upper=False, init=False):
+        """gram_centred of X^T (a: dim main and ea extra rows) with a workspace kept between calls."""
+        need = gram_centred_workspace_bytes(self.dim, ea, db, eb, a.shape[1], block, upper)
+        gram_centred(a, self.dim, ea, b, db, eb, c, block, upper, init, self._workspace(need))
 
     def _workspace(self, need):
         ws = getattr(self, "_gws", None)
@@ -299,20 +358,20 @@ class RidgeStats:
             return
         if self.cen_x is None:                          # the first block's means are the shifts (ridge.py:37-38)
             kp = (min(block, n) + 63) // 64 * 64
-            xt, _, part = self._buffers(kp)
+            _, _, part = self._buffers(kp)
             b = self.base
-            self.cen_x = Centring.of_rows(x[:block], xt, part, self._sq, None if b is None else b["cx"],
-                                          self.centre_max)
-            self.sxx = torch.zeros(d + 2 * self.cen_x.s, d + self.cen_x.lo_rows, dtype=torch.float64,
-                                   device=self.device)
+            self.cen_x = Centring.of_rows(x[:block], part, self._sq, None if b is None else b["cx"], self.centre_max)
         cx = self.cen_x
         self.n += n
         for r in range(0, n, PIECE):
             rows = self._x_piece(r, True)
             kp = (rows + 63) // 64 * 64
-            xt = self._xt
-            self._gram_upper(xt[:d + cx.lo_rows, :kp], d + 2 * cx.s, self.sxx, block)
-            self._sxx_upper = True
+            xt, e = self._xt[:, :kp], 2 * cx.s
+            init = self.sxx is None                     # the first product is stored, not added to zeros
+            if init:
+                self.sxx = torch.empty(d + e, d + cx.lo_rows, dtype=torch.float64, device=self.device)
+                self._sxx_upper = True
+            self._gram(xt, e, xt, d, e, self.sxx, block, upper=True, init=init)
 
     @torch.no_grad()
     def add_layer(self, i, y):
@@ -331,13 +390,11 @@ class RidgeStats:
         d, o, block, cx = self.dim, self.out_dim, self._block, self.cen_x
         if i not in self.cen_y:
             kp = (min(block, n) + 63) // 64 * 64
-            _, yt, part = self._buffers(kp)
+            _, _, part = self._buffers(kp)
             b = self.base
-            self.cen_y[i] = Centring.of_rows(y[:block], yt, part, self._sq, None if b is None else b["cy"][i],
+            self.cen_y[i] = Centring.of_rows(y[:block], part, self._sq, None if b is None else b["cy"][i],
                                              self.centre_max)
         cy = self.cen_y[i]
-        if i not in self.sxy:
-            self.sxy[i] = torch.zeros(d + 2 * cx.s, o + cy.lo_rows, dtype=torch.float64, device=self.device)
         for r in range(0, n, PIECE):
             rows = self._x_piece(r, False) if self._held != r else min(PIECE, n - r)
             kp = (rows + 63) // 64 * 64
@@ -345,7 +402,10 @@ class RidgeStats:
             py = tiles_view(part, kp // 64, o)
             transpose_centred(y[r:r + rows], yt[:o, :kp], yt[o:, :kp], cy.shift, cy.lo_row, py, n_centred=cy.s)
             _colsum_fold(py, self.s1y[i])
-            self._gram(xt[:d + 2 * cx.s, :kp], yt[:o + cy.lo_rows, :kp], self.sxy[i], block)
+            init = i not in self.sxy
+            if init:
+                self.sxy[i] = torch.empty(d + 2 * cx.s, o + cy.lo_rows, dtype=torch.float64, device=self.device)
+            self._gram(xt[:, :kp], 2 * cx.s, yt[:, :kp], o, 2 * cy.s, self.sxy[i], block, init=init)
 
     def add(self, x, ys, block=8192, w=None):
         """x [n, d] and ys {layer: [n, d_out]}: bf16 rows on the GPU (the same rows, in order)
@@ -363,9 +423,8 @@ class RidgeStats:
         n = float(self.n)
         d, o, cx = self.dim, self.out_dim, self.cen_x
         dx = cx.delta
-        if getattr(self, "_sxx_upper", False):      # X^T X accumulated on its block-upper tiles only
-            mirror_block_upper(self.sxx)
-        sxx = recentre(centred_products(self.sxx, d, cx, d, cx), self.s1x, self.s1x, dx, dx, n)
+        # X^T X is accumulated on its block-upper tiles only
+        sxx = centred_state(self.sxx, d, cx, d, cx, self.s1x, self.s1x, n, upper=getattr(self, "_sxx_upper", False))
         cy, sy, sxy = {}, {}, {}
         for i in self.layers:
             if i not in self.cen_y:                 # no rows of this layer yet: zero sums, no shift (ridge.py:73)
@@ -377,7 +436,7 @@ class RidgeStats:
             c = self.cen_y[i]
             cy[i] = c.c
             sy[i] = self.s1y[i] - n * c.delta
-            sxy[i] = recentre(centred_products(self.sxy[i], d, cx, o, c), self.s1x, self.s1y[i], dx, c.delta, n)
+            sxy[i] = centred_state(self.sxy[i], d, cx, o, c, self.s1x, self.s1y[i], n)
         mine = dict(split=self.split, layers=self.layers, dim=self.dim, n=self.n, cx=cx.c, cy=cy,
                     sx=self.s1x - n * dx, sxx=sxx, sy=sy, sxy=sxy)
         return _to(combine(self.base, mine, 1) if self.base is not None else mine, device)

@@ -246,3 +246,84 @@ def test_resumed_statistics_continue_the_device_sums(dev):
         wa, ba = fa.layer(6, (lam,))[lam]
         wb, bb = fb.layer(6, (lam,))[lam]
         assert rel(wa, wb) < 1e-5 and rel(ba, bb) < 1e-5
+
+
+@pytest.mark.parametrize("da,ea,db,eb,K,fold,upper", [
+    (256, 0, 512, 0, 640, 256, False), (256, 2, 512, 6, 64, 0, False), (512, 256, 256, 250, 1088, 512, False),
+    (512, 0, 512, 34, 2048, 0, False), (512, 66, 256, 0, 4160, 1024, False), (768, 8, 768, 8, 8192, 8192, True),
+    (512, 162, 512, 162, 3136, 2048, True), (512, 0, 512, 0, 1088, 256, True)])
+@pytest.mark.parametrize("init", [False, True])
+def test_gram_centred_is_the_augmented_product(dev, da, ea, db, eb, K, fold, upper, init):
+    """rf_gram_centred over its operands' main and extra rows (no extra rows, few, the most; one or two row blocks;
+    K of one step, not a multiple of the splits; short last runs) against fp64 products: 1e-6 of their norm, the
+    fp32 sums' bound as above. Columns past the extra ones stay untouched, with init the old values do not matter,
+    and only the workspace it asks for is written."""
+    from rfill import ridge
+    g = torch.Generator(device=dev).manual_seed(da + ea + eb + K)
+    a = torch.randn(da + 256, K + 64, generator=g, device=dev).to(torch.bfloat16)[:, :K]
+    b = a if upper else (torch.randn(db + 256, K + 64, generator=g, device=dev) * 2).to(torch.bfloat16)[:, :K]
+    c0 = torch.randn(da + ea, db + 256, generator=g, device=dev, dtype=torch.float64)
+    need = ridge.gram_centred_workspace_bytes(da, ea, db, eb, K, fold, upper)
+    buf = torch.full((need + 4096,), 0xFF, dtype=torch.uint8, device=dev)
+    c = torch.full_like(c0, float("nan")) if init else c0.clone()
+    old = c.clone()
+    ridge.gram_centred(a, da, ea, b, db, eb, c, fold, upper, init, buf[:need] if need else None)
+    torch.cuda.synchronize()
+    assert bool((buf[need:] == 0xFF).all()), "wrote past its workspace"
+    want = a[:da + ea].double() @ b[:db + eb].double().T + (0 if init else c0[:, :db + eb])
+    ti = torch.arange(da + ea, device=dev)[:, None] // 256
+    tj = torch.arange(db + eb, device=dev)[None, :] // 256
+    live = tj >= ti if upper else torch.ones(da + ea, db + eb, dtype=torch.bool, device=dev)
+    err = rel(c[:, :db + eb][live], want[live])
+    print(f"gram centred rel err {err:.2e}")
+    assert err < 1e-6
+    assert torch.equal(c[:, db + eb:].isnan(), old[:, db + eb:].isnan())
+    assert init or torch.equal(c[:, db + eb:], c0[:, db + eb:])
+
+
+@pytest.mark.parametrize("cols,cap,given,kind", [(256, 128, False, "few"), (4096, 128, False, "many"), (1088, 3, True, "ties"),
+                                                 (2048, 0, False, "many"), (3072, 128, False, "none"), (512, 512, False, "all")])
+def test_centring_and_state_on_the_gpu_match_the_host_path(dev, cols, cap, given, kind):
+    """rf_centre_select against Centring on the CPU from the same sums (nothing centred, few, more than the cap, equal
+    ratios), every output equal; then rf_gram_state against centred_products and recentre on the CPU, to fp64
+    rounding (4 parts and 3 rank-1 terms: 1e-14 of the largest term)."""
+    from rfill import ridge
+    g = torch.Generator().manual_seed(cols + cap)
+    n, f64 = 1000, torch.float64
+    mean = torch.randn(cols, generator=g, dtype=f64)
+    spread = torch.rand(cols, generator=g, dtype=f64) + 0.5
+    if kind == "few":
+        mean *= torch.where(torch.arange(cols) % 50 == 7, 8.0, 0.1)
+    elif kind == "ties":
+        mean, spread = torch.full_like(mean, 2.0), torch.ones_like(spread)
+    elif kind == "none":
+        mean *= 0.01
+    elif kind == "all":
+        mean = mean.sign() * 4 + mean
+    s1, s2 = mean * n, (spread ** 2 + mean ** 2) * n
+    c = (mean * 1.01).float().double() if given else None
+    want = ridge.Centring(s1, s2, n, c, cap)
+    got = ridge.Centring(s1.to(dev), s2.to(dev), n, c, cap)
+    for name in ("c", "shift", "lo_row", "idx", "delta"):
+        assert torch.equal(getattr(got, name).cpu(), getattr(want, name)), name
+    assert got.s == want.s and got.lo_rows == want.lo_rows
+    if cols > 1100:
+        return
+    for upper in (False, True):
+        rows = want.s if upper else min(want.s, 2)
+        A = want if upper else ridge.Centring(s1[:320] if cols >= 320 else s1, s2[:320] if cols >= 320 else s2, n, None, rows)
+        Ag = got if upper else ridge.Centring(s1[:A.c.numel()].to(dev), s2[:A.c.numel()].to(dev), n, None, rows)
+        ca = A.c.numel()
+        G = torch.randn(ca + 2 * A.s, cols + 2 * want.s + 8, generator=g, dtype=f64)
+        if upper:                                   # symmetric over its stored part, the block-lower tiles not stored
+            m = cols + 2 * want.s
+            G[:, :m] += G[:, :m].T.clone()
+        s1a, s1b = torch.randn(ca, generator=g, dtype=f64), torch.randn(cols, generator=g, dtype=f64)
+        ref = ridge.recentre(ridge.centred_products(G, ca, A, cols, want), s1a, s1b, A.delta, want.delta, float(n))
+        dG = G.to(dev)
+        if upper:
+            lower = torch.arange(G.shape[0])[:, None] // 256 > torch.arange(G.shape[1])[None, :] // 256
+            dG[lower.to(dev)] = float("nan")
+        out = ridge.centred_state(dG, ca, Ag, cols, got, s1a.to(dev), s1b.to(dev), float(n), upper)
+        big = n * float((A.delta.abs().max() * want.delta.abs().max())) + 10
+        assert float((out.cpu() - ref).abs().max()) < 1e-14 * big * 8, (upper, float((out.cpu() - ref).abs().max()))
