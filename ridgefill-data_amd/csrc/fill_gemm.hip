@@ -466,18 +466,59 @@ __global__ __launch_bounds__(NTHR) void k_rows_partial(const uint16_t* __restric
   rows_partial<RT>(X, ldx, W, ldw, M, N, K, kper, rblocks, part, lds, blockIdx.x, gridDim.x, N);
 }
 
-// The split sums of 8 consecutive columns col .. col + 7 of row gm: 8 fp32 values, splits added in order.
+// The split sums of 8 consecutive columns col .. col + 7 of row gm: 8 fp32 values, splits added in order. Four
+// splits' loads are in flight at a time (one load's latency per split made the reduce kernels of few rows 6 us,
+// most of it waiting; together with the statistics' loads below 4.5 to 5 us at 37 rows and 8 splits).
 __device__ __forceinline__ void split_sums(const float* __restrict__ part, int splits, int64_t plane, int64_t off,
                                            float (&v)[8]) {
   const float4* p = reinterpret_cast<const float4*>(part + off);
   float4 a = p[0], b = p[1];
-  for (int sp = 1; sp < splits; ++sp) {
-    const float4* q = reinterpret_cast<const float4*>(part + sp * plane + off);
-    const float4 c = q[0], d = q[1];
+  auto add = [&](const float4& c, const float4& d) {
     a.x += c.x; a.y += c.y; a.z += c.z; a.w += c.w;
     b.x += d.x; b.y += d.y; b.z += d.z; b.w += d.w;
+  };
+  auto batch = [&](int sp, auto n) {
+    float4 c[decltype(n)::value], d[decltype(n)::value];
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+      const float4* q = reinterpret_cast<const float4*>(part + (sp + i) * plane + off);
+      c[i] = q[0];
+      d[i] = q[1];
+    }
+#pragma unroll
+    for (int i = 0; i < n; ++i) add(c[i], d[i]);
+  };
+  int sp = 1;
+  for (; sp + 4 <= splits; sp += 4) batch(sp, std::integral_constant<int, 4>{});
+  switch (splits - sp) {
+    case 3: batch(sp, std::integral_constant<int, 3>{}); break;
+    case 2: batch(sp, std::integral_constant<int, 2>{}); break;
+    case 1: batch(sp, std::integral_constant<int, 1>{}); break;
+    default: break;
   }
   v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+
+// Sum of a row's nparts statistics partials q, in order. Up to 16 partials, a multiple of 4 (H 1024 .. 4096 and
+// H % 1024 == 0): all loaded before the first is added (loads past the end repeat the last).
+__device__ __forceinline__ float parts_total(const float* __restrict__ q, int nparts) {
+  float s = 0.f;
+  if (nparts % 4 == 0 && nparts <= 16) {            // uniform
+    float4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const float4*>(q + 4 * min(k, nparts / 4 - 1));
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (4 * k < nparts) {
+        s += v[k].x;
+        s += v[k].y;
+        s += v[k].z;
+        s += v[k].w;
+      }
+  } else {
+    for (int i = 0; i < nparts; ++i) s += q[i];
+  }
+  return s;
 }
 
 __global__ __launch_bounds__(NTHR) void k_map_apply(const uint16_t* __restrict__ B, int64_t ldb,
@@ -913,8 +954,7 @@ __global__ __launch_bounds__(256) void k_norm_linear_reduce(const float* __restr
   const int m = blockIdx.x * RED_ROWS + r;
   if (m >= M) return;
   const int nparts = K / SSQ_COLS;
-  float s2 = 0.f;
-  for (int i = 0; i < nparts; ++i) s2 += ssq[static_cast<int64_t>(m) * nparts + i];
+  const float s2 = parts_total(ssq + static_cast<int64_t>(m) * nparts, nparts);
   const float rs = 1.0f / sqrtf(s2 / static_cast<float>(K) + eps);
   float v[8];
   split_sums(part, splits, static_cast<int64_t>(M) * N, static_cast<int64_t>(m) * N + n0 + ch * 8, v);
@@ -933,8 +973,7 @@ __global__ __launch_bounds__(256) void k_swiglu_reduce(const float* __restrict__
   const int m = blockIdx.x * RED_ROWS + r;
   if (m >= M) return;
   const int nparts = K / SSQ_COLS;
-  float s2 = 0.f;
-  for (int i = 0; i < nparts; ++i) s2 += ssq[static_cast<int64_t>(m) * nparts + i];
+  const float s2 = parts_total(ssq + static_cast<int64_t>(m) * nparts, nparts);
   const float rs = 1.0f / sqrtf(s2 / static_cast<float>(K) + eps);
   float g[8], u[8], o[8];
   const int64_t plane = static_cast<int64_t>(M) * N, at = static_cast<int64_t>(m) * N + n0 + ch * 8;
@@ -950,16 +989,15 @@ __global__ __launch_bounds__(256) void k_swiglu_reduce(const float* __restrict__
 }
 
 // The unsplit K / V (or query) epilogue on split sums: the normed chunk bf16(sum * r_row), then k_norm,
-// RoPE and the cache write of kv_chunk_row.
-__global__ __launch_bounds__(256) void k_norm_kv_reduce(const float* __restrict__ part, int splits, int M, int N,
-                                                        KvArgs a) {
+// RoPE and the cache write of kv_chunk_row. `part` starts at the epilogue's first column, planes are M x N.
+__device__ __forceinline__ void norm_kv_reduce(const float* __restrict__ part, int splits, int M, int N, int cblk,
+                                               const KvArgs& a) {
   __shared__ uint4 img[RED_ROWS * 32];
-  const int t = threadIdx.x, r = t >> 5, ch = t & 31, n0 = blockIdx.y * BN;
+  const int t = threadIdx.x, r = t >> 5, ch = t & 31, n0 = cblk * BN;
   const int m = blockIdx.x * RED_ROWS + r;
   uint4 o = make_uint4(0u, 0u, 0u, 0u);
   if (m < M) {
-    float s2 = 0.f;
-    for (int i = 0; i < a.nparts; ++i) s2 += a.ssq[static_cast<int64_t>(m) * a.nparts + i];
+    const float s2 = parts_total(a.ssq + static_cast<int64_t>(m) * a.nparts, a.nparts);
     const float rs = 1.0f / sqrtf(s2 / a.h + a.eps);
     float v[8];
     split_sums(part, splits, static_cast<int64_t>(M) * N, static_cast<int64_t>(m) * N + n0 + ch * 8, v);
@@ -975,6 +1013,23 @@ __global__ __launch_bounds__(256) void k_norm_kv_reduce(const float* __restrict_
     ok = p >= 0 && p < a.pos_lim;
   }
   kv_chunk_row(a, L, [&](int c) { return image_chunk(img, r, c); }, ch, m, ok, rope_fetch(a, L, m, ok));
+}
+
+__global__ __launch_bounds__(256) void k_norm_kv_reduce(const float* __restrict__ part, int splits, int M, int N,
+                                                        KvArgs a) {
+  norm_kv_reduce(part, splits, M, N, blockIdx.y, a);
+}
+
+// The same for a product of several column groups, each with an epilogue of its own (queries; K / V; the output
+// gate, whose columns are copied): column blocks [0, c1) take a0, [c1, c2) a1, the rest a2. One product over [wq;
+// wgate; wkv] of at most 512 rows fills the CUs with fewer K splits than two or three: 37 rows of 8B width, the
+// products and this epilogue take 19 us, against 37 us as two products with an epilogue each.
+__global__ __launch_bounds__(256) void k_norm_attn_reduce(const float* __restrict__ part, int splits, int M, int N,
+                                                          KvArgs a0, KvArgs a1, KvArgs a2, int c1, int c2) {
+  const int y = blockIdx.y;                         // block-uniform
+  if (y < c1) norm_kv_reduce(part, splits, M, N, y, a0);
+  else if (y < c2) norm_kv_reduce(part + static_cast<int64_t>(c1) * BN, splits, M, N, y - c1, a1);
+  else norm_kv_reduce(part + static_cast<int64_t>(c2) * BN, splits, M, N, y - c2, a2);
 }
 
 // Adds a run's fp32 sums (acc) into the fp64 accumulator C for the tile at (m0, n0), rows < M. The sums go
@@ -2310,17 +2365,69 @@ extern "C" int rf_norm_qkv_rows(const uint16_t* x, int64_t ldx, const float* ssq
     KvArgs aq{s0, nparts, static_cast<float>(H), eps, hq, d, qnorm, norm_kind, cs, rot, q + r0 * ldq,
               q + r0 * ldq, static_cast<int64_t>(d), ldq, 0, pos + r0};
     aq.pos_lim = pos_limit;
-    const dim3 gq = reduce_grid(m, NQ), gkv = reduce_grid(m, NKV);
-    hipLaunchKernelGGL(k_norm_kv_reduce, gq, dim3(256), 0, stream, part, pl.splits, static_cast<int>(m),
-                       static_cast<int>(N), aq);
-    // the K / V columns [NQ, N): the partial planes' rows keep their stride N, the cache slot is the position
+    // the K / V columns [NQ, N): the cache slot is the position
     KvArgs akv{s0, nparts, static_cast<float>(H), eps, hkv, d, knorm, norm_kind, cs, rot, kbuf, vbuf, head_stride,
                row_stride, 0, pos + r0};
     akv.slot = pos + r0;
     akv.pos_lim = pos_limit;
-    hipLaunchKernelGGL(k_norm_kv_reduce, gkv, dim3(256), 0, stream, part + NQ, pl.splits, static_cast<int>(m),
-                       static_cast<int>(N), akv);
+    const int c1 = static_cast<int>(NQ / BN), c2 = static_cast<int>(N / BN);
+    hipLaunchKernelGGL(k_norm_attn_reduce, reduce_grid(m, N), dim3(256), 0, stream, part, pl.splits,
+                       static_cast<int>(m), static_cast<int>(N), aq, akv, akv, c1, c2);
   }
+  return check_launch(fn);
+}
+
+extern "C" int rf_norm_attn_rows(const uint16_t* x, int64_t ldx, const float* ssq, int64_t rows, int64_t H, float eps,
+                                 const uint16_t* w, int hq, int hkv, int d, const uint16_t* qnorm, const uint16_t* knorm,
+                                 int norm_kind, const uint16_t* cs, int rot, uint16_t* q, int64_t ldq, uint16_t* gate,
+                                 int64_t ldg, uint16_t* kbuf, uint16_t* vbuf, int64_t head_stride, int64_t row_stride,
+                                 int64_t slot_begin, int64_t cap, void* workspace, size_t ws_bytes, hipStream_t stream) {
+  const char* fn = "rf_norm_attn_rows";
+  if (!x || !ssq || !w || !cs || !q || !kbuf || !vbuf || !workspace) return fail(RF_EINVAL_ARG, "%s: null pointer", fn);
+  if (rows < 0 || rows > ROWS_MAX) return fail(RF_EINVAL_SHAPE, "%s: %lld rows (0 .. 512)", fn, (long long)rows);
+  if (H <= 0 || H % BK || H % SSQ_COLS)
+    return fail(RF_EINVAL_SHAPE, "%s: H = %lld must be a multiple of 256", fn, (long long)H);
+  if (d <= 0 || d % 8 || 256 % d || hq <= 0 || hkv <= 0 || (static_cast<int64_t>(hq) * d) % BN ||
+      (2ll * hkv * d) % BN)
+    return fail(RF_EUNSUPPORTED, "%s: head_dim %d, %d query / %d kv heads (need 256 %% d == 0, d %% 8 == 0, hq d and "
+                "2 hkv d multiples of 256)", fn, d, hq, hkv);
+  if (rot <= 0 || rot > d || rot % 2 || ((rot / 2) % 8 && rot / 2 != 4))
+    return fail(RF_EUNSUPPORTED, "%s: rotary dims %d of head_dim %d", fn, rot, d);
+  if ((qnorm || knorm) && norm_kind != 0 && norm_kind != 1) return fail(RF_EINVAL_ARG, "%s: norm_kind %d", fn, norm_kind);
+  const int64_t NQ = static_cast<int64_t>(hq) * d, NKV = 2ll * hkv * d, N = (gate ? 2 : 1) * NQ + NKV;
+  if (ldx < H || ldx % 8 || ldx > (1 << 21) || ldq < NQ || ldq % 8 || (gate && (ldg < NQ || ldg % 8)) ||
+      head_stride % 8 || row_stride % 8 || row_stride < d)
+    return fail(RF_EINVAL_SHAPE, "%s: strides (ldx %lld, ldq %lld, ldg %lld, head %lld, row %lld)", fn, (long long)ldx,
+                (long long)ldq, (long long)ldg, (long long)head_stride, (long long)row_stride);
+  if (slot_begin < 0 || slot_begin + rows > cap)
+    return fail(RF_EINVAL_SHAPE, "%s: rows [%lld, %lld) exceed cache capacity %lld", fn, (long long)slot_begin,
+                (long long)(slot_begin + rows), (long long)cap);
+  if (!aligned16(x) || !aligned16(w) || !aligned16(q) || !aligned16(kbuf) || !aligned16(vbuf) || !aligned16(cs) ||
+      !aligned16(workspace) || (gate && !aligned16(gate)) || (qnorm && !aligned16(qnorm)) || (knorm && !aligned16(knorm)))
+    return fail(RF_EINVAL_SHAPE, "%s: pointers must be 16-byte aligned", fn);
+  if (!(eps >= 0.f)) return fail(RF_EINVAL_ARG, "%s: eps %g", fn, static_cast<double>(eps));
+  if (rows == 0) return RF_OK;
+  const Plan pl = plan(rows, N, H);
+  const size_t need = split_bytes(rows, N, H);
+  if (ws_bytes < need)
+    return fail(RF_EINVAL_ARG, "%s: workspace %zu bytes, needs %zu (rf_gemm_workspace_bytes of %lld x %lld x %lld)", fn,
+                ws_bytes, need, (long long)rows, (long long)N, (long long)H);
+  launch_partials(x, ldx, w, H, rows, N, H, pl, workspace, stream);
+  const int nparts = static_cast<int>(H / SSQ_COLS);
+  // [queries | gate | K | V] columns: the queries as K columns of hq heads, the gate as V columns (copied)
+  const KvArgs aq{ssq, nparts, static_cast<float>(H), eps, hq, d, qnorm, norm_kind, cs, rot, q, q,
+                  static_cast<int64_t>(d), ldq, 0, nullptr};
+  KvArgs ag = aq;
+  ag.hkv = 0;
+  ag.knorm = nullptr;
+  ag.kbuf = ag.vbuf = gate;
+  ag.row_stride = ldg;
+  const KvArgs akv{ssq, nparts, static_cast<float>(H), eps, hkv, d, knorm, norm_kind, cs, rot, kbuf, vbuf, head_stride,
+                   row_stride, slot_begin, nullptr};
+  const int c1 = static_cast<int>(NQ / BN), c2 = gate ? 2 * c1 : static_cast<int>(N / BN);
+  hipLaunchKernelGGL(k_norm_attn_reduce, reduce_grid(rows, N), dim3(256), 0, stream,
+                     static_cast<const float*>(workspace), pl.splits, static_cast<int>(rows), static_cast<int>(N), aq,
+                     gate ? ag : akv, akv, c1, c2);
   return check_launch(fn);
 }
 

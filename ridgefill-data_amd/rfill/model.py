@@ -336,8 +336,8 @@ class FillModel:
         input norm gain folded into the projections (rf_fold_norm; the zero-centred 1 + g for Qwen3.5):
         attention -- the query projection (Qwen3.5: its query and output-gate halves apart), q_norm, o_proj;
         GDN -- the z projection, the gated output norm's weight, out_proj; every layer -- [gate; up] with
-        the post-attention norm gain folded in (zero rows to a multiple of 256), down (zero columns to a
-        multiple of 64)."""
+        the post-attention norm gain folded in (each with zero rows to a multiple of 256), down (zero columns
+        to the same width)."""
         w = self._layer(i, self.layer_types[i])
         if "wo" in w:
             return w
@@ -349,11 +349,15 @@ class FillModel:
             wq = dev(a + "q_proj.weight")
             if self.arch == "qwen3_5":                  # per head [q | gate] rows (code/kva/model.py:427-432)
                 qg = wq.view(self.n_heads, 2, self.head_dim, wq.shape[1])
-                w["wq"] = ops.fold_norm(qg[:, 0].reshape(-1, wq.shape[1]).contiguous(), w["ln1"], kind)
-                w["wgate"] = ops.fold_norm(qg[:, 1].reshape(-1, wq.shape[1]).contiguous(), w["ln1"], kind)
-            else:                                       # [wq; wkv] in one buffer: the exact rows' one product
-                wqkv = torch.cat((ops.fold_norm(wq, w["ln1"], kind), w["wkv"]), 0)
-                w["wqkv"], w["wq"], w["wkv"] = wqkv, wqkv[:wq.shape[0]], wqkv[wq.shape[0]:]
+                parts = [ops.fold_norm(qg[:, j].reshape(-1, wq.shape[1]).contiguous(), w["ln1"], kind) for j in (0, 1)]
+            else:
+                parts = [ops.fold_norm(wq, w["ln1"], kind)]
+            # [wq; wgate; wkv] in one buffer: one product for few rows
+            wattn = torch.cat(parts + [w["wkv"]], 0)
+            nq, n = parts[0].shape[0], wattn.shape[0] - w["wkv"].shape[0]
+            w["wattn"], w["wq"], w["wkv"] = wattn, wattn[:nq], wattn[n:]
+            if n > nq:
+                w["wgate"] = wattn[nq:n]
             if self.arch != "llama":
                 w["q_norm"] = dev(a + "q_norm.weight")
             w["wo"] = dev(a + "o_proj.weight")
@@ -362,18 +366,14 @@ class FillModel:
             w["wz"] = ops.fold_norm(dev(a + "in_proj_z.weight"), w["ln1"], 1)
             w["gnorm"] = dev(a + "norm.weight")
             w["wo"] = dev(a + "out_proj.weight")
-        gate, up = dev(p + "mlp.gate_proj.weight"), dev(p + "mlp.up_proj.weight")
-        inter = gate.shape[0]
-        gu = torch.cat((gate, up), 0)
-        pad = (-gu.shape[0]) % 256
-        if pad:
-            gu = torch.cat((gu, gu.new_zeros(pad, gu.shape[1])), 0)
-        w["wgu"] = ops.fold_norm(gu, dev(p + "post_attention_layernorm.weight"), kind)
-        down = dev(p + "mlp.down_proj.weight")
-        pad = (-inter) % 64
-        if pad:
+        gate, up, down = (dev(p + f"mlp.{n}_proj.weight") for n in ("gate", "up", "down"))
+        pad = (-gate.shape[0]) % 256
+        if pad:                                         # zero gate and up rows give zero act columns
+            rows = gate.new_zeros(pad, gate.shape[1])
+            gate, up = torch.cat((gate, rows), 0), torch.cat((up, rows), 0)
             down = torch.cat((down, down.new_zeros(down.shape[0], pad)), 1).contiguous()
-        w["wd"], w["inter"] = down, inter
+        w["wgu"] = ops.fold_norm(torch.cat((gate, up), 0), dev(p + "post_attention_layernorm.weight"), kind)
+        w["wd"] = down
         return w
 
     def _gdn_forward_workspace(self, rows, device):
@@ -406,11 +406,13 @@ class FillModel:
         y = ops.gated_rms_norm(out, z, w["gnorm"], self.nv, self.dv, self.eps)
         return self._out_mlp(w, h, y)
 
-    def _gate(self, w, x, ssq, o):
-        """Qwen3.5's output gate: o * sigmoid(x_normed W_gate^T) in place (code/kva/model.py:444-445)."""
+    def _gate(self, w, x, ssq, o, g=None):
+        """Qwen3.5's output gate: o * sigmoid(x_normed W_gate^T) in place (code/kva/model.py:444-445); g: that
+        product if already formed."""
         if "wgate" in w:
-            g = ops.norm_linear(x, ssq, self.eps, w["wgate"],
-                                workspace=self.gemm_workspace(x.shape[0], w["wgate"].shape[0], x.shape[1], x.device))
+            if g is None:
+                g = ops.norm_linear(x, ssq, self.eps, w["wgate"],
+                                    workspace=self.gemm_workspace(x.shape[0], w["wgate"].shape[0], x.shape[1], x.device))
             ops.sigmoid_mul(o, g, out=o)
         return o
 
@@ -467,11 +469,11 @@ class FillModel:
                              workspace=self.gemm_workspace(R, wl["wkv"].shape[0], H, h.device, rows=True))
             return None
         w = self._pack_rows(i)
-        if "wqkv" in w:                                 # queries and the rows' K / V from one product
-            q = ops.norm_qkv_rows(h, ssq, self.eps, w["wqkv"], self.n_heads, self.n_kv, self.head_dim,
+        if "wgate" not in w:                            # queries and the rows' K / V from one product
+            q = ops.norm_qkv_rows(h, ssq, self.eps, w["wattn"], self.n_heads, self.n_kv, self.head_dim,
                                   w.get("q_norm"), w.get("k_norm"), self.knorm_kind, cs, rows, c["kbuf"], c["vbuf"],
                                   pos_max=rows_max,
-                                  workspace=self.gemm_workspace(R, w["wqkv"].shape[0], H, h.device, rows=True))
+                                  workspace=self.gemm_workspace(R, w["wattn"].shape[0], H, h.device, rows=True))
         else:
             ops.norm_kv_rows(h, ssq, self.eps, w["wkv"], self.n_kv, self.head_dim, w.get("k_norm"), self.knorm_kind,
                              cs, rows, c["kbuf"], c["vbuf"], pos_max=rows_max,
@@ -494,15 +496,8 @@ class FillModel:
         R, dev = h.shape[0], h.device
         gws = self.gemm_workspace
         h1, s1 = ops.map_apply_residual(o, w["wo"], h, workspace=gws(R, w["wo"].shape[0], w["wo"].shape[1], dev))
-        inter = w["inter"]
-        act = (torch.zeros if w["wd"].shape[1] != inter else torch.empty)(R, w["wd"].shape[1],
-                                                                          dtype=torch.bfloat16, device=dev)
         wgu = w["wgu"]
-        if wgu.shape[0] == 2 * inter and inter % 256 == 0:
-            ops.norm_linear_swiglu(h1, s1, self.eps, wgu, out=act, workspace=gws(R, wgu.shape[0], wgu.shape[1], dev))
-        else:                                           # [gate; up] padded to a multiple of 256 rows
-            gu = ops.norm_linear(h1, s1, self.eps, wgu, workspace=gws(R, wgu.shape[0], wgu.shape[1], dev))
-            ops.silu_mul(gu[:, :2 * inter], act[:, :inter])
+        act = ops.norm_linear_swiglu(h1, s1, self.eps, wgu, workspace=gws(R, wgu.shape[0], wgu.shape[1], dev))
         return ops.map_apply_residual(act, w["wd"], h1, workspace=gws(R, w["wd"].shape[0], w["wd"].shape[1], dev))
 
     def layer(self, i, h, pos, cache, ssq=None, cs=None):
@@ -524,20 +519,27 @@ class FillModel:
             cs = self.rope_table(pos)
         slot = self.reserve(c, T, self.n_kv, self.head_dim, h.device)
         H = h.shape[1]
-        ops.norm_kv_write(h, ssq, self.eps, w["wkv"], self.n_kv, self.head_dim, w.get("k_norm"), self.knorm_kind,
-                          cs, c["kbuf"], c["vbuf"], slot,
-                          workspace=self.gemm_workspace(T, w["wkv"].shape[0], H, h.device))
+        gate = None
+        if 0 < T <= ops.ROWS_MAX:                       # few rows: queries, gate, K and V from one product
+            q, gate = ops.norm_attn_rows(h, ssq, self.eps, w["wattn"], self.n_heads, self.n_kv, self.head_dim,
+                                         w.get("q_norm"), w.get("k_norm"), self.knorm_kind, cs, c["kbuf"], c["vbuf"],
+                                         slot, gate="wgate" in w,
+                                         workspace=self.gemm_workspace(T, w["wattn"].shape[0], H, h.device))
+        else:
+            ops.norm_kv_write(h, ssq, self.eps, w["wkv"], self.n_kv, self.head_dim, w.get("k_norm"), self.knorm_kind,
+                              cs, c["kbuf"], c["vbuf"], slot,
+                              workspace=self.gemm_workspace(T, w["wkv"].shape[0], H, h.device))
+            q = ops.norm_q(h, ssq, self.eps, w["wq"], self.n_heads, self.head_dim, w.get("q_norm"), self.knorm_kind, cs,
+                           torch.arange(T, device=h.device),
+                           workspace=self.gemm_workspace(T, w["wq"].shape[0], H, h.device))
         self.commit(c, T)
-        idx = torch.arange(T, device=h.device)
-        q = ops.norm_q(h, ssq, self.eps, w["wq"], self.n_heads, self.head_dim, w.get("q_norm"), self.knorm_kind, cs,
-                       idx, workspace=self.gemm_workspace(T, w["wq"].shape[0], H, h.device))
         if self._causal_ok():
             o = ops.attend_causal(q, slot, c["kbuf"], c["vbuf"], c["n"], self.n_heads, self.scale,
                                   workspace=self._causal_workspace(T, c["n"], h.device))
         else:
-            o = ops.attend_rows(q, idx + slot, c["kbuf"], c["vbuf"], c["n"], self.n_heads, self.scale,
-                                workspace=self._attn_workspace(T, c["n"], h.device))
-        return self._out_mlp(w, h, self._gate(w, h, ssq, o))
+            o = ops.attend_rows(q, torch.arange(slot, slot + T, device=h.device), c["kbuf"], c["vbuf"], c["n"],
+                                self.n_heads, self.scale, workspace=self._attn_workspace(T, c["n"], h.device))
+        return self._out_mlp(w, h, self._gate(w, h, ssq, o, gate))
 
     def embed(self, ids):
         """Embedding rows of token ids [T] (code/kva/model.py:108-109): a bit-exact row gather from the bf16

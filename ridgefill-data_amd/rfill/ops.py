@@ -98,6 +98,7 @@ def map_apply(b, w, c, out=None, ssq=None, workspace=None):
     return out, ssq
 
 
+ROWS_MAX = 512            # rows up to which a product runs as one of few rows (the library's ROWS_MAX)
 MAP_BATCH_MAX = 32        # layers per batched map / K-V launch (the library's per-layer pointer tables)
 
 
@@ -372,6 +373,37 @@ def norm_qkv_rows(x, ssq, eps, wqkv, hq, hkv, d, qnorm, knorm, norm_kind, cs, po
     return out
 
 
+def norm_attn_rows(x, ssq, eps, w, hq, hkv, d, qnorm, knorm, norm_kind, cs, kbuf, vbuf, slot_begin, gate=False,
+                   workspace="auto"):
+    """The queries, the output gate (gate) and the K / V of at most ROWS_MAX new rows from one product over w =
+    [wq; wgate; wkv] (without gate [wq; wkv]): queries [rows, hq d] as norm_q at table rows 0 .., the gate's
+    projection [rows, hq d] (None without gate) as norm_linear, and K / V into cache slots slot_begin .. as
+    norm_kv_write. Returns (queries, gate)."""
+    _need(x, "x", torch.bfloat16, 2)
+    _need(ssq, "ssq", torch.float32, 2)
+    _need(w, "w", torch.bfloat16, 2)
+    _need(cs, "cs", torch.bfloat16, 2)
+    rows, H = x.shape
+    n = ((2 if gate else 1) * hq + 2 * hkv) * d
+    if rows > ROWS_MAX or tuple(ssq.shape) != (rows, ssq_parts(H)) or not ssq.is_contiguous():
+        raise ValueError(f"norm_attn_rows: {rows} rows (at most {ROWS_MAX}), ssq {tuple(ssq.shape)}")
+    if tuple(w.shape) != (n, H) or not w.is_contiguous() or cs.shape[0] != rows or not cs.is_contiguous():
+        raise ValueError(f"norm_attn_rows: w {tuple(w.shape)}, expected ({n}, {H}); cs {tuple(cs.shape)}")
+    for name, t in (("qnorm", qnorm), ("knorm", knorm)):
+        if t is not None:
+            _need(t, name, torch.bfloat16, 1)
+            if t.shape[0] != d:
+                raise ValueError(f"norm_attn_rows: {name} width")
+    hs, rs, cap = _cache_args(kbuf, vbuf, hkv, d, slot_begin, rows)
+    out = torch.empty(2 if gate else 1, rows, hq * d, dtype=torch.bfloat16, device=x.device)
+    q, g = out[0], out[1] if gate else None
+    ws, nb = _ws(workspace, rows, n, H, x.device)
+    _lib.call("rf_norm_attn_rows", _ptr(x), x.stride(0), _ptr(ssq), rows, H, float(eps), _ptr(w), hq, hkv, d,
+              _ptr(qnorm), _ptr(knorm), int(norm_kind), _ptr(cs), cs.shape[1], _ptr(q), q.stride(0), _ptr(g),
+              g.stride(0) if gate else 0, _ptr(kbuf), _ptr(vbuf), hs, rs, int(slot_begin), cap, _ptr(ws), nb, _stream(x))
+    return q, g
+
+
 def rope_kv_write(k, v, cs, kbuf, vbuf, slot_begin):
     """fill_kv: RoPE on pre-RoPE k and the write of k / v [m, hkv, d] into rows [slot_begin, +m)."""
     for name, t in (("k", k), ("v", v)):
@@ -580,7 +612,7 @@ def norm_linear_swiglu(x, ssq, eps, w, out=None, workspace=None):
     if out.shape[0] != P or out.shape[1] < I:
         raise ValueError(f"norm_linear_swiglu: out {tuple(out.shape)} for {P} rows of {I}")
     ws, nb = _ws(workspace, P, 2 * I, H, x.device)
-    fused = ws is not None and P <= 512
+    fused = ws is not None and P <= ROWS_MAX
     gu = None if fused else torch.empty(P, 2 * I, dtype=torch.bfloat16, device=x.device)
     _lib.call("rf_norm_linear_swiglu", _ptr(x), x.stride(0), _ptr(ssq), P, H, float(eps), _ptr(w), I, _ptr(out),
               out.stride(0), _ptr(gu), 0 if gu is None else gu.stride(0), _ptr(ws), nb, _stream(x))

@@ -445,3 +445,54 @@ def test_fused_residual_and_swiglu_epilogues_are_bit_identical(dev, R):
     torch.cuda.synchronize()
     assert torch.equal(h1, want_h1) and torch.equal(s1, want_s1)
     assert torch.equal(act, want_act)
+
+
+@pytest.mark.parametrize("rows,H,hq,hkv,d,rot,gate,norms", [
+    (1, 256, 4, 2, 64, 64, False, False), (37, 1024, 8, 2, 128, 128, False, True), (512, 1024, 8, 2, 128, 128, False, False),
+    (9, 2048, 16, 2, 256, 64, True, True), (161, 1280, 4, 1, 256, 64, True, True)])
+def test_norm_attn_rows_matches_the_separate_products(dev, rows, H, hq, hkv, d, rot, gate, norms):
+    """rf_norm_attn_rows (one row, odd counts, the most rows; one and two row blocks; statistics of 1, 4, 5 and 8
+    partials; with the output gate and partial rotary) against norm_q, norm_linear and norm_kv_write of the same
+    weights without a split: only the fp32 order of the K splits differs, i.e. bf16 rounding (5e-3 as above). Other
+    cache slots stay as they were."""
+    from rfill import ops
+    g = torch.Generator().manual_seed(rows + H)
+    n, slot, cap = ((2 if gate else 1) * hq + 2 * hkv) * d, 77, 700
+    x = torch.randn(rows, H, generator=g).to(torch.bfloat16).to(dev)
+    ssq = ops.row_ssq(x)
+    w = (torch.randn(n, H, generator=g) / H ** 0.5).to(torch.bfloat16).to(dev)
+    qn, kn = [(1 + 0.1 * torch.randn(d, generator=g)).to(torch.bfloat16).to(dev) if norms else None for _ in range(2)]
+    kind = 1 if gate else 0
+    cs = ops.rope_table(torch.arange(slot, slot + rows, device=dev), ops.inv_freq_default(1e6, rot).to(dev))
+    kb, vb, kb2, vb2 = (torch.full((hkv, cap, d), 3.0, dtype=torch.bfloat16, device=dev) for _ in range(4))
+    q, gt = ops.norm_attn_rows(x, ssq, 1e-6, w, hq, hkv, d, qn, kn, kind, cs, kb, vb, slot, gate=gate)
+    wq, wkv = w[:hq * d], w[n - 2 * hkv * d:]
+    q2 = ops.norm_q(x, ssq, 1e-6, wq, hq, d, qn, kind, cs, torch.arange(rows, device=dev))
+    ops.norm_kv_write(x, ssq, 1e-6, wkv, hkv, d, kn, kind, cs, kb2, vb2, slot)
+    torch.cuda.synchronize()
+    pairs = [(q, q2), (kb[:, slot:slot + rows], kb2[:, slot:slot + rows]), (vb[:, slot:slot + rows], vb2[:, slot:slot + rows])]
+    if gate:
+        pairs.append((gt, ops.norm_linear(x, ssq, 1e-6, w[hq * d:2 * hq * d])))
+    for got, want in pairs:
+        assert rel_err(got, want) < 5e-3
+    for t in (kb, vb):
+        assert bool((t[:, :slot] == 3.0).all()) and bool((t[:, slot + rows:] == 3.0).all())
+
+
+@pytest.mark.parametrize("nq,n_keys,hq,hkv,d", [(1, 300, 4, 4, 64), (37, 3038, 32, 8, 128), (5, 9000, 8, 1, 64),
+                                                (17, 8193, 16, 2, 256), (33, 20000, 2, 2, 256), (3, 257, 8, 2, 128)])
+def test_causal_splits_of_few_queries_match_one_pass(dev, nq, n_keys, hq, hkv, d):
+    """Few queries over many keys: the key-range splits (up to 64 of them, counts that are not a multiple of the
+    combine's batches) against one pass (a workspace that holds no split): fp32 sums in another order before one
+    bf16 rounding (2^-8 of a value; 4e-3 of the norm)."""
+    from rfill import ops
+    g = torch.Generator().manual_seed(n_keys)
+    q = torch.randn(nq, hq * d, generator=g).to(torch.bfloat16).to(dev)
+    kb, vb = (torch.randn(hkv, n_keys + 3, d, generator=g).to(torch.bfloat16).to(dev) for _ in range(2))
+    slot = n_keys - nq
+    need = ops.attend_causal_workspace_bytes(nq, hq, hkv, d, n_keys)
+    assert need > 0
+    got = ops.attend_causal(q, slot, kb, vb, n_keys, hq, d ** -0.5,
+                            workspace=torch.full((need,), 0xFF, dtype=torch.uint8, device=dev))
+    want = ops.attend_causal(q, slot, kb, vb, n_keys, hq, d ** -0.5, workspace=torch.empty(16, dtype=torch.uint8, device=dev))
+    assert rel_err(got, want) < 4e-3
