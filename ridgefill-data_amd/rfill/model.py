@@ -352,10 +352,11 @@ class FillModel:
                 parts = [ops.fold_norm(qg[:, j].reshape(-1, wq.shape[1]).contiguous(), w["ln1"], kind) for j in (0, 1)]
             else:
                 parts = [ops.fold_norm(wq, w["ln1"], kind)]
-            # [wq; wgate; wkv] in one buffer: one product for few rows
+            # [wq; wgate; wkv] in one buffer: one product for few rows. The fill's own wkv stays where it is: a
+            # captured fill or one on another stream may still read it
             wattn = torch.cat(parts + [w["wkv"]], 0)
             nq, n = parts[0].shape[0], wattn.shape[0] - w["wkv"].shape[0]
-            w["wattn"], w["wq"], w["wkv"] = wattn, wattn[:nq], wattn[n:]
+            w["wattn"], w["wq"] = wattn, wattn[:nq]
             if n > nq:
                 w["wgate"] = wattn[nq:n]
             if self.arch != "llama":
