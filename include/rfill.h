@@ -510,7 +510,7 @@ int rf_read_cosine(const uint16_t* pred, int64_t ld_pred, const uint16_t* truth,
  * target side by side), written to w + l w_stride as [d, R] (row stride ldw); and, if bias is not NULL,
  * bias + l bias_stride = mean_y - mean_x W_lam ([R]; mean_x [d], mean_y [R] on the device): the unpenalised
  * bias of the centred fit. The inverse of C + lam scale I comes from a block recursion on its Schur
- * complements over a 64 x 64 Gauss-Jordan base (the matrix padded with an identity block to a multiple of 64)
+ * complements over a 128 x 128 Gauss-Jordan base (the matrix padded with an identity block to a multiple of 128)
  * and every product runs on fp64 MFMA; the reference's eigendecomposition gives the same closed form.
  * Needs d, R, ldb, ldw even; cxy, w, mean_x and the workspace 16-byte aligned; a workspace of
  * rf_ridge_solve_workspace_bytes(d, nlam) bytes. */
@@ -518,6 +518,14 @@ int rf_ridge_solve(const double* cxx, int64_t ldc, int64_t d, const double* cxy,
                    const double* mean_x, const double* mean_y, const double* lams, int nlam, double scale, double* w,
                    int64_t ldw, int64_t w_stride, double* bias, int64_t bias_stride, void* workspace, size_t ws_bytes,
                    hipStream_t stream);
+
+/* The same solve for `targets` targets of `width` columns each (cxy [d, targets width], target j's columns from
+ * j width), the weights rounded to fp32 in F.linear layout: wt[j] (host array of device pointers) is target j's
+ * [nlam, width, d]. bias [nlam, targets width] in fp64, may be null. Width even; the rest as rf_ridge_solve. */
+int rf_ridge_solve_wt(const double* cxx, int64_t ldc, int64_t d, const double* cxy, int64_t ldb, int targets,
+                      int64_t width, const double* mean_x, const double* mean_y, const double* lams, int nlam,
+                      double scale, float* const* wt, double* bias, int64_t bias_stride, void* workspace,
+                      size_t ws_bytes, hipStream_t stream);
 
 /* Bytes of rf_ridge_solve's workspace for dimension d and nlam lambdas (up to 8 are inverted together).
  * Host only. */

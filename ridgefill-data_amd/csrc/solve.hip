@@ -2,24 +2,26 @@
 // W(lam) = (C + lam s I)^-1 Cxy with s = mean(diag C), by one eigendecomposition of C; this computes the same
 // closed form through the inverse of C + lam s I).
 //
-//   k_dgemm       C = alpha A B + beta C, row-major fp64, v_mfma_f64_16x16x4f64. A workgroup of 4 wave64s
-//                 computes a 128 x 128 tile over K in 16-deep blocks; each wave a 64 x 64 quarter as 4 x 4
-//                 MFMA tiles (lane l feeds A[l % 16][l / 16] and B[l / 16][l % 16] and holds
+//   k_dgemm       C = alpha op(A) op(B) + beta Ci, row-major fp64, v_mfma_f64_16x16x4f64. A workgroup of 4 wave64s
+//                 computes a T x T tile (128, 64 or 32) over K in BK-deep blocks; each wave a T/2 x T/2 quarter of
+//                 16 x 16 MFMA tiles (lane l feeds A[l % 16][l / 16] and B[l / 16][l % 16] and holds
 //                 D[l / 16 + 4 i][l % 16] in its register pair i: the fp64 output's rows interleave, unlike the
-//                 fp32 16x16x4 variant's 4 (l / 16) + i). Blocks are double-buffered in LDS (72 KB, so two
-//                 workgroups share a CU and fill each other's barrier and LDS-latency gaps), the next block
-//                 loaded into registers while the current one is multiplied. LDS strides: A rows of 18 doubles and B rows of 144 doubles, so
-//                 the 16 rows x 2 k (A) and 16 columns x 2 k (B) of each half-wave's fragment reads fall in
-//                 distinct banks. The k order of the sums is that of one pass over K in steps of 4.
-//   k_spd_inv64   the inverse of a 64 x 64 symmetric positive definite block by in-place Gauss-Jordan
-//                 elimination without pivoting (stable for SPD matrices), one workgroup, the matrix in
-//                 registers and each step's pivot row and column exchanged through LDS.
-//   the inverse   of an n x n SPD matrix (n a multiple of 64) by block recursion on [A11 A12; A21 A22]:
-//                 X11 = A11^-1, T = A21 X11, S = A22 - T A12 (the Schur complement, SPD), X22 = S^-1,
-//                 X21 = -X22 T, U = X11 A12 (= T^T), X11 -= U X21, X12 = X21^T -- every product a k_dgemm.
+//                 fp32 16x16x4 variant's 4 (l / 16) + i). Blocks are double-buffered in LDS (72 KB at T 128, BK 16,
+//                 so two workgroups share a CU and fill each other's barrier and LDS-latency gaps), the next block
+//                 loaded into registers while the current one is multiplied. LDS rows of BK + 2 doubles (k
+//                 contiguous) or T + 16 (k-major), so the fragment reads of each half-wave fall in distinct
+//                 banks. The k order of the sums is that of one pass over K in steps of 4.
+//   k_spd_inv128  the inverse of a 128 x 128 symmetric positive definite block, one workgroup (below).
+//   the inverse   of an n x n SPD matrix (n a multiple of 128, its lower triangle) by block recursion on
+//                 [A11 .; A21 A22]: X11 = A11^-1, T = A21 X11, S = A22 - T A21^T (the Schur complement, SPD),
+//                 X22 = S^-1, X21 = -X22 T, X11 -= T^T X21, X12 = X21^T. Symmetric results are computed on their
+//                 lower tiles only; the product that forms X21 stores X12 too. d 4096, three lambdas: 8.0 ms for
+//                 the inverses (19.7 with 64 x 64 leaves, every product in full and separate copies and
+//                 transposes), one lambda 4.5 (15.8), d 1024 0.7 (3.1).
 //   k_gemv_rows   out = init + alpha v M, rows summed by 4 waves in order (the bias's vector products).
-//   rf_ridge_solve  per lambda: A = C + lam s I padded to a multiple of 64 with an identity block, X = A^-1,
-//                 W = X[:d, :d] Cxy (k_dgemm, the dominant 2 d^2 R flops), bias = mean_y - (mean_x X) Cxy
+//   rf_ridge_solve  per lambda: A = C + lam s I padded to a multiple of 128 with an identity block, X = A^-1,
+//                 W = X[:d, :d] Cxy (k_dgemm, or k_solve_wt's W^T; the dominant 2 d^2 R flops, 26.6 ms for four
+//                 targets of 4096 and three lambdas, 79 % of the fp64 MFMA peak), bias = mean_y - (mean_x X) Cxy
 //                 (= mean_y - mean_x W; one pass over Cxy for every lambda). Up to 8 lambdas go together:
 //                 every launch of the recursion carries all of them in its grid.
 #include <algorithm>
@@ -31,152 +33,293 @@ namespace {
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-constexpr int DBM = 128, DBN = 128, DBK = 16;
-constexpr int AST = DBK + 2;      // A block row stride in doubles (16-byte aligned rows, conflict-free reads)
-constexpr int DLD = DBM * DBK / 2 / 256;   // double2 loads per thread per block and operand (A; B has the same)
-constexpr int BST = DBN + 16;     // B block row stride in doubles
-
+// C = alpha op(A) op(B) + beta Ci for each matrix of a batch (blockIdx.y, element strides s*).
 struct DgemmArgs {
-  const double* A;
+  const double* A;        // [M, K], or with AT [K, M]
   int64_t lda;
-  const double* B;
+  const double* B;        // [K, N], or with BT [N, K]
   int64_t ldb;
   double* C;
   int64_t ldc;
   int M, N, K;
   double alpha, beta;
-  int64_t sa, sb, sc;     // element strides between the batch's matrices (blockIdx.y)
+  int64_t sa, sb, sc;
+  const double* Ci;       // read when beta != 0 (may be C itself)
+  int64_t ldci, sci;
+  double* Ct;             // if given: C^T is stored there too (with lower: its tiles above the diagonal)
+  int64_t ldct, sct;
+  int lower;              // M == N: only the tiles on and below the diagonal are computed
 };
 
-// Requires K and N even, lda / ldb even, A and B 16-byte aligned (checked by the host callers). Loads past
-// M, N or K read a clamped in-bounds address and are replaced by zeros (no divergent branches in the loop).
-__global__ __launch_bounds__(256, 2) void k_dgemm(DgemmArgs a) {
-  __shared__ __align__(16) double As[2][DBM * AST];
-  __shared__ __align__(16) double Bs[2][DBK * BST];
+// A T x T tile per workgroup, K in BK-deep blocks. Requires K and N even (with AT also M), even strides and
+// 16-byte aligned operands (checked by the host callers). Loads past M, N or K read a clamped in-bounds address
+// and are replaced by zeros (no divergent branches in the loop).
+// T and BK: the solve's large products take 128 and 16 (two workgroups per CU); the inverse's take the largest
+// tile that still gives the batch about a workgroup per CU, with deeper K blocks for the smaller tiles, whose
+// time is the chain of loads, barriers and MFMAs of one workgroup (64 x 64 x 64 took 21 us in a 128 x 128 tile
+// with 16-deep blocks, most of it waiting).
+// store(row, col, value) takes the elements inside M x N; ROWS_FAST: the order of the tiles in flight.
+template <int T, int BK, bool AT, bool BT, bool ROWS_FAST, class Store>
+__device__ __forceinline__ void dgemm(const DgemmArgs& a, Store store) {
+  constexpr int MT = T / 32;                      // 16 x 16 MFMA tiles per wave and dimension
+  constexpr int RST = BK + 2, CST = T + 16;       // LDS row strides in doubles: [T][BK] and [BK][T] images
+  constexpr int LD = T * BK / 512;                // double2 loads per thread, block and operand
+  constexpr int AS = AT ? BK * CST : T * RST, BS = BT ? T * RST : BK * CST;
+  __shared__ __align__(16) double As[2][AS];
+  __shared__ __align__(16) double Bs[2][BS];
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6), wm = w >> 1, wn = w & 1;
-  // tile rows fastest: the blocks in flight share B's column panels (B is the large operand of the solve)
-  const int tiles_m = (a.M + DBM - 1) / DBM;
-  const int tn = blockIdx.x / tiles_m, tm = blockIdx.x - tn * tiles_m;
-  const int m0 = tm * DBM, n0 = tn * DBN;
+  int tm, tn;
+  if (a.lower) {
+    tm = static_cast<int>((sqrtf(8.f * static_cast<float>(blockIdx.x) + 1.f) - 1.f) * 0.5f);
+    while (tm * (tm + 1) / 2 > static_cast<int>(blockIdx.x)) --tm;
+    while ((tm + 1) * (tm + 2) / 2 <= static_cast<int>(blockIdx.x)) ++tm;
+    tn = static_cast<int>(blockIdx.x) - tm * (tm + 1) / 2;
+  } else {                                        // the fast direction's blocks share the other's panel
+    const int per = ((ROWS_FAST ? a.M : a.N) + T - 1) / T, q = blockIdx.x / per, r = blockIdx.x - q * per;
+    tm = ROWS_FAST ? r : q;
+    tn = ROWS_FAST ? q : r;
+  }
+  const int m0 = tm * T, n0 = tn * T;
   const int64_t z = blockIdx.y;
   const double* __restrict__ Ag = a.A + z * a.sa;
   const double* __restrict__ Bg = a.B + z * a.sb;
-  double* __restrict__ Cg = a.C + z * a.sc;
-  // loader mapping: A chunk j = t + 256 i: row j / 8, k pair j % 8; B chunk j: k row j / 64, column pair j % 64
-  // the zero masks are applied when the block is written to LDS, after the multiply that hides the loads
-  double2 ra[DLD], rb[DLD];
+  double2 ra[LD], rb[LD];
   unsigned ok = 0;
+  // chunk j = t + 256 i of a [T][BK] image: row j / (BK / 2), k pair j % (BK / 2); of a [BK][T] image: k row
+  // j / (T / 2), column pair j % (T / 2). The zero masks are applied when the block is written to LDS, after
+  // the multiply that hides the loads.
+  auto load_one = [&](const double* __restrict__ g, int64_t ld, int r0, int R, int k0, bool kmajor, int j, bool& in) {
+    const int r = kmajor ? r0 + 2 * (j % (T / 2)) : r0 + j / (BK / 2);
+    const int k = kmajor ? k0 + j / (T / 2) : k0 + 2 * (j % (BK / 2));
+    in = r < R && k < a.K;
+    const int rc = kmajor ? min(r, R - 2) : min(r, R - 1), kc = kmajor ? min(k, a.K - 1) : min(k, a.K - 2);
+    return *reinterpret_cast<const double2*>(kmajor ? g + static_cast<int64_t>(kc) * ld + rc
+                                                    : g + static_cast<int64_t>(rc) * ld + kc);
+  };
   auto gload = [&](int k0) {
     ok = 0;
 #pragma unroll
-    for (int i = 0; i < DLD; ++i) {
-      const int j = t + 256 * i;
-      const int ar = j >> 3, ak = k0 + 2 * (j & 7);
-      const int gr = m0 + ar;
-      ok |= (gr < a.M && ak < a.K) ? 1u << i : 0u;
-      ra[i] = *reinterpret_cast<const double2*>(Ag + static_cast<int64_t>(min(gr, a.M - 1)) * a.lda +
-                                                min(ak, a.K - 2));
-      const int bk = k0 + (j >> 6), bc = n0 + 2 * (j & 63);
-      ok |= (bk < a.K && bc < a.N) ? 1u << (DLD + i) : 0u;
-      rb[i] = *reinterpret_cast<const double2*>(Bg + static_cast<int64_t>(min(bk, a.K - 1)) * a.ldb +
-                                                min(bc, a.N - 2));
+    for (int i = 0; i < LD; ++i) {
+      bool in;
+      ra[i] = load_one(Ag, a.lda, m0, a.M, k0, AT, t + 256 * i, in);
+      ok |= in ? 1u << i : 0u;
+      rb[i] = load_one(Bg, a.ldb, n0, a.N, k0, !BT, t + 256 * i, in);
+      ok |= in ? 1u << (LD + i) : 0u;
     }
+  };
+  auto put = [&](double* s, bool kmajor, int j, bool in, const double2& v) {
+    const int at = kmajor ? j / (T / 2) * CST + 2 * (j % (T / 2)) : j / (BK / 2) * RST + 2 * (j % (BK / 2));
+    *reinterpret_cast<double2*>(s + at) = double2{in ? v.x : 0.0, in ? v.y : 0.0};
   };
   auto swrite = [&](int s) {
 #pragma unroll
-    for (int i = 0; i < DLD; ++i) {
-      const int j = t + 256 * i;
-      const bool ka = (ok >> i) & 1, kb = (ok >> (DLD + i)) & 1;
-      const double2 va{ka ? ra[i].x : 0.0, ka ? ra[i].y : 0.0}, vb{kb ? rb[i].x : 0.0, kb ? rb[i].y : 0.0};
-      *reinterpret_cast<double2*>(&As[s][(j >> 3) * AST + 2 * (j & 7)]) = va;
-      *reinterpret_cast<double2*>(&Bs[s][(j >> 6) * BST + 2 * (j & 63)]) = vb;
+    for (int i = 0; i < LD; ++i) {
+      put(As[s], AT, t + 256 * i, (ok >> i) & 1, ra[i]);
+      put(Bs[s], !BT, t + 256 * i, (ok >> (LD + i)) & 1, rb[i]);
     }
   };
-  f64x4 acc[4][4];
+  f64x4 acc[MT][MT];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = f64x4{0.0, 0.0, 0.0, 0.0};
-  const int nkb = (a.K + DBK - 1) / DBK;
+    for (int nt = 0; nt < MT; ++nt) acc[mt][nt] = f64x4{0.0, 0.0, 0.0, 0.0};
+  const int nkb = (a.K + BK - 1) / BK;
   gload(0);
   swrite(0);
   __syncthreads();
   const int lr = lane & 15, lk = lane >> 4;
+  const int ma = wm * (T / 2) + lr, nb = wn * (T / 2) + lr;
   for (int kb = 0; kb < nkb; ++kb) {
     const int s = kb & 1;
-    if (kb + 1 < nkb) gload((kb + 1) * DBK);
-    const double* as = As[s] + (wm * 64 + lr) * AST + lk;
-    const double* bs = Bs[s] + lk * BST + wn * 64 + lr;
+    if (kb + 1 < nkb) gload((kb + 1) * BK);
+    const double* as = AT ? As[s] + lk * CST + ma : As[s] + ma * RST + lk;
+    const double* bs = BT ? Bs[s] + nb * RST + lk : Bs[s] + lk * CST + nb;
 #pragma unroll
-    for (int kk = 0; kk < DBK / 4; ++kk) {
-      double af[4], bf[4];
+    for (int kk = 0; kk < BK / 4; ++kk) {
+      double af[MT], bf[MT];
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt) af[mt] = as[mt * 16 * AST + kk * 4];
+      for (int mt = 0; mt < MT; ++mt) af[mt] = AT ? as[kk * 4 * CST + mt * 16] : as[mt * 16 * RST + kk * 4];
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) bf[nt] = bs[kk * 4 * BST + nt * 16];
+      for (int nt = 0; nt < MT; ++nt) bf[nt] = BT ? bs[nt * 16 * RST + kk * 4] : bs[kk * 4 * CST + nt * 16];
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
+        for (int nt = 0; nt < MT; ++nt)
           acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[mt], bf[nt], acc[mt][nt], 0, 0, 0);
     }
     if (kb + 1 < nkb) swrite(s ^ 1);                // stage s ^ 1 was last read before the previous barrier
     __syncthreads();
   }
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int col = n0 + wn * 64 + nt * 16 + lr;
+    for (int nt = 0; nt < MT; ++nt) {
+      const int col = n0 + nb + nt * 16;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int64_t row = static_cast<int64_t>(m0) + wm * 64 + mt * 16 + lk + 4 * i;
-        if (row < a.M && col < a.N) {
-          double* c = Cg + row * a.ldc + col;
-          double v = a.alpha * acc[mt][nt][i];
-          if (a.beta != 0.0) v += a.beta * *c;
-          *c = v;
-        }
+        const int row = m0 + wm * (T / 2) + mt * 16 + lk + 4 * i;
+        if (row < a.M && col < a.N) store(row, col, a.alpha * acc[mt][nt][i], tm != tn);
       }
     }
 }
 
-// X = A^-1 for a 64 x 64 SPD block: Gauss-Jordan elimination in place, thread t keeping row t / 4, columns
-// 16 (t % 4) .. + 15 in registers. Step k: p = M[k][k]; row k /= p (M[k][k] = 1 / p); every other row i:
-// M[i][j] -= M[i][k] M[k][j] (j != k), M[i][k] = -M[i][k] / p. Row k and column k as they were before the
-// step are published in LDS (double-buffered by step parity, one barrier per step); the 64 steps are
-// unrolled so that every register index is a constant.
-__global__ __launch_bounds__(256) void k_spd_inv64(const double* __restrict__ A, int64_t lda, double* __restrict__ X,
-                                                   int64_t ldx, int64_t sa, int64_t sx) {
-  __shared__ double prow[2][64], pcol[2][64];
-  const int t = threadIdx.x, r = t >> 2, q = t & 3, c0 = q * 16;
-  A += static_cast<int64_t>(blockIdx.x) * sa;           // one block per matrix of the batch
+template <int T, int BK, bool AT, bool BT>
+__global__ __launch_bounds__(256, T == 32 ? 1 : 2) void k_dgemm(DgemmArgs a) {
+  const int64_t z = blockIdx.y;
+  double* C = a.C + z * a.sc;
+  const double* Ci = a.Ci + z * a.sci;
+  double* Ct = a.Ct ? a.Ct + z * a.sct : nullptr;
+  dgemm<T, BK, AT, BT, true>(a, [&](int64_t row, int64_t col, double v, bool off_diagonal) {
+    if (a.beta != 0.0) v += a.beta * Ci[row * a.ldci + col];
+    C[row * a.ldc + col] = v;
+    if (Ct && (off_diagonal || !a.lower)) Ct[col * a.ldct + row] = v;
+  });
+}
+
+// The weights in F.linear layout, W^T = Cxy^T X (X symmetric), rounded to fp32 where they are formed: row j width + r
+// of the product is output r of target j. A pass that transposed and rounded fp64 weights afterwards took 1.2 ms for
+// four targets and three lambdas at d 4096, beside writing and keeping them in fp64 (1.6 GB).
+constexpr int WT_TARGETS = 64;
+struct WtOut {
+  float* p[WT_TARGETS];     // per target: [lambda][width][d]
+  int width;
+};
+__global__ __launch_bounds__(256, 2) void k_solve_wt(DgemmArgs a, WtOut o) {
+  const int64_t z = blockIdx.y, d = a.N;
+  dgemm<128, 16, true, false, false>(a, [&](int row, int col, double v, bool) {
+    const int j = row / o.width, r = row - j * o.width;
+    o.p[j][(z * o.width + r) * d + col] = static_cast<float>(v);
+  });
+}
+
+// A double of the lane in row position n of this lane's 16-lane row (DPP row_newbcast).
+template <int n>
+__device__ __forceinline__ double row_bcast(double v) {
+  const int2 u = __builtin_bit_cast(int2, v);
+  return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_update_dpp(0, u.x, 0x150 + n, 0xf, 0xf, true),
+                                              __builtin_amdgcn_update_dpp(0, u.y, 0x150 + n, 0xf, 0xf, true)));
+}
+
+// One elimination step KK of a wave's 16 x 16 inverse: lane (r = l % 16, g = l / 16) holds row r, columns 4 g ..
+// 4 g + 3. p = M[KK][KK]; row KK /= p (M[KK][KK] = 1 / p); every other row: M[r][j] -= M[r][KK] / p M[KK][j],
+// M[r][KK] = -M[r][KK] / p.
+template <int KK>
+__device__ __forceinline__ void inv16_step(double (&m)[4], int r, int g) {
+  constexpr int GK = KK / 4, EK = KK & 3;
+  const double rinv = 1.0 / __shfl(m[EK], GK * 16 + KK, 64);
+  const double f = __shfl(m[EK], GK * 16 + r, 64) * rinv;       // M[r][KK] / p
+  const bool own = r == KK;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const double prow = row_bcast<KK>(m[e]);
+    const double v = own ? prow * rinv : m[e] - f * prow;
+    m[e] = (e == EK && g == GK) ? (own ? rinv : -f) : v;
+  }
+}
+
+constexpr int LEAF = 128;
+
+// X = A^-1 for a 128 x 128 SPD block (its lower triangle is read), one workgroup of 4 wave64s per matrix: blocked
+// Gauss-Jordan without pivoting (stable for SPD matrices) in 16-wide block steps. The matrix stays in registers as
+// MFMA accumulators, wave w holding block rows 2 w and 2 w + 1. Step k, with P = M[k][k]^-1, R the block row k and
+// C the block column k before the step (both published in LDS, double-buffered, one barrier per step):
+//   G_i = C_i P;  M[i][j] -= G_i R_j (i, j != k);  M[i][k] = -G_i;  M[k][j] = P R_j;  M[k][k] = P.
+// Every wave forms P itself (inv16_step, lane = row and column group) rather than wait for one that does. P is
+// symmetric up to rounding, so a lane's P[l % 16][4 s + l / 16] serves as A and as B operand of k-step s;
+// G_i^T = P C_i^T comes out of the MFMA in the A operand's order, so no product passes through LDS.
+// Bound by its chain: 8 steps of 16 dependent eliminations and 72 MFMAs a wave. It replaces two 64 x 64 leaves of
+// 64 elimination steps each (37 us a launch) and the seven launches that joined them (about 20 us a product).
+__global__ __launch_bounds__(256, 1) void k_spd_inv128(const double* __restrict__ A, int64_t lda,
+                                                       double* __restrict__ X, int64_t ldx, int64_t sa, int64_t sx) {
+  constexpr int NB = LEAF / 16, RS = LEAF + 16, CS = 18;
+  __shared__ __align__(16) double Rp[2][16 * RS];       // block row k: [16][128]
+  __shared__ __align__(16) double Cp[2][LEAF * CS];     // block column k: [128][16]
+  A += static_cast<int64_t>(blockIdx.x) * sa;
   X += static_cast<int64_t>(blockIdx.x) * sx;
-  double m[16];
+  const int t = threadIdx.x, lane = t & 63, lr = lane & 15, g = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  f64x4 m[2][NB];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) m[j] = A[static_cast<int64_t>(r) * lda + c0 + j];
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-  for (int k = 0; k < 64; ++k) {
-    const int b = k & 1;
-    if (r == k) {
+    for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int j = 0; j < 16; ++j) prow[b][c0 + j] = m[j];
+      for (int i = 0; i < 4; ++i) {
+        const int row = 16 * (2 * w + a) + g + 4 * i, col = 16 * j + lr;
+        m[a][j][i] = A[static_cast<int64_t>(max(row, col)) * lda + min(row, col)];
+      }
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    double* rp = Rp[k & 1];
+    double* cp = Cp[k & 1];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) cp[(16 * (2 * w + a) + g + 4 * i) * CS + lr] = m[a][k][i];
+    if (w == k / 2) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rp[(g + 4 * i) * RS + 16 * j + lr] = m[k & 1][j][i];
     }
-    if (q == (k >> 4)) pcol[b][r] = m[k & 15];
     __syncthreads();
-    const double rinv = 1.0 / prow[b][k];
-    const double f = pcol[b][r];
+    double p[4];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const bool diag = q == (k >> 4) && j == (k & 15);
-      const double p = diag ? rinv : prow[b][c0 + j] * rinv;
-      if (r == k) m[j] = p;
-      else m[j] = diag ? -f * rinv : m[j] - f * p;
+    for (int e = 0; e < 4; ++e) p[e] = rp[lr * RS + 16 * k + 4 * g + e];
+    inv16_step<0>(p, lr, g);  inv16_step<1>(p, lr, g);  inv16_step<2>(p, lr, g);  inv16_step<3>(p, lr, g);
+    inv16_step<4>(p, lr, g);  inv16_step<5>(p, lr, g);  inv16_step<6>(p, lr, g);  inv16_step<7>(p, lr, g);
+    inv16_step<8>(p, lr, g);  inv16_step<9>(p, lr, g);  inv16_step<10>(p, lr, g); inv16_step<11>(p, lr, g);
+    inv16_step<12>(p, lr, g); inv16_step<13>(p, lr, g); inv16_step<14>(p, lr, g); inv16_step<15>(p, lr, g);
+    // the operand order of k-step s: P[lr][4 s + g], from lane (lr, group s), element g
+    double pf[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      double v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = __shfl(p[e], s * 16 + lr, 64);
+      pf[s] = g < 2 ? (g == 0 ? v[0] : v[1]) : (g == 2 ? v[2] : v[3]);
+    }
+    double ng[2][4];                                    // -G_i[lr][4 s + g]
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      f64x4 gt = f64x4{0.0, 0.0, 0.0, 0.0}, gn = gt;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const double c = cp[(16 * (2 * w + a) + lr) * CS + 4 * s + g];
+        gt = __builtin_amdgcn_mfma_f64_16x16x4f64(pf[s], c, gt, 0, 0, 0);
+        gn = __builtin_amdgcn_mfma_f64_16x16x4f64(c, pf[s], gn, 0, 0, 0);
+      }
+      const bool own = 2 * w + a == k;                  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        ng[a][i] = own ? pf[i] : -gt[i];
+        m[a][k][i] = own ? pf[i] : -gn[i];
+      }
+      if (own) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          if (j != k) m[a][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      if (j == k) continue;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const double b = rp[(4 * s + g) * RS + 16 * j + lr];
+#pragma unroll
+        for (int a = 0; a < 2; ++a) m[a][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ng[a][s], b, m[a][j], 0, 0, 0);
+      }
     }
   }
 #pragma unroll
-  for (int j = 0; j < 16; ++j) X[static_cast<int64_t>(r) * ldx + c0 + j] = m[j];
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        X[static_cast<int64_t>(16 * (2 * w + a) + g + 4 * i) * ldx + 16 * j + lr] = m[a][j][i];
 }
 
 // out_l[c] = init[c] + alpha sum_r v_l[r] M_l[r][c] for the batch's NL vectors v_l (sv apart) and matrices M_l
@@ -242,27 +385,6 @@ __global__ __launch_bounds__(256) void k_gemv_rows(const double* __restrict__ v,
   }
 }
 
-// dst[j][i] = src[i][j] for an rows x cols block (32 x 32 tiles through LDS).
-__global__ __launch_bounds__(256) void k_dtranspose(const double* __restrict__ src, int64_t lds, double* __restrict__ dst,
-                                                    int64_t ldd, int rows, int cols, int64_t ss, int64_t sd) {
-  __shared__ double tile[32][33];
-  src += static_cast<int64_t>(blockIdx.z) * ss;
-  dst += static_cast<int64_t>(blockIdx.z) * sd;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  const int r0 = blockIdx.y * 32, c0 = blockIdx.x * 32;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = r0 + ty + 8 * i, c = c0 + tx;
-    if (r < rows && c < cols) tile[ty + 8 * i][tx] = src[static_cast<int64_t>(r) * lds + c];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int c = c0 + ty + 8 * i, r = r0 + tx;
-    if (r < rows && c < cols) dst[static_cast<int64_t>(c) * ldd + r] = tile[tx][ty + 8 * i];
-  }
-}
-
 // dst[i][j] = src[i][j] + (i == j ? shift : 0) for i, j < n_src, and the identity on the padding up to n.
 struct Shifts {
   double v[8];
@@ -281,17 +403,6 @@ __global__ __launch_bounds__(256) void k_dshift(const double* __restrict__ src, 
   dst[static_cast<int64_t>(i) * ldd + j] = v;
 }
 
-// dst = src for an rows x cols block; also the bias rows' initial mean_y (rows = 1).
-__global__ __launch_bounds__(256) void k_dcopy(const double* __restrict__ src, int64_t lds, double* __restrict__ dst,
-                                               int64_t ldd, int rows, int cols, int64_t ss, int64_t sd) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  src += static_cast<int64_t>(blockIdx.y) * ss;
-  dst += static_cast<int64_t>(blockIdx.y) * sd;
-  if (idx >= static_cast<int64_t>(rows) * cols) return;
-  const int64_t i = idx / cols, j = idx % cols;
-  dst[i * ldd + j] = src[i * lds + j];
-}
-
 // Launches on one stream for a batch of `nb` matrices laid out at fixed element strides (the lambdas of one
 // solve): every matrix argument is the batch's first matrix and its stride.
 struct Solver {
@@ -304,68 +415,65 @@ struct Solver {
     if (rc == RF_OK) rc = check_launch(fn);
     return rc == RF_OK;
   }
-  void gemm(const double* A, int64_t lda, int64_t sa, const double* B, int64_t ldb, int64_t sb, double* C, int64_t ldc,
-            int64_t sc, int M, int N, int K, double alpha, double beta) {
-    if (rc != RF_OK || M <= 0 || N <= 0) return;
-    const int tiles = ((M + DBM - 1) / DBM) * ((N + DBN - 1) / DBN);
-    const DgemmArgs args{A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, sa, sb, sc};
-    hipLaunchKernelGGL(k_dgemm, dim3(tiles, nb), dim3(256), 0, stream, args);
+  // One k_dgemm per product: 128 x 128 tiles where they give the batch 192 workgroups or more, else 64 x 64, else
+  // 32 x 32. us per product of edge m (M = N = K = m) over three matrices, as 128 x 128 tiles -> as chosen here:
+  // m 128 21 -> 6, 256 47 -> 8 (32 x 32), 512 89 -> 32 (64 x 64), 1024 179 (128 x 128), 2048 990.
+  template <bool AT, bool BT>
+  void gemm(const DgemmArgs& a) {
+    if (rc != RF_OK || a.M <= 0 || a.N <= 0) return;
+    auto tiles = [&](int T) {
+      const int64_t tm = (a.M + T - 1) / T, tn = (a.N + T - 1) / T;
+      return a.lower ? tm * (tm + 1) / 2 : tm * tn;
+    };
+    auto grid = [&](int T) { return dim3(static_cast<unsigned>(tiles(T)), nb); };
+    if (tiles(128) * nb >= 192)
+      hipLaunchKernelGGL((k_dgemm<128, 16, AT, BT>), grid(128), dim3(256), 0, stream, a);
+    else if (tiles(64) * nb >= 192)
+      hipLaunchKernelGGL((k_dgemm<64, 32, AT, BT>), grid(64), dim3(256), 0, stream, a);
+    else
+      hipLaunchKernelGGL((k_dgemm<32, 64, AT, BT>), grid(32), dim3(256), 0, stream, a);
     ok();
   }
-  void transpose(const double* src, int64_t lds, int64_t ss, double* dst, int64_t ldd, int64_t sd, int rows, int cols) {
-    if (rc != RF_OK) return;
-    hipLaunchKernelGGL(k_dtranspose, dim3((cols + 31) / 32, (rows + 31) / 32, nb), dim3(256), 0, stream, src, lds, dst,
-                       ldd, rows, cols, ss, sd);
-    ok();
-  }
-  void copy(const double* src, int64_t lds, int64_t ss, double* dst, int64_t ldd, int64_t sd, int rows, int cols) {
-    if (rc != RF_OK) return;
-    const int64_t n = static_cast<int64_t>(rows) * cols;
-    hipLaunchKernelGGL(k_dcopy, dim3(static_cast<unsigned>((n + 255) / 256), nb), dim3(256), 0, stream, src, lds, dst,
-                       ldd, rows, cols, ss, sd);
-    ok();
-  }
-  // X = A^-1 for each matrix of the batch (n x n SPD, n a multiple of 64; matrices sa / sx apart); work: each
-  // matrix's own work_doubles(n) doubles, sw apart.
+  // X = A^-1 for each matrix of the batch (n x n SPD, n a multiple of 128, its lower triangle read; matrices sa / sx
+  // apart); work: each matrix's own work_doubles(n) doubles, sw apart.
   void inverse(const double* A, int64_t lda, int64_t sa, double* X, int64_t ldx, int64_t sx, int n, double* work,
                int64_t sw) {
     if (rc != RF_OK) return;
-    if (n == 64) {
-      hipLaunchKernelGGL(k_spd_inv64, dim3(nb), dim3(256), 0, stream, A, lda, X, ldx, sa, sx);
+    if (n == LEAF) {
+      hipLaunchKernelGGL(k_spd_inv128, dim3(nb), dim3(256), 0, stream, A, lda, X, ldx, sa, sx);
       ok();
       return;
     }
-    const int h = 64 * ((n + 127) / 128), h2 = n - h;
-    const double* A12 = A + h;
+    const int h = LEAF * ((n + 2 * LEAF - 1) / (2 * LEAF)), h2 = n - h;
     const double* A21 = A + static_cast<int64_t>(h) * lda;
     const double* A22 = A21 + h;
     double* X12 = X + h;
     double* X21 = X + static_cast<int64_t>(h) * ldx;
     double* X22 = X21 + h;
     double* T = work;                                   // [h2, h]
-    double* S = work + static_cast<int64_t>(h2) * h;    // [h2, h2], later U [h, h2]
-    double* deeper = S + static_cast<int64_t>(std::max(h2, h)) * std::max(h2, h);
-    inverse(A, lda, sa, X, ldx, sx, h, work, sw);                              // X11 (T and S are not live yet)
-    gemm(A21, lda, sa, X, ldx, sx, T, h, sw, h2, h, h, 1.0, 0.0);              // T = A21 X11
-    copy(A22, lda, sa, S, h2, sw, h2, h2);
-    gemm(T, h, sw, A12, lda, sa, S, h2, sw, h2, h2, h, -1.0, 1.0);             // S = A22 - T A12
-    inverse(S, h2, sw, X22, ldx, sx, h2, deeper, sw);                          // X22 = S^-1
-    gemm(X22, ldx, sx, T, h, sw, X21, ldx, sx, h2, h, h2, -1.0, 0.0);          // X21 = -X22 T
-    gemm(X, ldx, sx, A12, lda, sa, S, h2, sw, h, h2, h, 1.0, 0.0);             // U = X11 A12 (into S's space)
-    gemm(S, h2, sw, X21, ldx, sx, X, ldx, sx, h, h, h2, -1.0, 1.0);            // X11 -= U X21
-    transpose(X21, ldx, sx, X12, ldx, sx, h2, h);                              // X12 = X21^T
+    double* S = work + static_cast<int64_t>(h2) * h;    // [h2, h2], its lower tiles
+    double* deeper = S + static_cast<int64_t>(h2) * h2;
+    inverse(A, lda, sa, X, ldx, sx, h, work, sw);       // X11 (T and S are not live yet)
+    // T = A21 X11
+    gemm<false, false>({A21, lda, X, ldx, T, h, h2, h, h, 1.0, 0.0, sa, sx, sw, T, h, sw, nullptr, 0, 0, 0});
+    // S = A22 - T A21^T
+    gemm<false, true>({T, h, A21, lda, S, h2, h2, h2, h, -1.0, 1.0, sw, sa, sw, A22, lda, sa, nullptr, 0, 0, 1});
+    inverse(S, h2, sw, X22, ldx, sx, h2, deeper, sw);   // X22 = S^-1
+    // X21 = -X22 T, and X12 = X21^T
+    gemm<false, false>({X22, ldx, T, h, X21, ldx, h2, h, h2, -1.0, 0.0, sx, sw, sx, X21, ldx, sx, X12, ldx, sx, 0});
+    // X11 -= T^T X21, symmetric
+    gemm<true, false>({T, h, X21, ldx, X, ldx, h, h, h2, -1.0, 1.0, sw, sx, sx, X, ldx, sx, X, ldx, sx, 1});
   }
 };
 
-// doubles of work the recursion needs for n (T and S / U at this level, then the deeper levels)
+// doubles of work the recursion needs for n (T and S at this level, then the deeper levels)
 int64_t work_doubles(int n) {
-  if (n <= 64) return 0;
-  const int h = 64 * ((n + 127) / 128), h2 = n - h;
-  const int64_t mx = std::max(h2, h);
-  return static_cast<int64_t>(h2) * h + mx * mx + std::max(work_doubles(h), work_doubles(h2));
+  if (n <= LEAF) return 0;
+  const int64_t h = LEAF * ((n + 2 * LEAF - 1) / (2 * LEAF)), h2 = n - h;
+  return std::max(work_doubles(static_cast<int>(h)), h2 * h + h2 * h2 + work_doubles(static_cast<int>(h2)));
 }
 
-int64_t padded(int64_t d) { return (d + 63) / 64 * 64; }
+int64_t padded(int64_t d) { return (d + LEAF - 1) / LEAF * LEAF; }
 
 constexpr int MAX_LAMBDAS = 8;           // lambdas solved together (one batch of inverses)
 
@@ -400,19 +508,19 @@ extern "C" int rf_ridge_solve_workspace_bytes(int64_t d, int nlam, size_t* bytes
   return RF_OK;
 }
 
-extern "C" int rf_ridge_solve(const double* cxx, int64_t ldc, int64_t d, const double* cxy, int64_t ldb, int64_t R,
-                              const double* mean_x, const double* mean_y, const double* lams, int nlam, double scale,
-                              double* w, int64_t ldw, int64_t w_stride, double* bias, int64_t bias_stride,
-                              void* workspace, size_t ws_bytes, hipStream_t stream) {
-  const char* fn = "rf_ridge_solve";
-  if (!cxx || !cxy || !lams || !w || !workspace) return fail(RF_EINVAL_ARG, "%s: null pointer", fn);
+// Shared by the two entry points: fp64 weights into w, or (wt) fp32 ones in F.linear layout per target.
+static int ridge_solve(const char* fn, const double* cxx, int64_t ldc, int64_t d, const double* cxy, int64_t ldb,
+                       int64_t R, const double* mean_x, const double* mean_y, const double* lams, int nlam, double scale,
+                       double* w, int64_t ldw, int64_t w_stride, float* const* wt, int64_t width, double* bias,
+                       int64_t bias_stride, void* workspace, size_t ws_bytes, hipStream_t stream) {
+  if (!cxx || !cxy || !lams || (!w && !wt) || !workspace) return fail(RF_EINVAL_ARG, "%s: null pointer", fn);
   if (bias && (!mean_x || !mean_y)) return fail(RF_EINVAL_ARG, "%s: the bias needs mean_x and mean_y", fn);
   if (d <= 0 || d > 65536 || R <= 0 || R > (1ll << 30) || R % 2 || d % 2 || ldc < d || ldb < R || ldb % 2 ||
       ldw < R || ldw % 2 || nlam <= 0 || (nlam > 1 && w_stride < d * ldw) || (bias && nlam > 1 && bias_stride < R))
     return fail(RF_EINVAL_SHAPE, "%s: d %lld, R %lld (even), ldc %lld, ldb %lld, ldw %lld (even, >= R), nlam %d, "
                 "w_stride %lld, bias_stride %lld", fn, (long long)d, (long long)R, (long long)ldc, (long long)ldb,
                 (long long)ldw, nlam, (long long)w_stride, (long long)bias_stride);
-  if (!aligned16(cxy) || !aligned16(w) || !aligned16(workspace) || (mean_x && !aligned16(mean_x)) ||
+  if (!aligned16(cxy) || (w && !aligned16(w)) || !aligned16(workspace) || (mean_x && !aligned16(mean_x)) ||
       (bias && (!aligned16(bias) || !aligned16(mean_y) || (nlam > 1 && bias_stride % 2))))
     return fail(RF_EINVAL_SHAPE, "%s: cxy, w, mean_x, mean_y, bias and the workspace must be 16-byte aligned "
                 "(bias_stride even)", fn);
@@ -436,9 +544,25 @@ extern "C" int rf_ridge_solve(const double* cxx, int64_t ldc, int64_t d, const d
                        static_cast<int>(d), A, static_cast<int64_t>(n), n, nn, sh);
     if (!s.ok()) return s.rc;
     s.inverse(A, n, nn, X, n, nn, n, work, nw);
-    double* wl = w + l0 * w_stride;
-    s.gemm(X, n, nn, cxy, ldb, 0, wl, ldw, w_stride, static_cast<int>(d), static_cast<int>(R), static_cast<int>(d),
-           1.0, 0.0);
+    const int di = static_cast<int>(d), ri = static_cast<int>(R);
+    if (w) {
+      double* wl = w + l0 * w_stride;
+      s.gemm<false, false>({X, n, cxy, ldb, wl, ldw, di, ri, di, 1.0, 0.0, nn, 0, w_stride, wl, ldw, w_stride, nullptr, 0,
+                            0, 0});
+    } else {
+      for (int64_t j = 0; j < R / width && s.rc == RF_OK; j += WT_TARGETS) {
+        const int nt = static_cast<int>(std::min<int64_t>(WT_TARGETS, R / width - j));
+        WtOut o{};
+        o.width = static_cast<int>(width);
+        for (int i = 0; i < nt; ++i) o.p[i] = wt[j + i] + static_cast<int64_t>(l0) * width * d;
+        const int m = static_cast<int>(nt * width);
+        const DgemmArgs g{cxy + j * width, ldb, X, n, nullptr, 0, m, di, di, 1.0, 0.0, 0, nn, 0, nullptr, 0, 0, nullptr,
+                          0, 0, 0};
+        hipLaunchKernelGGL(k_solve_wt, dim3(static_cast<unsigned>(((m + 127) / 128) * ((di + 127) / 128)), nb), dim3(256),
+                           0, stream, g, o);
+        s.ok();
+      }
+    }
     if (bias && s.rc == RF_OK) {                       // mean_y - mean_x W = mean_y - (mean_x X) Cxy
       double* u = work + nb * nw;
       hipLaunchKernelGGL(k_gemv_rows<1>, dim3(static_cast<unsigned>((d + 127) / 128), nb), dim3(256), 0, stream,
@@ -452,4 +576,28 @@ extern "C" int rf_ridge_solve(const double* cxx, int64_t ldc, int64_t d, const d
     if (s.rc != RF_OK) return s.rc;
   }
   return RF_OK;
+}
+
+extern "C" int rf_ridge_solve(const double* cxx, int64_t ldc, int64_t d, const double* cxy, int64_t ldb, int64_t R,
+                              const double* mean_x, const double* mean_y, const double* lams, int nlam, double scale,
+                              double* w, int64_t ldw, int64_t w_stride, double* bias, int64_t bias_stride,
+                              void* workspace, size_t ws_bytes, hipStream_t stream) {
+  if (!w) return fail(RF_EINVAL_ARG, "rf_ridge_solve: null pointer");
+  return ridge_solve("rf_ridge_solve", cxx, ldc, d, cxy, ldb, R, mean_x, mean_y, lams, nlam, scale, w, ldw, w_stride,
+                     nullptr, R, bias, bias_stride, workspace, ws_bytes, stream);
+}
+
+extern "C" int rf_ridge_solve_wt(const double* cxx, int64_t ldc, int64_t d, const double* cxy, int64_t ldb, int targets,
+                                 int64_t width, const double* mean_x, const double* mean_y, const double* lams, int nlam,
+                                 double scale, float* const* wt, double* bias, int64_t bias_stride, void* workspace,
+                                 size_t ws_bytes, hipStream_t stream) {
+  const char* fn = "rf_ridge_solve_wt";
+  if (!wt) return fail(RF_EINVAL_ARG, "%s: null pointer", fn);
+  if (targets <= 0 || width <= 0 || width % 2 || width * targets > (1ll << 30) || width > (1ll << 24))
+    return fail(RF_EINVAL_SHAPE, "%s: %d targets of width %lld (even)", fn, targets, (long long)width);
+  for (int j = 0; j < targets; ++j)
+    if (!wt[j]) return fail(RF_EINVAL_ARG, "%s: null pointer for target %d", fn, j);
+  const int64_t R = width * targets;
+  return ridge_solve(fn, cxx, ldc, d, cxy, ldb, R, mean_x, mean_y, lams, nlam, scale, nullptr, R, d * R, wt, width, bias,
+                     bias_stride, workspace, ws_bytes, stream);
 }

@@ -61,6 +61,7 @@ SIGNATURES = {
     "rf_gram_state": [_P, _I64, _I64, _I64, _P, _I64, _I64, _P, _I32, _P, _P, _P, _P, _F64, _P, _I64, _P],
     "rf_col_moments": [_P, _I64, _I64, _I64, _P, _P, _P],
     "rf_centre_select": [_P, _P, _F64, _P, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P],
+    "rf_ridge_solve_wt": [_P, _I64, _I64, _P, _I64, _I32, _I64, _P, _P, _P, _I32, _F64, _P, _P, _I64, _P, _SZ, _P],
     "rf_ridge_solve": [_P, _I64, _I64, _P, _I64, _I64, _P, _P, _P, _I32, _F64, _P, _I64, _I64, _P, _I64, _P, _SZ, _P],
     "rf_ridge_solve_workspace_bytes": [_I64, _I32, _PSZ],
     "rf_row_gather": [_P, _I64, _I64, _I64, _P, _I64, _P, _I64, _P, _P],

@@ -506,6 +506,24 @@ class RidgeFit:
                   _ptr(bias), R, _ptr(ws), ws.numel(), _stream(cxy))
         return w, bias
 
+    def _solve_wt(self, cxy, width, lams, mean_y):
+        """solve() of targets of `width` columns each, the weights rounded to fp32 in F.linear layout: ([per target:
+        [nlam, width, d] fp32], bias [nlam, R] fp64)."""
+        lams = [float(v) for v in lams]
+        d, R = cxy.shape
+        if d % 2 or width % 2:
+            raise ValueError(f"ridge solve: d {d} and R {R} must be even")
+        wts = [torch.empty(len(lams), width, d, dtype=torch.float32, device=self.device) for _ in range(R // width)]
+        bias = torch.empty(len(lams), R, dtype=torch.float64, device=self.device)
+        ws = torch.empty(ridge_solve_workspace_bytes(d, len(lams)), dtype=torch.uint8, device=self.device)
+        arr = (ctypes.c_double * len(lams))(*lams)
+        ptrs = (ctypes.c_void_p * len(wts))(*[_ptr(t) for t in wts])
+        mx, my = self.mean_x.contiguous(), mean_y.to(self.device, torch.float64).contiguous()
+        _lib.call("rf_ridge_solve_wt", _ptr(self.cxx), self.cxx.stride(0), d, _ptr(cxy), cxy.stride(0), len(wts), width,
+                  _ptr(mx), _ptr(my), arr, len(lams), float(self.scale), ptrs, _ptr(bias), R, _ptr(ws), ws.numel(),
+                  _stream(cxy))
+        return wts, bias
+
     def layer(self, i, lams):
         """{lam: (weight [d_out, d_in] fp32, bias [d_out] fp32)} for layer i (F.linear layout)."""
         return self.layers([i], lams)[i]
@@ -520,9 +538,16 @@ class RidgeFit:
             cols.append(cols[-1] + k)
         cxy = torch.empty(self.cxx.shape[0], cols[-1], dtype=torch.float64, device=self.device)
         means = [self.cross(i, out=cxy[:, cols[j]:cols[j + 1]])[1] for j, i in enumerate(ids)]
+        out = {i: {} for i in ids}
+        if len(set(widths)) == 1 and widths[0] % 2 == 0:    # one width: fp32 weights in F.linear layout straight from the solve
+            wts, b_all = self._solve_wt(cxy, widths[0], lams, torch.cat(means))
+            for j, i in enumerate(ids):
+                bt = b_all[:, cols[j]:cols[j + 1]].float()
+                for li, lam in enumerate(lams):
+                    out[i][lam] = (wts[j][li], bt[li])
+            return out
         w_all, b_all = self.solve(cxy, lams, torch.cat(means))
         del cxy
-        out = {i: {} for i in ids}
         for j, i in enumerate(ids):             # one transposing fp32 copy per target for all lambdas
             c0, c1 = cols[j], cols[j + 1]
             wt = w_all[:, :, c0:c1].transpose(1, 2).to(torch.float32, memory_format=torch.contiguous_format)
