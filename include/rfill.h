@@ -143,6 +143,24 @@ int rf_norm_linear_batch(int nl, const uint16_t* const* x, int64_t ldx, const fl
                          int64_t H, float eps, const uint16_t* const* w, const int64_t* n, uint16_t* const* out,
                          int64_t ldo, hipStream_t stream);
 
+/* The batched launches with a workspace, which may be NULL (as the forms without): rows that would take a last round
+ * of tiles by themselves then run as products of few rows with K split over the CUs, whose results differ from the
+ * tiles' by the order of the fp32 sums. rf_batch_workspace_bytes(nl, P, N, K): for the map (N = h_out, K = h_in) and
+ * the K / V write (N = 2 hkv d, K = H); 0 when nothing runs that way. A smaller workspace counts as none. */
+int rf_batch_workspace_bytes(int nl, int64_t M, int64_t N, int64_t K, size_t* bytes);
+int rf_norm_linear_batch_workspace_bytes(int nl, const int64_t* rows, const int64_t* n, int64_t H, size_t* bytes);
+int rf_map_apply_batch_ws(int nl, const uint16_t* b, int64_t ldb, const uint16_t* const* w, const uint16_t* const* c,
+                          uint16_t* const* x, int64_t ldx, float* const* ssq, int64_t P, int64_t h_in, int64_t h_out,
+                          void* workspace, size_t ws_bytes, hipStream_t stream);
+int rf_norm_kv_write_batch_ws(int nl, const uint16_t* const* x, int64_t ldx, const float* const* ssq, int64_t P,
+                              int64_t H, float eps, const uint16_t* const* wkv, int hkv, int d,
+                              const uint16_t* const* knorm, int knorm_kind, const uint16_t* cs, int rot,
+                              uint16_t* const* kbuf, uint16_t* const* vbuf, int64_t head_stride, int64_t row_stride,
+                              int64_t slot_begin, int64_t cap, void* workspace, size_t ws_bytes, hipStream_t stream);
+int rf_norm_linear_batch_ws(int nl, const uint16_t* const* x, int64_t ldx, const float* const* ssq,
+                            const int64_t* rows, int64_t H, float eps, const uint16_t* const* w, const int64_t* n,
+                            uint16_t* const* out, int64_t ldo, void* workspace, size_t ws_bytes, hipStream_t stream);
+
 /* RoPE on given pre-RoPE K and the K / V cache write of m rows.
  * Replaces Model.fill_kv (code/kva/model.py:161-165): ops.apply_rope (ops.py:66-77) + _append_kv.
  * k / v: [m, hkv, d] with token strides ld_k / ld_v (a head's d values contiguous, heads d apart);

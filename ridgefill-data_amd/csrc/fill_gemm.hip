@@ -909,10 +909,10 @@ constexpr int RED_ROWS = 8;
 // this 256-column group, formed in the order every producer uses (one wave per row).
 // res (optional): the residual stream, X = bf16(res + bf16(sum + bias)) (rf_residual_add's rounding after
 // the product's), the statistics then being X's.
-__global__ __launch_bounds__(256) void k_map_apply_reduce(const float* __restrict__ part, int splits,
-                                                          const uint16_t* __restrict__ bias, uint16_t* __restrict__ X,
-                                                          int64_t ldx, float* __restrict__ ssq, int M, int N,
-                                                          const uint16_t* __restrict__ res = nullptr, int64_t ldr = 0) {
+__device__ __forceinline__ void map_apply_reduce(const float* __restrict__ part, int splits,
+                                                 const uint16_t* __restrict__ bias, uint16_t* __restrict__ X, int64_t ldx,
+                                                 float* __restrict__ ssq, int M, int N, const uint16_t* __restrict__ res,
+                                                 int64_t ldr) {
   __shared__ uint4 img[RED_ROWS * 32];
   const int t = threadIdx.x, r = t >> 5, ch = t & 31, tn = blockIdx.y, n0 = tn * BN;
   const int m = blockIdx.x * RED_ROWS + r;
@@ -946,10 +946,17 @@ __global__ __launch_bounds__(256) void k_map_apply_reduce(const float* __restric
   }
 }
 
+__global__ __launch_bounds__(256) void k_map_apply_reduce(const float* __restrict__ part, int splits,
+                                                          const uint16_t* __restrict__ bias, uint16_t* __restrict__ X,
+                                                          int64_t ldx, float* __restrict__ ssq, int M, int N,
+                                                          const uint16_t* __restrict__ res = nullptr, int64_t ldr = 0) {
+  map_apply_reduce(part, splits, bias, X, ldx, ssq, M, N, res, ldr);
+}
+
 // The unsplit norm + linear epilogue on split sums: out = bf16(sum * r_row).
-__global__ __launch_bounds__(256) void k_norm_linear_reduce(const float* __restrict__ part, int splits,
-                                                            const float* __restrict__ ssq, int K, float eps,
-                                                            uint16_t* __restrict__ out, int64_t ldo, int M, int N) {
+__device__ __forceinline__ void norm_linear_reduce(const float* __restrict__ part, int splits,
+                                                   const float* __restrict__ ssq, int K, float eps,
+                                                   uint16_t* __restrict__ out, int64_t ldo, int M, int N) {
   const int t = threadIdx.x, r = t >> 5, ch = t & 31, n0 = blockIdx.y * BN;
   const int m = blockIdx.x * RED_ROWS + r;
   if (m >= M) return;
@@ -961,6 +968,12 @@ __global__ __launch_bounds__(256) void k_norm_linear_reduce(const float* __restr
   *reinterpret_cast<uint4*>(out + static_cast<int64_t>(m) * ldo + n0 + ch * 8) =
       make_uint4(bf16_pair(v[0] * rs, v[1] * rs), bf16_pair(v[2] * rs, v[3] * rs), bf16_pair(v[4] * rs, v[5] * rs),
                  bf16_pair(v[6] * rs, v[7] * rs));
+}
+
+__global__ __launch_bounds__(256) void k_norm_linear_reduce(const float* __restrict__ part, int splits,
+                                                            const float* __restrict__ ssq, int K, float eps,
+                                                            uint16_t* __restrict__ out, int64_t ldo, int M, int N) {
+  norm_linear_reduce(part, splits, ssq, K, eps, out, ldo, M, N);
 }
 
 // SwiGLU on the split sums of a [gate; up] product (gate columns [0, I), up columns [I, 2 I) of the partial
@@ -1962,6 +1975,55 @@ __global__ __launch_bounds__(NTHR) void k_norm_linear_p(LinLayers ll, int nl, in
   stream_tiles(sh.cnt, K / BK, ldx, K, ops, begin, [](int, uint4*) {}, end, lds);
 }
 
+// ---- the rows a batched launch leaves over (batch_plan): every entry's last rows as products of few rows.
+//
+// Entry l: m[l] rows of x[l] against the n[l] rows of w[l]; its blocks are [start[l], start[l + 1]), its split
+// planes start at part + off[l].
+struct RowJobs {
+  const uint16_t* x[MAXL];
+  const uint16_t* w[MAXL];
+  int m[MAXL], n[MAXL], rblocks[MAXL];
+  int start[MAXL + 1];
+  int64_t off[MAXL];
+};
+template <int RT>
+__global__ __launch_bounds__(NTHR) void k_rows_batch(RowJobs j, int nl, int64_t ldx, int64_t ldw, int K, int kper,
+                                                     float* __restrict__ part) {
+#ifdef __HIP_DEVICE_COMPILE__   // (as k_gram_strips)
+  __shared__ uint4 lds[RowsCfg<RT>::S * RowsCfg<RT>::STAGE_U4];
+  const int b = blockIdx.x;
+  int l = 0;
+  while (l + 1 < nl && b >= j.start[l + 1]) ++l;
+  rows_partial<RT>(j.x[l], ldx, j.w[l], ldw, j.m[l], j.n[l], K, kper, j.rblocks[l], part + j.off[l], lds, b - j.start[l],
+                   j.start[l + 1] - j.start[l], j.n[l]);
+#endif
+}
+
+// The epilogues over those planes, entry blockIdx.z; mf: the entry's rows before them.
+__global__ __launch_bounds__(256) void k_map_reduce_batch(const float* __restrict__ part, int splits, MapLayers ml,
+                                                          int64_t ldx, int64_t mf, int M, int N) {
+  const int l = blockIdx.z;
+  map_apply_reduce(part + static_cast<int64_t>(l) * splits * M * N, splits, ml.c[l], ml.x[l] + mf * ldx, ldx,
+                   ml.ssq[l] + mf * (N / SSQ_COLS), M, N, nullptr, 0);
+}
+__global__ __launch_bounds__(256) void k_norm_kv_reduce_batch(const float* __restrict__ part, int splits, KvLayers kl,
+                                                              KvArgs a, int64_t mf, int M, int N) {
+  const int l = blockIdx.z;
+  a.ssq = kl.ssq[l] + mf * a.nparts;
+  a.knorm = kl.knorm[l];
+  a.kbuf = kl.kbuf[l];
+  a.vbuf = kl.vbuf[l];
+  a.slot0 += mf;
+  a.cs += mf * a.rot;
+  norm_kv_reduce(part + static_cast<int64_t>(l) * splits * M * N, splits, M, N, blockIdx.y, a);
+}
+__global__ __launch_bounds__(256) void k_norm_linear_reduce_batch(const float* __restrict__ part, int splits, RowJobs j,
+                                                                  LinLayers ll, int K, float eps, int64_t ldo) {
+  const int l = blockIdx.z;
+  if (static_cast<int>(blockIdx.y) * BN >= j.n[l]) return;
+  norm_linear_reduce(part + j.off[l], splits, ll.ssq[l], K, eps, ll.out[l], ldo, j.m[l], j.n[l]);
+}
+
 int grid_of(int64_t M, int64_t N) { return static_cast<int>(((M + BM - 1) / BM) * (N / BN)); }
 
 // The persistent K / V kernel takes H a multiple of 1024 up to 4096 (its row statistics: 4 .. 16 partials,
@@ -2078,6 +2140,108 @@ void launch_partials(const uint16_t* X, int64_t ldx, const uint16_t* W, int64_t 
   hipLaunchKernelGGL(k_gemm_partial, dim3(grid_of(rows, N) * p.splits), dim3(NTHR), 0, stream, X + p.m_fused * ldx,
                      ldx, W, ldw, static_cast<int>(rows), static_cast<int>(N), static_cast<int>(K), kper,
                      static_cast<float*>(ws));
+}
+
+// How a batched launch of nl products, each M x N x K, runs: rows [0, m_fused) of every entry as 256 x 256 tiles,
+// the rest (at most BATCH_ROWS rows, rblocks row blocks of at most 160 each) as products of few rows with K split
+// `splits` ways. A round of tiles on the 256 CUs costs the same whether all of them have one or only a few do, and a
+// tile row is a whole one however few of its rows exist; the few-rows products cost what their rows do. The times
+// compared, in us (measured at K 2048 and 4096): a round 1.45 per 64-deep step + 8; a round of few-rows blocks
+// 0.55 + 0.1 per 32 rows a step + 4, 6 for the second launch, and the split planes written and read at 4 TB/s.
+// 6160 rows of four 8B layers: the 64 map tiles (32 K / V tiles) that held the last 16 rows took a seventh (fourth)
+// round, 743 (507) us in all; now 685 (401) for whole rounds and 32 (22) for the rows, product and epilogue.
+struct BatchPlan {
+  int64_t m_fused = 0;
+  int splits = 0, rt = 0, rblocks = 0;
+  bool rows() const { return rt > 0; }
+};
+constexpr int64_t BATCH_ROWS = 1024;
+
+struct RowShape {
+  int splits, rt, rblocks;
+  double us;
+};
+// cblocks: the column blocks of every entry together, for m rows each.
+RowShape batch_rows_shape(int64_t cblocks, int64_t m, int64_t K) {
+  const int64_t rb = (m + 159) / 160, rt = ((m + rb - 1) / rb + 31) / 32, blocks = rb * cblocks;
+  const int64_t s = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / blocks, K / 512), 16));
+  const double rounds = static_cast<double>((blocks * s + 255) / 256), steps = static_cast<double>(K / BK) / s;
+  const double planes = static_cast<double>(cblocks) * RN * m * 4 * 2 * s;
+  return RowShape{static_cast<int>(s), static_cast<int>(rt), static_cast<int>(rb),
+                  rounds * (steps * (0.55 + 0.1 * rt) + 4) + 6 + planes / 4e6};
+}
+
+BatchPlan batch_plan(int64_t cblocks, int64_t M, int64_t K) {
+  BatchPlan best;
+  best.m_fused = M;
+  if (K < 1024 || M <= 0) return best;
+  const double round = 1.45 * static_cast<double>(K / BK) + 8;
+  auto rounds = [&](int64_t trows) { return static_cast<double>((trows * cblocks + 255) / 256); };
+  const int64_t trows = (M + BM - 1) / BM;
+  double cost = rounds(trows) * round - 5;           // 5 us: what a plan has to gain at least
+  for (int64_t fr = trows - 1; fr >= 0 && M - fr * BM <= BATCH_ROWS; --fr) {
+    const RowShape r = batch_rows_shape(cblocks, M - fr * BM, K);
+    const double c = rounds(fr) * round + r.us;
+    if (c < cost) {
+      cost = c;
+      best = BatchPlan{fr * BM, r.splits, r.rt, r.rblocks};
+    }
+  }
+  return best;
+}
+
+size_t batch_bytes(int64_t nl, int64_t M, int64_t N, int64_t K) {
+  const BatchPlan p = batch_plan(nl * (N / BN), M, K);
+  return p.rows() ? static_cast<size_t>(nl) * p.splits * (M - p.m_fused) * N * 4 : 0;
+}
+
+// The few-rows products of `nl` entries filled into j (x, w, m, n): block and plane offsets, then one launch.
+void launch_rows_batch(RowJobs& j, int nl, const BatchPlan& p, int64_t ldx, int64_t ldw, int64_t K, void* ws,
+                       hipStream_t stream) {
+  j.start[0] = 0;
+  int64_t off = 0;
+  for (int l = 0; l < nl; ++l) {
+    j.rblocks[l] = (j.m[l] + 159) / 160;
+    j.start[l + 1] = j.start[l] + j.n[l] / RN * j.rblocks[l] * p.splits;
+    j.off[l] = off;
+    off += static_cast<int64_t>(p.splits) * j.m[l] * j.n[l];
+  }
+  const dim3 grid(static_cast<unsigned>(j.start[nl])), block(NTHR);
+  const int k = static_cast<int>(K), kper = static_cast<int>((K / p.splits + BK - 1) / BK * BK);
+  float* part = static_cast<float*>(ws);
+  switch (p.rt) {
+    case 1: hipLaunchKernelGGL(k_rows_batch<1>, grid, block, 0, stream, j, nl, ldx, ldw, k, kper, part); break;
+    case 2: hipLaunchKernelGGL(k_rows_batch<2>, grid, block, 0, stream, j, nl, ldx, ldw, k, kper, part); break;
+    case 3: hipLaunchKernelGGL(k_rows_batch<3>, grid, block, 0, stream, j, nl, ldx, ldw, k, kper, part); break;
+    case 4: hipLaunchKernelGGL(k_rows_batch<4>, grid, block, 0, stream, j, nl, ldx, ldw, k, kper, part); break;
+    default: hipLaunchKernelGGL(k_rows_batch<5>, grid, block, 0, stream, j, nl, ldx, ldw, k, kper, part); break;
+  }
+}
+
+// An entry of at most this many rows has no tile rows of its own when a norm + linear batch is planned.
+constexpr int64_t LIN_SMALL = 256;
+
+// The plan of a norm + linear batch: its large entries (all of one row count, else no plan) share m_fused; small
+// entries go with the rest rows entirely.
+BatchPlan lin_plan(int nl, const int64_t* rows, const int64_t* n, int64_t H, int64_t* m_large) {
+  int64_t M = 0, cb = 0;
+  for (int l = 0; l < nl; ++l) {
+    if (rows[l] <= LIN_SMALL) continue;
+    if (M && rows[l] != M) return BatchPlan{rows[l]};
+    M = rows[l];
+    cb += n[l] / BN;
+  }
+  *m_large = M;
+  return M && persistent_lin_ok(H) ? batch_plan(cb, M, H) : BatchPlan{M};
+}
+
+size_t lin_bytes(int nl, const int64_t* rows, const int64_t* n, int64_t H) {
+  int64_t M = 0, b = 0;
+  const BatchPlan p = lin_plan(nl, rows, n, H, &M);
+  if (!p.rows()) return 0;
+  for (int l = 0; l < nl; ++l)
+    if (rows[l] > 0) b += p.splits * (rows[l] <= LIN_SMALL ? rows[l] : rows[l] - p.m_fused) * n[l] * 4;
+  return static_cast<size_t>(b);
 }
 
 dim3 reduce_grid(int64_t M, int64_t N) {
@@ -2700,9 +2864,36 @@ extern "C" int rf_norm_linear(const uint16_t* x, int64_t ldx, const float* ssq, 
   return check_launch("rf_norm_linear");
 }
 
+extern "C" int rf_batch_workspace_bytes(int nl, int64_t M, int64_t N, int64_t K, size_t* bytes) {
+  if (!bytes || nl < 1 || nl > MAXL || M < 0 || M > (1ll << 30) || N <= 0 || N % BN || K <= 0 || K % BK)
+    return fail(RF_EINVAL_ARG, "rf_batch_workspace_bytes: %d layers, M %lld, N %lld (multiple of 256), K %lld (multiple "
+                "of 64)", nl, (long long)M, (long long)N, (long long)K);
+  *bytes = batch_bytes(nl, M, N, K);
+  return RF_OK;
+}
+
+extern "C" int rf_norm_linear_batch_workspace_bytes(int nl, const int64_t* rows, const int64_t* n, int64_t H,
+                                                    size_t* bytes) {
+  const char* fn = "rf_norm_linear_batch_workspace_bytes";
+  if (!bytes || !rows || !n || nl < 1 || nl > MAXL || H <= 0 || H % BK) return fail(RF_EINVAL_ARG, "%s: arguments", fn);
+  for (int l = 0; l < nl; ++l)
+    if (rows[l] < 0 || rows[l] > (1ll << 30) || n[l] <= 0 || n[l] % BN)
+      return fail(RF_EINVAL_SHAPE, "%s: entry %d: rows %lld, N %lld (multiple of 256)", fn, l, (long long)rows[l],
+                  (long long)n[l]);
+  *bytes = lin_bytes(nl, rows, n, H);
+  return RF_OK;
+}
+
 extern "C" int rf_map_apply_batch(int nl, const uint16_t* b, int64_t ldb, const uint16_t* const* w,
                                   const uint16_t* const* c, uint16_t* const* x, int64_t ldx, float* const* ssq, int64_t P,
                                   int64_t h_in, int64_t h_out, hipStream_t stream) {
+  return rf_map_apply_batch_ws(nl, b, ldb, w, c, x, ldx, ssq, P, h_in, h_out, nullptr, 0, stream);
+}
+
+extern "C" int rf_map_apply_batch_ws(int nl, const uint16_t* b, int64_t ldb, const uint16_t* const* w,
+                                     const uint16_t* const* c, uint16_t* const* x, int64_t ldx, float* const* ssq,
+                                     int64_t P, int64_t h_in, int64_t h_out, void* workspace, size_t ws_bytes,
+                                     hipStream_t stream) {
   if (nl < 1 || nl > MAXL) return fail(RF_EINVAL_ARG, "rf_map_apply_batch: %d layers (1 .. %d)", nl, MAXL);
   if (!b || !w || !x || !ssq) return fail(RF_EINVAL_ARG, "rf_map_apply_batch: null pointer");
   if (P < 0 || P > (1ll << 30)) return fail(RF_EINVAL_SHAPE, "rf_map_apply_batch: P = %lld out of range", (long long)P);
@@ -2724,10 +2915,30 @@ extern "C" int rf_map_apply_batch(int nl, const uint16_t* b, int64_t ldb, const 
     ml.ssq[l] = ssq[l];
   }
   if (!aligned16(b)) return fail(RF_EINVAL_SHAPE, "rf_map_apply_batch: b must be 16-byte aligned");
+  if (workspace && !aligned16(workspace)) return fail(RF_EINVAL_SHAPE, "rf_map_apply_batch: workspace alignment");
   if (P == 0) return RF_OK;
-  hipLaunchKernelGGL(k_map_apply_p<false>, dim3(persistent_grid(nl * static_cast<int64_t>(grid_of(P, h_out)))),
-                     dim3(NTHR), 0, stream, b, ldb, ml, nl, ldx, static_cast<int>(P), static_cast<int>(h_out),
-                     static_cast<int>(h_in), static_cast<const uint16_t*>(nullptr), static_cast<int64_t>(0));
+  BatchPlan pl = batch_plan(nl * (h_out / BN), P, h_in);
+  if (pl.rows() && (!workspace || ws_bytes < batch_bytes(nl, P, h_out, h_in))) pl = BatchPlan{P};
+  const int64_t mf = pl.m_fused;
+  if (mf > 0)
+    hipLaunchKernelGGL(k_map_apply_p<false>, dim3(persistent_grid(nl * static_cast<int64_t>(grid_of(mf, h_out)))),
+                       dim3(NTHR), 0, stream, b, ldb, ml, nl, ldx, static_cast<int>(mf), static_cast<int>(h_out),
+                       static_cast<int>(h_in), static_cast<const uint16_t*>(nullptr), static_cast<int64_t>(0));
+  if (pl.rows()) {
+    const int m = static_cast<int>(P - mf), n = static_cast<int>(h_out);
+    RowJobs j{};
+    for (int l = 0; l < nl; ++l) {
+      j.x[l] = b + mf * ldb;
+      j.w[l] = w[l];
+      j.m[l] = m;
+      j.n[l] = n;
+    }
+    launch_rows_batch(j, nl, pl, ldb, h_in, h_in, workspace, stream);
+    dim3 grid = reduce_grid(m, n);
+    grid.z = nl;
+    hipLaunchKernelGGL(k_map_reduce_batch, grid, dim3(256), 0, stream, static_cast<const float*>(workspace), pl.splits, ml,
+                       ldx, mf, m, n);
+  }
   return check_launch("rf_map_apply_batch");
 }
 
@@ -2736,6 +2947,16 @@ extern "C" int rf_norm_kv_write_batch(int nl, const uint16_t* const* x, int64_t 
                                       const uint16_t* const* knorm, int knorm_kind, const uint16_t* cs, int rot,
                                       uint16_t* const* kbuf, uint16_t* const* vbuf, int64_t head_stride,
                                       int64_t row_stride, int64_t slot_begin, int64_t cap, hipStream_t stream) {
+  return rf_norm_kv_write_batch_ws(nl, x, ldx, ssq, P, H, eps, wkv, hkv, d, knorm, knorm_kind, cs, rot, kbuf, vbuf,
+                                   head_stride, row_stride, slot_begin, cap, nullptr, 0, stream);
+}
+
+extern "C" int rf_norm_kv_write_batch_ws(int nl, const uint16_t* const* x, int64_t ldx, const float* const* ssq, int64_t P,
+                                         int64_t H, float eps, const uint16_t* const* wkv, int hkv, int d,
+                                         const uint16_t* const* knorm, int knorm_kind, const uint16_t* cs, int rot,
+                                         uint16_t* const* kbuf, uint16_t* const* vbuf, int64_t head_stride,
+                                         int64_t row_stride, int64_t slot_begin, int64_t cap, void* workspace,
+                                         size_t ws_bytes, hipStream_t stream) {
   if (nl < 1 || nl > MAXL) return fail(RF_EINVAL_ARG, "rf_norm_kv_write_batch: %d layers (1 .. %d)", nl, MAXL);
   if (!x || !ssq || !wkv || !cs || !kbuf || !vbuf) return fail(RF_EINVAL_ARG, "rf_norm_kv_write_batch: null pointer");
   if (P < 0 || P > (1ll << 30))
@@ -2778,8 +2999,27 @@ extern "C" int rf_norm_kv_write_batch(int nl, const uint16_t* const* x, int64_t 
   KvArgs a{nullptr, static_cast<int>(H / SSQ_COLS), static_cast<float>(H), eps, hkv, d, nullptr, knorm_kind, cs, rot,
            nullptr, nullptr, head_stride, row_stride, slot_begin, nullptr};
   a.knorm = knorm ? knorm[0] : nullptr;            // the K epilogue's mode follows the (shared) configuration
+  if (workspace && !aligned16(workspace)) return fail(RF_EINVAL_SHAPE, "rf_norm_kv_write_batch: workspace alignment");
   if (persistent_kv_ok(H, rot, P)) {
-    launch_norm_kv_p(kl, nl, ldx, P, N, H, a, stream);
+    BatchPlan pl = batch_plan(nl * (N / BN), P, H);
+    if (pl.rows() && (!workspace || ws_bytes < batch_bytes(nl, P, N, H))) pl = BatchPlan{P};
+    const int64_t mf = pl.m_fused;
+    if (mf > 0) launch_norm_kv_p(kl, nl, ldx, mf, N, H, a, stream);
+    if (pl.rows()) {
+      const int m = static_cast<int>(P - mf), n = static_cast<int>(N);
+      RowJobs j{};
+      for (int l = 0; l < nl; ++l) {
+        j.x[l] = kl.x[l] + mf * ldx;
+        j.w[l] = kl.wkv[l];
+        j.m[l] = m;
+        j.n[l] = n;
+      }
+      launch_rows_batch(j, nl, pl, ldx, H, H, workspace, stream);
+      dim3 grid = reduce_grid(m, n);
+      grid.z = nl;
+      hipLaunchKernelGGL(k_norm_kv_reduce_batch, grid, dim3(256), 0, stream, static_cast<const float*>(workspace),
+                         pl.splits, kl, a, mf, m, n);
+    }
   } else {                                          // other widths: the per-tile kernel, one launch per layer
     for (int l = 0; l < nl; ++l) {
       KvArgs al = a;
@@ -2797,6 +3037,13 @@ extern "C" int rf_norm_kv_write_batch(int nl, const uint16_t* const* x, int64_t 
 extern "C" int rf_norm_linear_batch(int nl, const uint16_t* const* x, int64_t ldx, const float* const* ssq,
                                     const int64_t* rows, int64_t H, float eps, const uint16_t* const* w,
                                     const int64_t* n, uint16_t* const* out, int64_t ldo, hipStream_t stream) {
+  return rf_norm_linear_batch_ws(nl, x, ldx, ssq, rows, H, eps, w, n, out, ldo, nullptr, 0, stream);
+}
+
+extern "C" int rf_norm_linear_batch_ws(int nl, const uint16_t* const* x, int64_t ldx, const float* const* ssq,
+                                       const int64_t* rows, int64_t H, float eps, const uint16_t* const* w,
+                                       const int64_t* n, uint16_t* const* out, int64_t ldo, void* workspace,
+                                       size_t ws_bytes, hipStream_t stream) {
   const char* fn = "rf_norm_linear_batch";
   if (nl < 1 || nl > MAXL) return fail(RF_EINVAL_ARG, "%s: %d entries (1 .. %d)", fn, nl, MAXL);
   if (!x || !ssq || !w || !out || !rows || !n) return fail(RF_EINVAL_ARG, "%s: null pointer", fn);
@@ -2804,9 +3051,10 @@ extern "C" int rf_norm_linear_batch(int nl, const uint16_t* const* x, int64_t ld
   if (ldx < H || ldx % 8 || ldx > (1 << 21) || ldo % 8)
     return fail(RF_EINVAL_SHAPE, "%s: strides ldx %lld, ldo %lld", fn, (long long)ldx, (long long)ldo);
   if (!(eps >= 0.f)) return fail(RF_EINVAL_ARG, "%s: eps", fn);
-  LinLayers ll{};
+  LinLayers ll{}, rest{};                           // the entries' tiles; the rows left to the few-rows products
+  RowJobs j{};
   int64_t tiles = 0;
-  int live = 0;
+  int live = 0, nj = 0, mmax = 0, nmax = 0;
   for (int l = 0; l < nl; ++l) {
     if (rows[l] < 0 || rows[l] > (1ll << 30) || n[l] <= 0 || n[l] % BN || ldo < n[l])
       return fail(RF_EINVAL_SHAPE, "%s: entry %d: rows %lld, N %lld (multiple of 256, <= ldo %lld)", fn, l,
@@ -2814,20 +3062,50 @@ extern "C" int rf_norm_linear_batch(int nl, const uint16_t* const* x, int64_t ld
     if (!x[l] || !ssq[l] || !w[l] || !out[l]) return fail(RF_EINVAL_ARG, "%s: null pointer in entry %d", fn, l);
     if (!aligned16(x[l]) || !aligned16(w[l]) || !aligned16(out[l]))
       return fail(RF_EINVAL_SHAPE, "%s: entry %d pointers must be 16-byte aligned", fn, l);
+  }
+  if (workspace && !aligned16(workspace)) return fail(RF_EINVAL_SHAPE, "%s: workspace alignment", fn);
+  int64_t large = 0;
+  BatchPlan pl = lin_plan(nl, rows, n, H, &large);
+  if (pl.rows() && (!workspace || ws_bytes < lin_bytes(nl, rows, n, H))) pl = BatchPlan{large};
+  for (int l = 0; l < nl; ++l) {
     if (rows[l] == 0) continue;                     // nothing to compute: left out of the launch
+    const int64_t mf = !pl.rows() ? rows[l] : rows[l] <= LIN_SMALL ? 0 : pl.m_fused;
+    if (mf < rows[l]) {
+      j.x[nj] = x[l] + mf * ldx;
+      j.w[nj] = w[l];
+      j.m[nj] = static_cast<int>(rows[l] - mf);
+      j.n[nj] = static_cast<int>(n[l]);
+      rest.ssq[nj] = ssq[l] + mf * (H / SSQ_COLS);
+      rest.out[nj] = out[l] + mf * ldo;
+      mmax = std::max(mmax, j.m[nj]);
+      nmax = std::max(nmax, j.n[nj]);
+      ++nj;
+    }
+    if (mf == 0) continue;
     ll.x[live] = x[l];
     ll.ssq[live] = ssq[l];
     ll.w[live] = w[l];
     ll.out[live] = out[l];
-    ll.m[live] = static_cast<int>(rows[l]);
+    ll.m[live] = static_cast<int>(mf);
     ll.n[live] = static_cast<int>(n[l]);
     ll.start[live] = static_cast<int>(tiles);
-    tiles += grid_of(rows[l], n[l]);
+    tiles += grid_of(mf, n[l]);
     if (tiles > (1ll << 30)) return fail(RF_EINVAL_SHAPE, "%s: too many tiles", fn);
     ++live;
   }
   ll.start[live] = static_cast<int>(tiles);
-  if (live == 0) return RF_OK;
+  if (nj > 0) {
+    for (int l = 0; l < nj; ++l) {                  // an entry's row blocks may be taller than the plan's
+      const int rb = (j.m[l] + 159) / 160;
+      pl.rt = std::max(pl.rt, ((j.m[l] + rb - 1) / rb + 31) / 32);
+    }
+    launch_rows_batch(j, nj, pl, ldx, H, H, workspace, stream);
+    dim3 grid = reduce_grid(mmax, nmax);
+    grid.z = nj;
+    hipLaunchKernelGGL(k_norm_linear_reduce_batch, grid, dim3(256), 0, stream, static_cast<const float*>(workspace),
+                       pl.splits, j, rest, static_cast<int>(H), eps, ldo);
+  }
+  if (live == 0) return check_launch(fn);
   if (persistent_lin_ok(H)) {
     hipLaunchKernelGGL(k_norm_linear_p, dim3(persistent_grid(tiles)), dim3(NTHR), 0, stream, ll, live, ldx, ldo,
                        static_cast<int>(H), eps);

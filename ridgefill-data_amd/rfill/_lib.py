@@ -36,6 +36,12 @@ SIGNATURES = {
     "rf_map_apply_batch": [_I32, _P, _I64, _PP, _PP, _PP, _I64, _PP, _I64, _I64, _I64, _P],
     "rf_norm_kv_write_batch": [_I32, _PP, _I64, _PP, _I64, _I64, _F32, _PP, _I32, _I32, _PP, _I32, _P, _I32,
                                _PP, _PP, _I64, _I64, _I64, _I64, _P],
+    "rf_batch_workspace_bytes": [_I32, _I64, _I64, _I64, _PSZ],
+    "rf_norm_linear_batch_workspace_bytes": [_I32, _PI64, _PI64, _I64, _PSZ],
+    "rf_map_apply_batch_ws": [_I32, _P, _I64, _PP, _PP, _PP, _I64, _PP, _I64, _I64, _I64, _P, _SZ, _P],
+    "rf_norm_kv_write_batch_ws": [_I32, _PP, _I64, _PP, _I64, _I64, _F32, _PP, _I32, _I32, _PP, _I32, _P, _I32,
+                                  _PP, _PP, _I64, _I64, _I64, _I64, _P, _SZ, _P],
+    "rf_norm_linear_batch_ws": [_I32, _PP, _I64, _PP, _PI64, _I64, _F32, _PP, _PI64, _PP, _I64, _P, _SZ, _P],
     "rf_row_ssq": [_P, _I64, _P, _I64, _I64, _P],
     "rf_row_scatter": [_P, _I64, _P, _I64, _I64, _P, _I64, _P, _I64, _P],
     "rf_fold_norm": [_P, _P, _I32, _P, _I64, _I64, _P],

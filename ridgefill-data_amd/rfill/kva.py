@@ -147,11 +147,11 @@ class Projector:
         W, B = self._maps(b.device)
         return ops.map_apply(b, W[i], B[i], out, ssq, workspace=workspace)
 
-    def apply_batch(self, ids, b, outs, ssqs):
+    def apply_batch(self, ids, b, outs, ssqs, workspace=None):
         """apply() of several layers in one launch (ops.map_apply_batch): outs[k] / ssqs[k] receive layer ids[k]'s
-        x and row statistics, bit-identical to apply() of it alone without a workspace."""
+        x and row statistics, without a workspace bit-identical to apply() of it alone without one."""
         W, B = self._maps(b.device)
-        ops.map_apply_batch(b, [W[i] for i in ids], [B[i] for i in ids], outs, ssqs)
+        ops.map_apply_batch(b, [W[i] for i in ids], [B[i] for i in ids], outs, ssqs, workspace)
 
     def __call__(self, i, b):
         return self.apply(i, b)[0]
@@ -490,7 +490,13 @@ def fill_late(model, h_split, arm, exact_rows=None, hr=None, cache=None, overlap
         (xi, qi), (xj, qj) = inputs[si], inputs[sj]
         model.fill_batch([i, j], [xi, xj], cache, ssqs=[qi, qj])
 
-    gbuf = []
+    gbuf, gws = [], []
+
+    def batch_ws(need):
+        """This call's workspace of its batched launches (one stream, so they share it)."""
+        if need and (not gws or gws[0].numel() < need):
+            gws[:] = [torch.empty(need, dtype=torch.uint8, device=dev)]
+        return gws[0] if need else None
 
     def can_group(i):                                   # layers filled by their maps, no rows computed between
         return (not computed or decoupled) and fills[i] == "proj"
@@ -499,13 +505,14 @@ def fill_late(model, h_split, arm, exact_rows=None, hr=None, cache=None, overlap
         """The maps of several late layers in one launch (the GEMM fills whole waves of the GPU, with no tail
         per layer), then the group's attention layers' K / V fills in one launch and its GDN layers' fills in
         pairs (any two: the layers' fills are independent), each pair's in-projections in one launch right
-        before its delta-rule fill; each layer's results are bit-identical to its unsplit map apply and fill
-        alone."""
+        before its delta-rule fill. Whole rounds of tiles give each layer the bits of its unsplit map apply and
+        fill alone; rows left over run as products of few rows (the launches' workspace)."""
         while len(gbuf) < len(ids):
             gbuf.append((torch.empty(P, H, dtype=torch.bfloat16, device=dev),
                          torch.empty(P, ops.ssq_parts(H), dtype=torch.float32, device=dev)))
         xs, ss = [g[0] for g in gbuf[:len(ids)]], [g[1] for g in gbuf[:len(ids)]]
-        arm.projector.apply_batch(ids, b, xs, ss)
+        W = arm.projector._maps(dev)[0][ids[0]]
+        arm.projector.apply_batch(ids, b, xs, ss, batch_ws(ops.batch_workspace_bytes(len(ids), P, *W.shape)))
         if rows is not None and not computed:           # given row inputs
             for i, x, q in zip(ids, xs, ss):
                 hri = (hr[i] if isinstance(hr, dict) else hr).to(dev, torch.bfloat16)
@@ -515,11 +522,12 @@ def fill_late(model, h_split, arm, exact_rows=None, hr=None, cache=None, overlap
         attn = [k for k, i in enumerate(ids) if model.layer_types[i] == "attn"]
         if attn:
             model.fill_attn_batch([ids[k] for k in attn], [xs[k] for k in attn], pos, cache,
-                                  ssqs=[ss[k] for k in attn], cs=cs)
+                                  ssqs=[ss[k] for k in attn], cs=cs, get_ws=batch_ws)
         gdn = [k for k, i in enumerate(ids) if model.layer_types[i] == "gdn"]
         for j in range(0, len(gdn), 2):                 # each pair's in-projections, then its fill: the
             ks = gdn[j:j + 2]                           # projected rows are read back while still cached
-            model.fill_batch([ids[k] for k in ks], [xs[k] for k in ks], cache, ssqs=[ss[k] for k in ks])
+            model.fill_batch([ids[k] for k in ks], [xs[k] for k in ks], cache, ssqs=[ss[k] for k in ks],
+                             get_ws=batch_ws)
 
     if overlap:
         two_stream(layers, produce, consume, dev)

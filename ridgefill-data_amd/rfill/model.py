@@ -178,10 +178,11 @@ class FillModel:
         self.commit(c, P)
         return {}
 
-    def fill_attn_batch(self, ids, xs, pos, cache, ssqs=None, cs=None):
+    def fill_attn_batch(self, ids, xs, pos, cache, ssqs=None, cs=None, get_ws=None):
         """fill() of several attention layers over the same rows at once (ops.norm_kv_write_batch): every
         layer's K / V bit-identical to its fill() without a split-K workspace. Layers whose caches do not take
-        the rows at one slot in one buffer layout are filled one at a time."""
+        the rows at one slot in one buffer layout are filled one at a time. get_ws(bytes): gives the batched launch
+        a workspace (ops.norm_kv_write_batch), which changes the order of the last rows' fp32 sums."""
         ids = list(ids)
         if any(self.layer_types[i] != "attn" for i in ids):
             raise ValueError(f"fill_attn_batch: attention layers only, got {ids}")
@@ -205,7 +206,9 @@ class FillModel:
             ws = [self._layer(i) for i in ids]
             ops.norm_kv_write_batch(xs, ssqs, self.eps, [w["wkv"] for w in ws], self.n_kv, self.head_dim,
                                     [w.get("k_norm") for w in ws], self.knorm_kind, cs,
-                                    [cache[i]["kbuf"] for i in ids], [cache[i]["vbuf"] for i in ids], slots[0])
+                                    [cache[i]["kbuf"] for i in ids], [cache[i]["vbuf"] for i in ids], slots[0],
+                                    None if get_ws is None else get_ws(ops.batch_workspace_bytes(
+                                        len(ids), P, 2 * self.n_kv * self.head_dim, xs[0].shape[1])))
         for i in ids:
             self.commit(cache[i], P)
 
@@ -248,7 +251,7 @@ class FillModel:
         those 3 rows alone and the other rows' q columns stay unwritten."""
         return self._fill_rows_batch([w], [x], [ssq])[0]
 
-    def _fill_rows_batch(self, ws, xs, ssqs):
+    def _fill_rows_batch(self, ws, xs, ssqs, get_ws=None):
         """_fill_rows of several GDN layers over the same rows in one launch (ops.norm_linear_batch): per layer
         one entry of every row against the k | v | b | a rows and one of the last 3 rows against the q rows.
         Each value is the bits of the full projection of its row (the same kernel on the same row and weights)."""
@@ -263,13 +266,16 @@ class FillModel:
             es += [q, q[P - 3:]]
             ew += [w["w_in"][nq:], w["w_in"][:nq]]
             eo += [pre[:, nq:], pre[P - 3:, :nq]]
-        ops.norm_linear_batch(ex, es, self.eps, ew, eo)
+        space = None if get_ws is None else get_ws(ops.norm_linear_batch_workspace_bytes(
+            [x.shape[0] for x in ex], [w.shape[0] for w in ew], xs[0].shape[1]))
+        ops.norm_linear_batch(ex, es, self.eps, ew, eo, space)
         return pres
 
-    def fill_batch(self, ids, xs, cache, ssqs=None):
+    def fill_batch(self, ids, xs, cache, ssqs=None, get_ws=None):
         """fill() of up to ops.GDN_BATCH_MAX GDN layers over the same rows at once: their in-projections in one launch
         (_fill_rows_batch), then one batched delta-rule fill (rf_gdn_fill_batch), so the layers' sequential chunk
-        scans run side by side. Every layer's conv and recurrent state is bit-identical to fill() of it alone."""
+        scans run side by side. Without get_ws (as fill_attn_batch) every layer's conv and recurrent state is
+        bit-identical to fill() of it alone."""
         ids = list(ids)
         if not 1 <= len(ids) <= ops.GDN_BATCH_MAX or any(self.layer_types[i] != "gdn" for i in ids):
             raise ValueError(f"fill_batch: 1 .. {ops.GDN_BATCH_MAX} GDN layers, got {ids}")
@@ -279,7 +285,7 @@ class FillModel:
         if P == 0:
             return
         ssqs = [ops.row_ssq(x) if q is None else q for x, q in zip(xs, ssqs or [None] * len(ids))]
-        pres = self._fill_rows_batch([self._layer(i, "gdn") for i in ids], xs, ssqs)
+        pres = self._fill_rows_batch([self._layer(i, "gdn") for i in ids], xs, ssqs, get_ws)
         jobs = []
         for i, x, ssq, pre in zip(ids, xs, ssqs, pres):
             w = self._layer(i, "gdn")

@@ -107,10 +107,34 @@ def _ptr_array(ts):
     return (ctypes.c_void_p * len(ts))(*[_ptr(t) for t in ts])
 
 
-def map_apply_batch(b, ws, cs, outs, ssqs):
+def batch_workspace_bytes(nl, M, N, K):
+    """Bytes of the workspace with which map_apply_batch / norm_kv_write_batch of nl layers, each M x N x K, run the
+    rows that would fill a last round of tiles poorly as products of few rows (0: none do)."""
+    b = ctypes.c_size_t(0)
+    _lib.call("rf_batch_workspace_bytes", nl, M, N, K, ctypes.byref(b))
+    return b.value
+
+
+def norm_linear_batch_workspace_bytes(rows, ns, H):
+    """The same for norm_linear_batch's entries."""
+    b, nl = ctypes.c_size_t(0), len(rows)
+    _lib.call("rf_norm_linear_batch_workspace_bytes", nl, (ctypes.c_int64 * nl)(*rows), (ctypes.c_int64 * nl)(*ns), H,
+              ctypes.byref(b))
+    return b.value
+
+
+def _batch_ws(workspace):
+    if workspace is None:
+        return None, 0
+    _need(workspace, "workspace", torch.uint8, 1)
+    return _ptr(workspace), workspace.numel()
+
+
+def map_apply_batch(b, ws, cs, outs, ssqs, workspace=None):
     """Several late layers' maps in one launch (the fill loop of finish(), code/kva/kva.py:413-415, over
     every layer at once): outs[l] = b ws[l]^T + cs[l] and ssqs[l] its row sum-of-squares partials, each
-    bit-identical to map_apply of that layer alone. Every layer reads the same rows b [P, h_in]; ws[l]
+    bit-identical to map_apply of that layer alone; with a workspace (batch_workspace_bytes) the last rows may run
+    as products of few rows instead, their fp32 sums in another order. Every layer reads the same rows b [P, h_in]; ws[l]
     [h_out, h_in], cs[l] [h_out] or None, outs[l] [P, h_out] (one row stride for all), ssqs[l]
     [P, h_out / 256] contiguous."""
     nl = len(ws)
@@ -134,13 +158,14 @@ def map_apply_batch(b, ws, cs, outs, ssqs):
                              " with the row stride of layer 0's")
         if tuple(ssqs[i].shape) != (P, h_out // SSQ_COLS) or not ssqs[i].is_contiguous():
             raise ValueError(f"map_apply_batch: layer {i} statistics shape")
-    _lib.call("rf_map_apply_batch", nl, _ptr(b), b.stride(0), _ptr_array(ws), _ptr_array(cs), _ptr_array(outs),
-              outs[0].stride(0), _ptr_array(ssqs), P, h_in, h_out, _stream(b))
+    wp, nb = _batch_ws(workspace)
+    _lib.call("rf_map_apply_batch_ws", nl, _ptr(b), b.stride(0), _ptr_array(ws), _ptr_array(cs), _ptr_array(outs),
+              outs[0].stride(0), _ptr_array(ssqs), P, h_in, h_out, wp, nb, _stream(b))
 
 
-def norm_kv_write_batch(xs, ssqs, eps, wkvs, hkv, d, knorms, knorm_kind, cs, kbufs, vbufs, slot_begin):
+def norm_kv_write_batch(xs, ssqs, eps, wkvs, hkv, d, knorms, knorm_kind, cs, kbufs, vbufs, slot_begin, workspace=None):
     """The fused K / V fill (norm_kv_write) of several attention layers in one launch, each layer
-    bit-identical to norm_kv_write of it alone: xs[l] [P, H] (one row stride), ssqs[l], wkvs[l]
+    bit-identical to norm_kv_write of it alone (workspace: as map_apply_batch): xs[l] [P, H] (one row stride), ssqs[l], wkvs[l]
     [2 hkv d, H], knorms[l] [d] (all given or all None), one RoPE table cs [P, rot] for every layer, and
     caches kbufs[l] / vbufs[l] [hkv, cap, d] of one shape and stride, rows [slot_begin, slot_begin + P)."""
     nl = len(xs)
@@ -171,16 +196,18 @@ def norm_kv_write_batch(xs, ssqs, eps, wkvs, hkv, d, knorms, knorm_kind, cs, kbu
             raise ValueError(f"norm_kv_write_batch: layer {i} cache shape or strides differ from layer 0's")
     if cs.shape[0] != P or not cs.is_contiguous():
         raise ValueError("norm_kv_write_batch: cs rows")
-    _lib.call("rf_norm_kv_write_batch", nl, _ptr_array(xs), xs[0].stride(0), _ptr_array(ssqs), P, H, float(eps),
+    wp, nb = _batch_ws(workspace)
+    _lib.call("rf_norm_kv_write_batch_ws", nl, _ptr_array(xs), xs[0].stride(0), _ptr_array(ssqs), P, H, float(eps),
               _ptr_array(wkvs), hkv, d, _ptr_array(knorms) if has_kn else None, int(knorm_kind), _ptr(cs),
-              cs.shape[1], _ptr_array(kbufs), _ptr_array(vbufs), hs, rs, int(slot_begin), cap, _stream(xs[0]))
+              cs.shape[1], _ptr_array(kbufs), _ptr_array(vbufs), hs, rs, int(slot_begin), cap, wp, nb,
+              _stream(xs[0]))
 
 
-def norm_linear_batch(xs, ssqs, eps, ws, outs):
+def norm_linear_batch(xs, ssqs, eps, ws, outs, workspace=None):
     """norm_linear of several entries in one launch (rf_norm_linear_batch): outs[l] = bf16(rms-normed xs[l] @
     ws[l]^T), each bit-identical to norm_linear of it alone without a workspace. Entry l: xs[l] [M_l, H] (one
     row stride for all), ssqs[l] [M_l, H / 256] contiguous, ws[l] [N_l, H] contiguous (N_l % 256 == 0),
-    outs[l] [M_l, N_l] (one row stride for all)."""
+    outs[l] [M_l, N_l] (one row stride for all). workspace (norm_linear_batch_workspace_bytes): as map_apply_batch."""
     nl = len(xs)
     if not 0 < nl <= MAP_BATCH_MAX or not (len(ssqs) == len(ws) == len(outs) == nl):
         raise ValueError("norm_linear_batch: one input, statistics, weight and output per entry")
@@ -204,9 +231,10 @@ def norm_linear_batch(xs, ssqs, eps, ws, outs):
                              " with entry 0's row stride")
         rows.append(M)
         ns.append(N)
-    _lib.call("rf_norm_linear_batch", nl, _ptr_array(xs), xs[0].stride(0), _ptr_array(ssqs),
+    wp, nb = _batch_ws(workspace)
+    _lib.call("rf_norm_linear_batch_ws", nl, _ptr_array(xs), xs[0].stride(0), _ptr_array(ssqs),
               (ctypes.c_int64 * nl)(*rows), H, float(eps), _ptr_array(ws), (ctypes.c_int64 * nl)(*ns),
-              _ptr_array(outs), outs[0].stride(0), _stream(xs[0]))
+              _ptr_array(outs), outs[0].stride(0), wp, nb, _stream(xs[0]))
 
 
 def row_ssq(x, ssq=None):

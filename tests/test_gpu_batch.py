@@ -241,3 +241,64 @@ def test_norm_linear_batch_ragged_entries(dev):
     assert torch.equal(out[P - 3:, :256], ops.norm_linear(x[P - 3:], ssq[P - 3:], 1e-6, w[1]))
     assert torch.equal(out[:130, :512], ops.norm_linear(x[:130], ssq[:130], 1e-6, w[2]))
     assert bool((out[130:P - 3, :512] == 3.0).all()) and bool((out[P - 3:, 256:512] == 3.0).all())
+
+
+# Rows left over by whole rounds of tiles: 1 row, a row block and its edge, several row blocks, every row of a short
+# prompt (3 layers of 1024 x 1024 maps: 12 map tiles a tile row, so 21 tile rows are a round; the linear entries: 32)
+@pytest.mark.parametrize("P", [1, 160, 161, 448, 21 * 256 + 1, 21 * 256 + 30, 32 * 256 + 30])
+@pytest.mark.parametrize("name", sorted(WIDE))
+def test_batch_rows_left_over(dev, name, P):
+    """Batched launches with a workspace against the same without: the rows of whole rounds keep their bits, the rest
+    differ by the order of fp32 sums alone. A sum's two orders differ by at most K 2^-24 of its absolute terms, far
+    below bf16's 2^-9, so a result moves by at most one bf16 spacing of the largest value that formed it, and few do:
+    1e-3 relative Frobenius, single values within 2^-7 of the row's largest."""
+    from rfill import ops
+    from rfill.model import FillModel
+    nl = 3
+    cfg, t = _case(name, nl)
+    H, hkv, d = cfg["hidden_size"], cfg["num_key_value_heads"], cfg["head_dim"]
+    m = FillModel(cfg, t, dev)
+    b = inputs(P, H, seed=41).to(dev)
+    W, B = _maps(H, list(range(nl)), 42)
+    W, B = [w.to(dev) for w in W], [c.to(dev) for c in B]
+    cs = m.rope_table(torch.arange(P, device=dev))
+    slot0, cap = 3, P + 3 + 64
+
+    def run(ws_map, ws_kv, ws_lin, given=None):
+        xs = [torch.empty(P, H, dtype=torch.bfloat16, device=dev) for _ in range(nl)]
+        ss = [torch.empty(P, H // 256, dtype=torch.float32, device=dev) for _ in range(nl)]
+        ops.map_apply_batch(b, W, B, xs, ss, ws_map)
+        gx, gs = (xs, ss) if given is None else given    # the same inputs for both sides of what follows
+        kb = [torch.full((hkv, cap, d), -7.0, dtype=torch.bfloat16, device=dev) for _ in range(nl)]
+        vb = [k.clone() for k in kb]
+        ops.norm_kv_write_batch(gx, gs, m.eps, [m.W[i]["wkv"] for i in range(nl)], hkv, d,
+                                [m.W[i].get("k_norm") for i in range(nl)], m.knorm_kind, cs, kb, vb, slot0, ws_kv)
+        lin = [torch.empty(P, H, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+        ops.norm_linear_batch([gx[0], gx[1], gx[0][:2]], [gs[0], gs[1], gs[0][:2]], m.eps, [W[1], W[2], W[0][:256]],
+                              lin + [torch.empty(2, H, dtype=torch.bfloat16, device=dev)[:, :256]]
+                              if P > 2 else lin + [torch.empty(1, H, dtype=torch.bfloat16, device=dev)[:, :256]], ws_lin)
+        return xs, ss, kb, vb, lin
+
+    n_kv, small = 2 * hkv * d, min(P, 2)
+    need = [ops.batch_workspace_bytes(nl, P, H, H), ops.batch_workspace_bytes(nl, P, n_kv, H),
+            ops.norm_linear_batch_workspace_bytes([P, P, small], [H, H, 256], H)]
+    assert need[2] > 0 if P in (448, 32 * 256 + 30) else need[0] > 0
+    ws = [torch.empty(n, dtype=torch.uint8, device=dev) if n else None for n in need]
+    ref = run(None, None, None)
+    got = run(*ws, given=ref[:2])
+    torch.cuda.synchronize()
+    whole = 21 * 256 if P > 21 * 256 else 0             # (P > 32 * 256: the maps' own plan may end later)
+    for a, r in zip(got[0], ref[0]):
+        assert torch.equal(a[:whole], r[:whole])
+
+    def near(a, r):
+        a, r = a.float(), r.float()
+        assert float((a - r).norm()) <= 1e-3 * float(r.norm())
+        assert bool(((a - r).abs() <= 2.0 ** -7 * r.abs().amax(-1, keepdim=True)).all())
+    for group in (0, 2, 3, 4):
+        for a, r in zip(got[group], ref[group]):
+            near(a, r)
+    for a, r in zip(got[1], ref[1]):
+        assert torch.allclose(a, r, rtol=2e-2)          # sums of 256 squares of bf16 values, each within 2^-8
+    for a in got[2] + got[3]:
+        assert bool((a[:, :slot0] == -7).all()) and bool((a[:, slot0 + P:] == -7).all())
