@@ -305,7 +305,17 @@ __global__ __launch_bounds__(Cfg<AD>::NTHR, 1) void k_attend_causal(CausalArgs a
   // through its L2. Head block hb: K / V head hb / (rep / hpb), its query heads from (hb % (rep / hpb)) hpb.
   const int qbs = gridDim.x, ns = gridDim.z;
   const int u = xcd_tile(blockIdx.x + qbs * (blockIdx.y + gridDim.y * blockIdx.z), qbs * gridDim.y * ns);
-  const int qb = u % qbs, sp = (u / qbs) % ns, hb = u / (qbs * ns);
+  const int qb = u % qbs, hb = u / (qbs * ns);
+  // With fewer than 8 head blocks several XCDs share one: each takes every xcds-th of its splits (class by class),
+  // so that the splits past the early queries, which end at once, are spread over them instead of idling the last.
+  const int xcds = gridDim.y < 8 ? 8 / static_cast<int>(gridDim.y) : 1;
+  int sp = (u / qbs) % ns;
+  if (xcds > 1 && ns > xcds) {
+    const int per = ns / xcds, more = ns % xcds, cut = more * (per + 1);
+    const int cls = sp < cut ? sp / (per + 1) : more + (sp - cut) / per;
+    const int at = sp < cut ? sp - cls * (per + 1) : (sp - cut) - (cls - more) * per;
+    sp = at * xcds + cls;
+  }
   const int hk = hb / (rep / a.hpb), hoff = (hb % (rep / a.hpb)) * a.hpb;
   const int j0 = qb * qp;
   const int jlast = min(j0 + qp, a.nq) - 1;
@@ -559,39 +569,58 @@ size_t part_bytes(int64_t nq, int hq, int hkv, int d, int splits) {
                     : 0;
 }
 
-// Key-range splits {ns, W}: W key tiles per split block, ns = ceil(key tiles / W) splits at most. With
-// enough query blocks to fill the CUs (blocks per CU: one at d 128, two at d 64, by LDS), none. Else W
-// minimises (rounds of live blocks) x (W + 2), the live blocks of query block qb being ceil(ntiles_qb / W)
-// per K / V head: ntiles_qb exact for consecutive queries (qpos null), else from query positions spread
-// evenly over the keys (the exact rows). A round is about 0.8 of the CUs' block slots: measured at 287
-// scattered queries over 28672 keys (32 / 8 heads, d 128), 208 live blocks of 56 tiles take 152 us and
-// 240 of 45 tiles 176 us (the blocks slow each other down through the shared K / V reads). Only the time
-// depends on these estimates, not the results.
+// Key-range splits {ns, W}: W key tiles per split block, ns = ceil(key tiles / W) splits, at most 64. The plan takes
+// the ns of the least estimated time. A block alone takes t us a key tile; all of them
+// together run at most R tiles a us (the chip's power limit: beyond about 200 live blocks more of them only slow each
+// other down, also the second block a CU holds at d 64), so a round of B <= 256 live blocks takes W max(t, B / R) and
+// 6 us to start and end; the splits write and read their partials (b us a block) and add the combine launch. Live blocks of query block qb:
+// ceil(ntiles_qb / W) per head block, ntiles_qb exact for consecutive queries (qpos null), else from query positions
+// spread evenly over the keys (the exact rows; a round then counts as 0.85 of the CUs). Fitted to 16 .. 2500 queries over 3000 .. 28672 keys (32 / 8 heads at
+// d 128, 16 / 2 at d 256), 1 to 64 splits; against the rule before it (rounds of 208 blocks, W + 2 tiles each, none
+// from 256 query blocks up), over 28672 keys, consecutive queries (us): d 128, 1021 queries 481 -> 422, 1499 801 -> 684, 2500 1453
+// -> 1071; d 256, 700 445 -> 357, 1499 914 -> 726, 2500 1411 -> 1152; scattered at d 256: 300 230 -> 145, 1021 513 ->
+// 420 (with the XCDs' interleaved splits). Only the time depends on these estimates, not the results.
 struct Splits {
   int ns, W;
 };
 
+constexpr size_t PART_MAX = 512u << 20;    // bytes of partials that a plan may ask for
+
 Splits causal_plan(int64_t nq, int hq, int hkv, int d, int64_t n_keys, bool scattered, int64_t slot0) {
   const int64_t T = key_tiles(n_keys, d), QB = query_blocks(nq, hq, hkv, d), qp = queries_per_block(hq, hkv, d);
-  const int64_t HB = head_blocks(hq, hkv, d), KT = kt_of(d);
-  if (QB * HB >= 256 * (d == 64 ? 2 : 1) || T <= 1) return Splits{1, static_cast<int>(std::max<int64_t>(T, 1))};
-  const int64_t slots = 208 * (d == 64 ? 2 : 1);
+  const int64_t HB = head_blocks(hq, hkv, d), KT = kt_of(d), slots = 256;
+  if (T <= 1 || QB * HB >= 8 * slots) return Splits{1, static_cast<int>(std::max<int64_t>(T, 1))};
+  const double t = d == 256 ? 1.7 : d == 128 ? 1.45 : 1.24, R = d == 256 ? 124 : d == 128 ? 135 : 190;
+  const double b = d == 256 ? 0.06 : d == 128 ? 0.03 : 0.015, cap = scattered ? 0.85 * slots : slots;
   auto tiles_of = [&](int64_t qb) {
     if (scattered) return std::max<int64_t>(1, (T * (qb + 1) + QB - 1) / QB);
     const int64_t last = slot0 + std::min<int64_t>((qb + 1) * qp, nq) - 1;
     return std::min<int64_t>(T, last / KT + 1);
   };
-  int64_t best_w = T, best_cost = INT64_MAX;
-  for (int64_t W = std::max<int64_t>(2, (T + 63) / 64); W <= T; ++W) {   // at most 64 splits
+  Splits best{1, static_cast<int>(T)};
+  double best_us = 0;
+  for (int64_t ns = 1, W = T + 1; ns <= 64; ++ns) {
+    if ((T + ns - 1) / ns == W) continue;
+    W = (T + ns - 1) / ns;
+    if (ns > 1 && (W < 2 || part_bytes(nq, hq, hkv, d, static_cast<int>((T + W - 1) / W)) > PART_MAX)) break;
     int64_t live = 0;
     for (int64_t qb = 0; qb < QB; ++qb) live += (tiles_of(qb) + W - 1) / W;
-    const int64_t cost = ((live * HB + slots - 1) / slots) * (W + 2);
-    if (cost < best_cost || (cost == best_cost && W > best_w)) {
-      best_cost = cost;
-      best_w = W;
+    live *= HB;
+    const int64_t real = (T + W - 1) / W;
+    if (HB < 8 && real % (8 / HB)) {              // the XCDs' shares of the splits are unequal
+      if (scattered && ns > 1) continue;
+      live = QB * HB * real;
+    }
+    const double whole = static_cast<double>(static_cast<int64_t>(live / cap)), rest = live - whole * cap;
+    double us = whole * (W * std::max(t, slots / R) + 6);
+    if (rest > 0) us += W * std::max(t, rest / R) + 6;
+    if (ns > 1) us += live * b + 0.1 * ns + 6;
+    if (ns == 1 || us < best_us) {
+      best_us = us;
+      best = Splits{static_cast<int>((T + W - 1) / W), static_cast<int>(W)};
     }
   }
-  return Splits{static_cast<int>((T + best_w - 1) / best_w), static_cast<int>(best_w)};
+  return best;
 }
 
 // head_dim 64 / 128: groups of 1 .. 8 (a block holds every head of a group); 256: groups of 1 .. 16 (runs of
@@ -612,7 +641,10 @@ extern "C" int rf_attend_causal_workspace_bytes(int64_t nq, int hq, int hkv, int
   if (!causal_shape_ok(hq, hkv, d))
     return fail(RF_EUNSUPPORTED, "rf_attend_causal_workspace_bytes: head_dim %d, %d query heads over %d K / V heads "
                 "(d 64, 128 or 256; a group of 1, 2, 4 or 8, or up to 16 at d 256)", d, hq, hkv);
-  *bytes = part_bytes(nq, hq, hkv, d, causal_plan(nq, hq, hkv, d, n_keys, true, 0).ns);
+  // for queries anywhere and for the last nq keys' own
+  const int ns = std::max(causal_plan(nq, hq, hkv, d, n_keys, true, 0).ns,
+                          causal_plan(nq, hq, hkv, d, n_keys, false, std::max<int64_t>(0, n_keys - nq)).ns);
+  *bytes = part_bytes(nq, hq, hkv, d, ns);
   return RF_OK;
 }
 
