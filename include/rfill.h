@@ -208,12 +208,13 @@ int rf_norm_qkv_rows(const uint16_t* x, int64_t ldx, const float* ssq, int64_t r
 int rf_row_gather(const uint16_t* x, int64_t ldx, int64_t P, int64_t H, const int64_t* rows, int64_t nrows,
                   uint16_t* out, int64_t ldo, float* ssq, hipStream_t stream);
 
-/* The attention layer's input products over at most 512 new rows (code/kva/model.py:247-257, :427-447), one product
+/* The attention layer's input products over at most 512 new rows, or as many as one round of 256 tiles of 256 x 256
+ * takes (code/kva/model.py:247-257, :427-447), one product
  * over w = [wq (hq d rows); wgate (hq d, present when gate is given); wk; wv (hkv d each)], the norm gain folded in:
  * q [rows, hq d] = the normed queries with q_norm and RoPE (table row j for input row j), gate [rows, hq d] = the
  * normed gate projection, K (k_norm, RoPE) and V into cache slots slot_begin .. Same arithmetic and limits as
  * rf_norm_q, rf_norm_linear and rf_norm_kv_write with a workspace; needs the workspace of rf_gemm_workspace_bytes
- * (rows, all w rows, H). */
+ * (rows, all w rows, H), if any. */
 int rf_norm_attn_rows(const uint16_t* x, int64_t ldx, const float* ssq, int64_t rows, int64_t H, float eps,
                       const uint16_t* w, int hq, int hkv, int d, const uint16_t* qnorm, const uint16_t* knorm,
                       int norm_kind, const uint16_t* cs, int rot, uint16_t* q, int64_t ldq, uint16_t* gate, int64_t ldg,

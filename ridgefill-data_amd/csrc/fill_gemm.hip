@@ -821,18 +821,14 @@ __device__ __forceinline__ void v_rows(const KvArgs& a, const KvLane& L, const u
   }
 }
 
-__global__ __launch_bounds__(NTHR) void k_norm_kv(const uint16_t* __restrict__ Xin, int64_t ldx,
-                                                  const uint16_t* __restrict__ W, int M, int N, int K,
-                                                  KvArgs a) {
-  __shared__ uint4 lds[LDS_U4];
+// The tile at rows m0 and weight rows w0 .. w0 + 255, which are the epilogue's columns n0 .. (its K or V columns).
+__device__ __forceinline__ void norm_kv_tile(const uint16_t* __restrict__ Xin, int64_t ldx,
+                                             const uint16_t* __restrict__ W, int M, int K, int m0, int w0, int n0,
+                                             const KvArgs& a, uint4* lds) {
   float* rsc = reinterpret_cast<float*>(lds + IMAGE_U4);         // [256] row norm scales
-  const int tiles_n = N / BN;
-  int tm, tn;
-  tile_coords(xcd_tile(blockIdx.x, gridDim.x), (M + BM - 1) / BM, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
   const float my_rs = row_scale(a.ssq, a.nparts, a.h, a.eps, M, m0);
   f32x16 acc[4][4];
-  mainloop(Xin, ldx, W, K, M, K, m0, n0, lds, acc);
+  mainloop(Xin, ldx, W, K, M, K, m0, w0, lds, acc);
   rsc[threadIdx.x] = my_rs;
   __syncthreads();
 
@@ -864,6 +860,29 @@ __global__ __launch_bounds__(NTHR) void k_norm_kv(const uint16_t* __restrict__ X
       kv_chunk_row(a, L, [&](int c) { return image_chunk(lds, row, c); }, ch, gm, gm < M, rope_fetch(a, L, gm, gm < M));
     }
   }
+}
+
+__global__ __launch_bounds__(NTHR) void k_norm_kv(const uint16_t* __restrict__ Xin, int64_t ldx,
+                                                  const uint16_t* __restrict__ W, int M, int N, int K,
+                                                  KvArgs a) {
+  __shared__ uint4 lds[LDS_U4];
+  int tm, tn;
+  tile_coords(xcd_tile(blockIdx.x, gridDim.x), (M + BM - 1) / BM, N / BN, tm, tn);
+  norm_kv_tile(Xin, ldx, W, M, K, tm * BM, tn * BN, tn * BN, a, lds);
+}
+
+// Column groups with an epilogue each, as k_norm_attn_reduce: column blocks [0, c1) take a0, [c1, c2) a1, the rest
+// a2. One round of tiles where the products apart leave CUs idle or pay for split planes: 1499 rows at 16 query and 2
+// K / V heads of 256 over width 2048, 216 tiles, 97 us against 138 as three products.
+__global__ __launch_bounds__(NTHR) void k_norm_attn(const uint16_t* __restrict__ Xin, int64_t ldx,
+                                                    const uint16_t* __restrict__ W, int M, int N, int K, KvArgs a0,
+                                                    KvArgs a1, KvArgs a2, int c1, int c2) {
+  __shared__ uint4 lds[LDS_U4];
+  int tm, tn;
+  tile_coords(xcd_tile(blockIdx.x, gridDim.x), (M + BM - 1) / BM, N / BN, tm, tn);
+  const int first = tn < c1 ? 0 : tn < c2 ? c1 : c2;              // block-uniform
+  const KvArgs a = tn < c1 ? a0 : tn < c2 ? a1 : a2;
+  norm_kv_tile(Xin, ldx, W, M, K, tm * BM, tn * BN, (tn - first) * BN, a, lds);
 }
 
 // out = bf16(r_row * (x W^T)) with W's columns carrying the input norm gain (rf_fold_norm) and
@@ -2061,87 +2080,6 @@ int split_count(int64_t M, int64_t N, int64_t K) {
   return static_cast<int>(std::max<int64_t>(s, 1));
 }
 
-// How an M x N x K product runs: rows [0, m_fused) through the fused kernel, rows [m_fused, M) with K split
-// `splits` ways (k_gemm_partial + a reduce kernel) when splits > 1. Too few tiles for the GPU: all rows
-// split. Otherwise, when whole tile rows fill the waves (N / 256 divides 256) and the last wave is at
-// most half full, its tile rows are split, so that wave takes a fraction of a tile's time.
-// Products of at most ROWS_MAX rows take k_rows_partial (rt row tiles per row block, rblocks row blocks)
-// for every row, split so that about one block runs per CU, then the reduce epilogue.
-struct Plan {
-  int64_t m_fused;
-  int splits;
-  int rt = 0;
-  int rblocks = 0;
-  bool split() const { return splits > 1 || rt > 0; }
-};
-
-Plan plan(int64_t M, int64_t N, int64_t K) {
-  if (M <= ROWS_MAX && N % RN == 0) {
-    const int64_t rb = (M + 159) / 160, per = (M + rb - 1) / rb;
-    const int64_t blocks = rb * (N / RN);
-    const int64_t s = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / blocks, K / 512), 16));
-    return Plan{0, static_cast<int>(s), static_cast<int>((per + 31) / 32), static_cast<int>(rb)};
-  }
-  const int64_t tiles_n = N / BN, trows = (M + BM - 1) / BM;
-  if (trows * tiles_n < 256) {
-    const int s = split_count(M, N, K);
-    return s > 1 ? Plan{0, s} : Plan{M, 1};
-  }
-  if (256 % tiles_n == 0) {
-    const int64_t rem = trows % (256 / tiles_n);
-    if (rem && 2 * rem * tiles_n <= 256) {
-      const int64_t s = std::min<int64_t>(std::min<int64_t>(256 / (rem * tiles_n), K / 512), 16);
-      if (s > 1) return Plan{(trows - rem) * BM, static_cast<int>(s)};
-    }
-  }
-  return Plan{M, 1};
-}
-
-size_t split_bytes(int64_t M, int64_t N, int64_t K) {
-  const Plan p = plan(M, N, K);
-  return p.split() ? static_cast<size_t>(p.splits) * (M - p.m_fused) * N * 4 : 0;
-}
-
-// Workspace of a product over `rows` scattered rows run in chunks of ROWS_MAX rows, each chunk planned on
-// its own: the largest of a full chunk's and the last (shorter) chunk's split bytes. A shorter chunk can
-// need more than a full one, since fewer row blocks leave room for more K splits.
-size_t rows_split_bytes(int64_t rows, int64_t N, int64_t K) {
-  size_t b = 0;
-  if (rows >= ROWS_MAX) b = split_bytes(ROWS_MAX, N, K);
-  if (rows % ROWS_MAX) b = std::max(b, split_bytes(rows % ROWS_MAX, N, K));
-  return b;
-}
-
-// The plan an entry point follows with this workspace: the split part only if the workspace holds it.
-Plan plan_with(int64_t M, int64_t N, int64_t K, const void* ws, size_t ws_bytes) {
-  const Plan p = plan(M, N, K);
-  if (!p.split() || !ws || ws_bytes < split_bytes(M, N, K)) return Plan{M, 1};
-  return p;
-}
-
-// The split partials of rows [m0, M) of an M x N x K product into ws.
-void launch_partials(const uint16_t* X, int64_t ldx, const uint16_t* W, int64_t ldw, int64_t M, int64_t N, int64_t K,
-                     const Plan& p, void* ws, hipStream_t stream) {
-  const int64_t rows = M - p.m_fused;
-  const int kper = static_cast<int>((K / p.splits + BK - 1) / BK * BK);
-  if (p.rt > 0) {
-    const dim3 grid(static_cast<unsigned>(N / RN * p.rblocks * p.splits));
-    const int m = static_cast<int>(rows), n = static_cast<int>(N), k = static_cast<int>(K);
-    float* out = static_cast<float*>(ws);
-    switch (p.rt) {
-      case 1: hipLaunchKernelGGL(k_rows_partial<1>, grid, dim3(NTHR), 0, stream, X, ldx, W, ldw, m, n, k, kper, p.rblocks, out); break;
-      case 2: hipLaunchKernelGGL(k_rows_partial<2>, grid, dim3(NTHR), 0, stream, X, ldx, W, ldw, m, n, k, kper, p.rblocks, out); break;
-      case 3: hipLaunchKernelGGL(k_rows_partial<3>, grid, dim3(NTHR), 0, stream, X, ldx, W, ldw, m, n, k, kper, p.rblocks, out); break;
-      case 4: hipLaunchKernelGGL(k_rows_partial<4>, grid, dim3(NTHR), 0, stream, X, ldx, W, ldw, m, n, k, kper, p.rblocks, out); break;
-      default: hipLaunchKernelGGL(k_rows_partial<5>, grid, dim3(NTHR), 0, stream, X, ldx, W, ldw, m, n, k, kper, p.rblocks, out); break;
-    }
-    return;
-  }
-  hipLaunchKernelGGL(k_gemm_partial, dim3(grid_of(rows, N) * p.splits), dim3(NTHR), 0, stream, X + p.m_fused * ldx,
-                     ldx, W, ldw, static_cast<int>(rows), static_cast<int>(N), static_cast<int>(K), kper,
-                     static_cast<float*>(ws));
-}
-
 // How a batched launch of nl products, each M x N x K, runs: rows [0, m_fused) of every entry as 256 x 256 tiles,
 // the rest (at most BATCH_ROWS rows, rblocks row blocks of at most 160 each) as products of few rows with K split
 // `splits` ways. A round of tiles on the 256 CUs costs the same whether all of them have one or only a few do, and a
@@ -2190,7 +2128,106 @@ BatchPlan batch_plan(int64_t cblocks, int64_t M, int64_t K) {
   return best;
 }
 
+// How an M x N x K product runs: rows [0, m_fused) through the fused kernel, rows [m_fused, M) with K split
+// `splits` ways (k_gemm_partial + a reduce kernel) when splits > 1. Too few tiles for the GPU: all rows
+// split. Otherwise, when whole tile rows fill the waves (N / 256 divides 256) and the last wave is at
+// most half full, its tile rows are split, so that wave takes a fraction of a tile's time.
+// Products of at most ROWS_MAX rows take k_rows_partial (rt row tiles per row block, rblocks row blocks)
+// for every row, split so that about one block runs per CU, then the reduce epilogue. So do the last rows of other
+// widths where batch_plan says so: 1499 x 12288 x 2048 (288 tiles) 102 us in two rounds, 93 as one
+// round and 219 rows.
+struct Plan {
+  int64_t m_fused;
+  int splits;
+  int rt = 0;
+  int rblocks = 0;
+  bool split() const { return splits > 1 || rt > 0; }
+};
+
+Plan plan(int64_t M, int64_t N, int64_t K) {
+  if (M <= ROWS_MAX && N % RN == 0) {
+    const int64_t rb = (M + 159) / 160, per = (M + rb - 1) / rb;
+    const int64_t blocks = rb * (N / RN);
+    const int64_t s = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / blocks, K / 512), 16));
+    return Plan{0, static_cast<int>(s), static_cast<int>((per + 31) / 32), static_cast<int>(rb)};
+  }
+  const int64_t tiles_n = N / BN, trows = (M + BM - 1) / BM;
+  if (trows * tiles_n < 256) {
+    const int s = split_count(M, N, K);
+    return s > 1 ? Plan{0, s} : Plan{M, 1};
+  }
+  if (256 % tiles_n == 0) {
+    const int64_t rem = trows % (256 / tiles_n);
+    if (rem && 2 * rem * tiles_n <= 256) {
+      const int64_t s = std::min<int64_t>(std::min<int64_t>(256 / (rem * tiles_n), K / 512), 16);
+      if (s > 1) return Plan{(trows - rem) * BM, static_cast<int>(s)};
+    }
+    return Plan{M, 1};
+  }
+  // tile rows that do not divide a round: the rows past the whole rounds as products of few rows, where that is less
+  const BatchPlan b = batch_plan(tiles_n, M, K);
+  return b.rows() ? Plan{b.m_fused, b.splits, b.rt, b.rblocks} : Plan{M, 1};
+}
+
+size_t split_bytes(int64_t M, int64_t N, int64_t K) {
+  const Plan p = plan(M, N, K);
+  return p.split() ? static_cast<size_t>(p.splits) * (M - p.m_fused) * N * 4 : 0;
+}
+
+// Workspace of a product over `rows` scattered rows run in chunks of ROWS_MAX rows, each chunk planned on
+// its own: the largest of a full chunk's and the last (shorter) chunk's split bytes. A shorter chunk can
+// need more than a full one, since fewer row blocks leave room for more K splits.
+size_t rows_split_bytes(int64_t rows, int64_t N, int64_t K) {
+  size_t b = 0;
+  if (rows >= ROWS_MAX) b = split_bytes(ROWS_MAX, N, K);
+  if (rows % ROWS_MAX) b = std::max(b, split_bytes(rows % ROWS_MAX, N, K));
+  return b;
+}
+
+// The plan an entry point follows with this workspace: the split part only if the workspace holds it.
+Plan plan_with(int64_t M, int64_t N, int64_t K, const void* ws, size_t ws_bytes) {
+  const Plan p = plan(M, N, K);
+  if (!p.split() || !ws || ws_bytes < split_bytes(M, N, K)) return Plan{M, 1};
+  return p;
+}
+
+// The split partials of rows [m0, M) of an M x N x K product into ws.
+void launch_partials(const uint16_t* X, int64_t ldx, const uint16_t* W, int64_t ldw, int64_t M, int64_t N, int64_t K,
+                     const Plan& p, void* ws, hipStream_t stream) {
+  const int64_t rows = M - p.m_fused;
+  const int kper = static_cast<int>((K / p.splits + BK - 1) / BK * BK);
+  if (p.rt > 0) {
+    const dim3 grid(static_cast<unsigned>(N / RN * p.rblocks * p.splits));
+    const int m = static_cast<int>(rows), n = static_cast<int>(N), k = static_cast<int>(K);
+    float* out = static_cast<float*>(ws);
+    X += p.m_fused * ldx;
+    switch (p.rt) {
+      case 1: hipLaunchKernelGGL(k_rows_partial<1>, grid, dim3(NTHR), 0, stream, X, ldx, W, ldw, m, n, k, kper, p.rblocks, out); break;
+      case 2: hipLaunchKernelGGL(k_rows_partial<2>, grid, dim3(NTHR), 0, stream, X, ldx, W, ldw, m, n, k, kper, p.rblocks, out); break;
+      case 3: hipLaunchKernelGGL(k_rows_partial<3>, grid, dim3(NTHR), 0, stream, X, ldx, W, ldw, m, n, k, kper, p.rblocks, out); break;
+      case 4: hipLaunchKernelGGL(k_rows_partial<4>, grid, dim3(NTHR), 0, stream, X, ldx, W, ldw, m, n, k, kper, p.rblocks, out); break;
+      default: hipLaunchKernelGGL(k_rows_partial<5>, grid, dim3(NTHR), 0, stream, X, ldx, W, ldw, m, n, k, kper, p.rblocks, out); break;
+    }
+    return;
+  }
+  hipLaunchKernelGGL(k_gemm_partial, dim3(grid_of(rows, N) * p.splits), dim3(NTHR), 0, stream, X + p.m_fused * ldx,
+                     ldx, W, ldw, static_cast<int>(rows), static_cast<int>(N), static_cast<int>(K), kper,
+                     static_cast<float*>(ws));
+}
+
+// A K / V batch of narrow models (H < 1024: the per-tile kernel, one launch a layer): every row of every layer as
+// products of few rows, one split (the tiles' bits), where that is less than the layers' launches one after another.
+// Three layers of 1792 x 256 x 256: 93 us as three launches of 7 tiles, 18 as one product and one epilogue launch.
+bool small_kv(int64_t nl, int64_t M, int64_t N, int64_t K, RowShape* r) {
+  if (K >= 1024 || M <= 0 || M > 4096) return false;
+  *r = batch_rows_shape(nl * (N / BN), M, K);
+  const double tiles = static_cast<double>(nl) * ((grid_of(M, N) + 255) / 256) * (1.45 * (K / BK) + 25);
+  return r->splits == 1 && r->us < tiles;
+}
+
 size_t batch_bytes(int64_t nl, int64_t M, int64_t N, int64_t K) {
+  RowShape r{};
+  if (small_kv(nl, M, N, K, &r)) return static_cast<size_t>(nl) * M * N * 4;
   const BatchPlan p = batch_plan(nl * (N / BN), M, K);
   return p.rows() ? static_cast<size_t>(nl) * p.splits * (M - p.m_fused) * N * 4 : 0;
 }
@@ -2547,8 +2584,8 @@ extern "C" int rf_norm_attn_rows(const uint16_t* x, int64_t ldx, const float* ss
                                  int64_t ldg, uint16_t* kbuf, uint16_t* vbuf, int64_t head_stride, int64_t row_stride,
                                  int64_t slot_begin, int64_t cap, void* workspace, size_t ws_bytes, hipStream_t stream) {
   const char* fn = "rf_norm_attn_rows";
-  if (!x || !ssq || !w || !cs || !q || !kbuf || !vbuf || !workspace) return fail(RF_EINVAL_ARG, "%s: null pointer", fn);
-  if (rows < 0 || rows > ROWS_MAX) return fail(RF_EINVAL_SHAPE, "%s: %lld rows (0 .. 512)", fn, (long long)rows);
+  if (!x || !ssq || !w || !cs || !q || !kbuf || !vbuf) return fail(RF_EINVAL_ARG, "%s: null pointer", fn);
+  if (rows < 0 || rows > (1 << 16)) return fail(RF_EINVAL_SHAPE, "%s: %lld rows", fn, (long long)rows);
   if (H <= 0 || H % BK || H % SSQ_COLS)
     return fail(RF_EINVAL_SHAPE, "%s: H = %lld must be a multiple of 256", fn, (long long)H);
   if (d <= 0 || d % 8 || 256 % d || hq <= 0 || hkv <= 0 || (static_cast<int64_t>(hq) * d) % BN ||
@@ -2567,16 +2604,17 @@ extern "C" int rf_norm_attn_rows(const uint16_t* x, int64_t ldx, const float* ss
     return fail(RF_EINVAL_SHAPE, "%s: rows [%lld, %lld) exceed cache capacity %lld", fn, (long long)slot_begin,
                 (long long)(slot_begin + rows), (long long)cap);
   if (!aligned16(x) || !aligned16(w) || !aligned16(q) || !aligned16(kbuf) || !aligned16(vbuf) || !aligned16(cs) ||
-      !aligned16(workspace) || (gate && !aligned16(gate)) || (qnorm && !aligned16(qnorm)) || (knorm && !aligned16(knorm)))
+      (workspace && !aligned16(workspace)) || (gate && !aligned16(gate)) || (qnorm && !aligned16(qnorm)) || (knorm && !aligned16(knorm)))
     return fail(RF_EINVAL_SHAPE, "%s: pointers must be 16-byte aligned", fn);
   if (!(eps >= 0.f)) return fail(RF_EINVAL_ARG, "%s: eps %g", fn, static_cast<double>(eps));
   if (rows == 0) return RF_OK;
+  if (rows > ROWS_MAX && grid_of(rows, N) > 256)
+    return fail(RF_EINVAL_SHAPE, "%s: %lld rows (at most 512, or one round of 256 tiles)", fn, (long long)rows);
   const Plan pl = plan(rows, N, H);
   const size_t need = split_bytes(rows, N, H);
-  if (ws_bytes < need)
+  if (need && (!workspace || ws_bytes < need))
     return fail(RF_EINVAL_ARG, "%s: workspace %zu bytes, needs %zu (rf_gemm_workspace_bytes of %lld x %lld x %lld)", fn,
                 ws_bytes, need, (long long)rows, (long long)N, (long long)H);
-  launch_partials(x, ldx, w, H, rows, N, H, pl, workspace, stream);
   const int nparts = static_cast<int>(H / SSQ_COLS);
   // [queries | gate | K | V] columns: the queries as K columns of hq heads, the gate as V columns (copied)
   const KvArgs aq{ssq, nparts, static_cast<float>(H), eps, hq, d, qnorm, norm_kind, cs, rot, q, q,
@@ -2589,6 +2627,12 @@ extern "C" int rf_norm_attn_rows(const uint16_t* x, int64_t ldx, const float* ss
   const KvArgs akv{ssq, nparts, static_cast<float>(H), eps, hkv, d, knorm, norm_kind, cs, rot, kbuf, vbuf, head_stride,
                    row_stride, slot_begin, nullptr};
   const int c1 = static_cast<int>(NQ / BN), c2 = gate ? 2 * c1 : static_cast<int>(N / BN);
+  if (!pl.split()) {                                // one round of tiles
+    hipLaunchKernelGGL(k_norm_attn, dim3(grid_of(rows, N)), dim3(NTHR), 0, stream, x, ldx, w, static_cast<int>(rows),
+                       static_cast<int>(N), static_cast<int>(H), aq, gate ? ag : akv, akv, c1, c2);
+    return check_launch(fn);
+  }
+  launch_partials(x, ldx, w, H, rows, N, H, pl, workspace, stream);
   hipLaunchKernelGGL(k_norm_attn_reduce, reduce_grid(rows, N), dim3(256), 0, stream,
                      static_cast<const float*>(workspace), pl.splits, static_cast<int>(rows), static_cast<int>(N), aq,
                      gate ? ag : akv, akv, c1, c2);
@@ -3000,9 +3044,12 @@ extern "C" int rf_norm_kv_write_batch_ws(int nl, const uint16_t* const* x, int64
            nullptr, nullptr, head_stride, row_stride, slot_begin, nullptr};
   a.knorm = knorm ? knorm[0] : nullptr;            // the K epilogue's mode follows the (shared) configuration
   if (workspace && !aligned16(workspace)) return fail(RF_EINVAL_SHAPE, "rf_norm_kv_write_batch: workspace alignment");
-  if (persistent_kv_ok(H, rot, P)) {
-    BatchPlan pl = batch_plan(nl * (N / BN), P, H);
-    if (pl.rows() && (!workspace || ws_bytes < batch_bytes(nl, P, N, H))) pl = BatchPlan{P};
+  RowShape few{};
+  const bool tiled = persistent_kv_ok(H, rot, P);
+  const bool small = !tiled && workspace && ws_bytes >= batch_bytes(nl, P, N, H) && small_kv(nl, P, N, H, &few);
+  if (tiled || small) {
+    BatchPlan pl = small ? BatchPlan{0, few.splits, few.rt, few.rblocks} : batch_plan(nl * (N / BN), P, H);
+    if (pl.rows() && !small && (!workspace || ws_bytes < batch_bytes(nl, P, N, H))) pl = BatchPlan{P};
     const int64_t mf = pl.m_fused;
     if (mf > 0) launch_norm_kv_p(kl, nl, ldx, mf, N, H, a, stream);
     if (pl.rows()) {

@@ -527,7 +527,7 @@ class FillModel:
         slot = self.reserve(c, T, self.n_kv, self.head_dim, h.device)
         H = h.shape[1]
         gate = None
-        if 0 < T <= ops.ROWS_MAX:                       # few rows: queries, gate, K and V from one product
+        if T and ops.attn_rows_ok(T, w["wattn"].shape[0]):      # queries, gate, K and V from one product
             q, gate = ops.norm_attn_rows(h, ssq, self.eps, w["wattn"], self.n_heads, self.n_kv, self.head_dim,
                                          w.get("q_norm"), w.get("k_norm"), self.knorm_kind, cs, c["kbuf"], c["vbuf"],
                                          slot, gate="wgate" in w,

@@ -401,9 +401,14 @@ def norm_qkv_rows(x, ssq, eps, wqkv, hq, hkv, d, qnorm, knorm, norm_kind, cs, po
     return out
 
 
+def attn_rows_ok(rows, n):
+    """Whether norm_attn_rows takes `rows` rows of n weight rows: few rows, or at most one tile of 256 x 256 per CU."""
+    return rows <= ROWS_MAX or -(-rows // 256) * (n // 256) <= 256
+
+
 def norm_attn_rows(x, ssq, eps, w, hq, hkv, d, qnorm, knorm, norm_kind, cs, kbuf, vbuf, slot_begin, gate=False,
                    workspace="auto"):
-    """The queries, the output gate (gate) and the K / V of at most ROWS_MAX new rows from one product over w =
+    """The queries, the output gate (gate) and the K / V of new rows (attn_rows_ok) from one product over w =
     [wq; wgate; wkv] (without gate [wq; wkv]): queries [rows, hq d] as norm_q at table rows 0 .., the gate's
     projection [rows, hq d] (None without gate) as norm_linear, and K / V into cache slots slot_begin .. as
     norm_kv_write. Returns (queries, gate)."""
@@ -413,8 +418,8 @@ def norm_attn_rows(x, ssq, eps, w, hq, hkv, d, qnorm, knorm, norm_kind, cs, kbuf
     _need(cs, "cs", torch.bfloat16, 2)
     rows, H = x.shape
     n = ((2 if gate else 1) * hq + 2 * hkv) * d
-    if rows > ROWS_MAX or tuple(ssq.shape) != (rows, ssq_parts(H)) or not ssq.is_contiguous():
-        raise ValueError(f"norm_attn_rows: {rows} rows (at most {ROWS_MAX}), ssq {tuple(ssq.shape)}")
+    if not attn_rows_ok(rows, n) or tuple(ssq.shape) != (rows, ssq_parts(H)) or not ssq.is_contiguous():
+        raise ValueError(f"norm_attn_rows: {rows} rows (at most {ROWS_MAX}, or one round of tiles), ssq {tuple(ssq.shape)}")
     if tuple(w.shape) != (n, H) or not w.is_contiguous() or cs.shape[0] != rows or not cs.is_contiguous():
         raise ValueError(f"norm_attn_rows: w {tuple(w.shape)}, expected ({n}, {H}); cs {tuple(cs.shape)}")
     for name, t in (("qnorm", qnorm), ("knorm", knorm)):

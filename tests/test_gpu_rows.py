@@ -449,15 +449,16 @@ def test_fused_residual_and_swiglu_epilogues_are_bit_identical(dev, R):
 
 @pytest.mark.parametrize("rows,H,hq,hkv,d,rot,gate,norms", [
     (1, 256, 4, 2, 64, 64, False, False), (37, 1024, 8, 2, 128, 128, False, True), (512, 1024, 8, 2, 128, 128, False, False),
-    (9, 2048, 16, 2, 256, 64, True, True), (161, 1280, 4, 1, 256, 64, True, True)])
+    (9, 2048, 16, 2, 256, 64, True, True), (161, 1280, 4, 1, 256, 64, True, True),
+    (600, 1024, 8, 2, 128, 128, False, True), (1030, 1024, 16, 2, 256, 64, True, True), (1281, 256, 4, 2, 64, 64, False, False)])
 def test_norm_attn_rows_matches_the_separate_products(dev, rows, H, hq, hkv, d, rot, gate, norms):
     """rf_norm_attn_rows (one row, odd counts, the most rows; one and two row blocks; statistics of 1, 4, 5 and 8
-    partials; with the output gate and partial rotary) against norm_q, norm_linear and norm_kv_write of the same
+    partials; with the output gate and partial rotary; more than 512 rows as split and as whole tiles) against norm_q, norm_linear and norm_kv_write of the same
     weights without a split: only the fp32 order of the K splits differs, i.e. bf16 rounding (5e-3 as above). Other
     cache slots stay as they were."""
     from rfill import ops
     g = torch.Generator().manual_seed(rows + H)
-    n, slot, cap = ((2 if gate else 1) * hq + 2 * hkv) * d, 77, 700
+    n, slot, cap = ((2 if gate else 1) * hq + 2 * hkv) * d, 77, rows + 177
     x = torch.randn(rows, H, generator=g).to(torch.bfloat16).to(dev)
     ssq = ops.row_ssq(x)
     w = (torch.randn(n, H, generator=g) / H ** 0.5).to(torch.bfloat16).to(dev)
@@ -496,3 +497,28 @@ def test_causal_splits_of_few_queries_match_one_pass(dev, nq, n_keys, hq, hkv, d
                             workspace=torch.full((need,), 0xFF, dtype=torch.uint8, device=dev))
     want = ops.attend_causal(q, slot, kb, vb, n_keys, hq, d ** -0.5, workspace=torch.empty(16, dtype=torch.uint8, device=dev))
     assert rel_err(got, want) < 4e-3
+
+
+@pytest.mark.parametrize("M", [1281, 1440, 1441, 1499])
+def test_last_tile_rows_as_few_rows(dev, M):
+    """48 tile columns: five tile rows are a round, the sixth's rows run as products of few rows (1 row, 160, 161, 219:
+    one and two row blocks). With a workspace the first 1280 rows keep the tiles' bits; the rest differ by the fp32
+    order of the K splits, i.e. bf16 rounding (5e-3 as above)."""
+    from rfill import ops
+    H, N = 2048, 48 * 256
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.randn(M, H, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(N, H, generator=g, device=dev) / H ** 0.5).to(torch.bfloat16)
+    c = torch.randn(N, generator=g, device=dev).to(torch.bfloat16)
+    res = torch.randn(M, N, generator=g, device=dev).to(torch.bfloat16)
+    ssq = ops.row_ssq(x)
+    ws = torch.empty(ops.gemm_workspace_bytes(M, N, H), dtype=torch.uint8, device=dev)
+    assert ws.numel() and ws.numel() % ((M - 1280) * N * 4) == 0            # the rows past the first round only
+    pairs = [(ops.norm_linear(x, ssq, 1e-6, w, workspace=ws), ops.norm_linear(x, ssq, 1e-6, w, workspace=None)),
+             (ops.map_apply(x, w, c, workspace=ws)[0], ops.map_apply(x, w, c, workspace=None)[0]),
+             (ops.map_apply_residual(x, w, res, workspace=ws)[0], ops.map_apply_residual(x, w, res, workspace=None)[0]),
+             (ops.norm_linear_swiglu(x, ssq, 1e-6, w, workspace=ws), ops.norm_linear_swiglu(x, ssq, 1e-6, w, workspace=None))]
+    torch.cuda.synchronize()
+    for a, b in pairs:
+        assert torch.equal(a[:1280], b[:1280])
+        assert rel_err(a[1280:], b[1280:]) < 5e-3
