@@ -124,7 +124,7 @@ def load():
 
 def call(name, *args):
     """Call an entry point; raise the mapped exception on a non-zero status."""
-    lib = load()
+    lib = _lib or load()
     status = getattr(lib, name)(*args)
     if status == RF_OK:
         return
