@@ -27,7 +27,7 @@
 // head o = Qd S_prev + P v_new with Qd = q_n e^gamma, P = tril(q_n k_n^T e^{gamma_i - gamma_j}) (q_n, k_n
 // the l2-normed conv outputs, q_n scaled by dk^-1/2) and v_new = T Y of the state before the chunk. The
 // prep also writes Qd, P, T, K and V in plain layouts, the scan stores the state before each chunk, and
-// k_gdn_out (chunk x value head) forms the outputs for all chunks in parallel on fp32 MFMA.
+// k_gdn_out (chunk x value head x half of its columns) forms the outputs for all chunks in parallel on fp32 MFMA.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -679,29 +679,30 @@ struct OutArgs {
   int64_t ldo;
 };
 
-constexpr int SST = DV + 4;                        // fp32 row stride of S and Y in LDS
+constexpr int OC = DV / 2, ONT = OC / 16;          // a block's columns, in 16-wide tiles
+static_assert(ONT == 4, "a lane's columns fill 16 bytes");
+constexpr int SST = OC + 4;                        // fp32 row stride of S and Y in LDS
 
-// Block = (chunk, value head h); wave w forms output rows 16w .. 16w + 15 of the chunk. On
+// Block = (chunk, value head h, half of the head's columns); wave w forms output rows 16w .. 16w + 15 of the chunk. On
 // v_mfma_f32_16x16x4f32 (lane l feeds A[l % 16][l / 16] and B[l / 16][l % 16], holds D[4 (l / 16) + r][l % 16]):
 //   X = K S, Y = beta (V - q X) (q = e^gamma r), v_new = T Y, O = Qd S + P v_new
-// with S the state before the chunk (LDS), Y then v_new shared through LDS; fp32 throughout, bf16 out.
-// T and P are lower triangular, but their products run over all 16 k-steps: two other shapes (a trip
-// count taken from the wave index; the k-steps unrolled by 8) gave wrong products. Both compiled to
-// accumulators rotated through v_accvgpr moves at the loop head, the first read 6 wait states after an
-// 8-pass MFMA. The shape used compiles fully unrolled: 768 MFMAs, no v_accvgpr moves or writes, and at
-// least 10 wait states between an MFMA and the first read of its result. The wave index is made
-// wave-uniform (an SGPR), which changes only the address arithmetic. Each product loads all its A values
-// first and reads the next k-step's B values from LDS before the current step's MFMAs (a scheduling
-// barrier keeps that order; left to itself the compiler read each pair of B values just before its two
-// MFMAs and waited on LDS before each pair). The code keeps those properties (768 MFMAs, no v_accvgpr
-// moves, at least 10 wait states). The outputs are checked against the oracle's chunked rule at the
-// hybrid's widths, and any change here must be rechecked on the GPU.
-__global__ __launch_bounds__(256) void k_gdn_out(OutArgs a) {
+// with S the state before the chunk (LDS), Y then v_new shared through LDS; fp32 throughout, bf16 out. T and P are
+// lower triangular, but their products run over all k-steps.
+// Which k a k-step takes and which columns a column tile takes is free: here a lane's A values are consecutive in
+// memory (20 16-byte loads in all; one value a load before, 96 of them) and its B values, results and outputs
+// consecutive columns (one 16-byte LDS read a k-step for four MFMAs, 8-byte stores). Half the columns take 52 KB of
+// LDS and 78 registers, so blocks share a CU and one's loads run under another's MFMAs. 24 chunks x 32 heads: 96 us
+// before (half the columns alone: 102), 58 now; the MFMAs alone need 31 at the fp32 matrix peak, the operands (126 MB) 25.
+// The code it compiles to keeps three properties, to be rechecked with any change: 384 MFMAs fully unrolled, no
+// v_accvgpr writes or moves, and at least 10 wait states between an MFMA and the first read of its result (34 here; two
+// earlier shapes that rotated accumulators through v_accvgpr moves, first read 6 wait states after an 8-pass MFMA, gave
+// wrong products). The outputs are checked against the oracle's chunked rule at the hybrid's widths.
+__global__ __launch_bounds__(256, 2) void k_gdn_out(OutArgs a) {
   __shared__ __align__(16) float s_l[DK * SST];
   __shared__ __align__(16) float y_l[CH * SST];
   const int t = threadIdx.x, lane = t & 63, lr = lane & 15, lk = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int c = blockIdx.x, h = blockIdx.y;
+  const int c = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * OC;
   const uint8_t* chunk = a.ws + static_cast<size_t>(c) * a.chunk_bytes;
   const uint8_t* ob = chunk + a.out_off + static_cast<size_t>(h) * OUT_HEAD_BYTES;
   const float* S = reinterpret_cast<const float*>(ob + OS_S);
@@ -712,76 +713,98 @@ __global__ __launch_bounds__(256) void k_gdn_out(OutArgs a) {
   const uint16_t* V = reinterpret_cast<const uint16_t*>(ob + OS_V);
   const float* sc = reinterpret_cast<const float*>(chunk + static_cast<size_t>(a.nk) * KH_BYTES +
                                                    static_cast<size_t>(h) * VH_BYTES + TP_BYTES + VP_BYTES);
-  for (int i = t; i < DK * DV / 4; i += 256) {
-    const int row = i / (DV / 4), c4 = i % (DV / 4);
-    *reinterpret_cast<float4*>(s_l + row * SST + 4 * c4) = reinterpret_cast<const float4*>(S)[i];
+#pragma unroll
+  for (int i = t; i < DK * OC / 4; i += 256) {
+    const int row = i / (OC / 4), c4 = i % (OC / 4);
+    *reinterpret_cast<float4*>(s_l + row * SST + 4 * c4) = *reinterpret_cast<const float4*>(S + row * DV + col0 + 4 * c4);
   }
   __syncthreads();
   const int r0 = 16 * w;
-  f32x4 acc[8];
-  // acc += A B over NKS 4-deep k-steps: A from a_of(ks) (this lane's row r0 + lr, k 4 ks + lk), B from the
-  // LDS rows bl (row 4 ks + lk, column 16 nt + lr), the next k-step's B values read before this step's MFMAs
-  auto product = [&](auto a_of, const float* bl, auto nks_c) {
+  f32x4 acc[ONT];
+  // acc += A B over NKS 4-deep k-steps: k-step ks takes k = NKS lk + ks of lane group lk, so that a lane's A values (row
+  // r0 + lr of A, NKS consecutive k) are contiguous in memory, and column tile nt takes the columns ONT lr + nt, so
+  // that a lane's B values of a k-step are contiguous in the LDS row NKS lk + ks (and its results in the output rows);
+  // the next k-step's B values are read before this step's MFMAs
+  auto product = [&](auto& avs, const float* bl, auto nks_c) {
     constexpr int NKS = decltype(nks_c)::value;
-    float avs[NKS];                                 // every A value of the product in flight at once
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) avs[ks] = a_of(ks);
-    float bv[2][8];
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) bv[0][nt] = bl[lk * SST + 16 * nt + lr];
+    const float* br = bl + NKS * lk * SST + ONT * lr;
+    f32x4 bv[2];
+    bv[0] = *reinterpret_cast<const f32x4*>(br);
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
-      const float av = avs[ks];
-      if (ks + 1 < NKS) {
+      if (ks + 1 < NKS) bv[(ks + 1) & 1] = *reinterpret_cast<const f32x4*>(br + (ks + 1) * SST);
+      __builtin_amdgcn_sched_barrier(0);            // (the read stays ahead of this step's MFMAs)
 #pragma unroll
-        for (int nt = 0; nt < 8; ++nt) bv[(ks + 1) & 1][nt] = bl[(4 * (ks + 1) + lk) * SST + 16 * nt + lr];
-      }
-      __builtin_amdgcn_sched_barrier(0);            // (the reads stay ahead of this step's MFMAs)
-#pragma unroll
-      for (int nt = 0; nt < 8; ++nt)
-        acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[ks & 1][nt], acc[nt], 0, 0, 0);
+      for (int nt = 0; nt < ONT; ++nt)
+        acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(avs[ks], bv[ks & 1][nt], acc[nt], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  // n floats of this lane's row of a row-major fp32 matrix, from its own lk-th part
+  auto row_part = [&](const float* m, int ld, auto& avs) {
+    constexpr int N = static_cast<int>(sizeof(avs) / sizeof(float));
+    const float4* src = reinterpret_cast<const float4*>(m + (r0 + lr) * ld + N * lk);
 #pragma unroll
-  for (int nt = 0; nt < 8; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  product([&](int ks) { return bf2f(K[(r0 + lr) * DK + 4 * ks + lk]); }, s_l,     // X = K S
-          std::integral_constant<int, DK / 4>{});
+    for (int q = 0; q < N / 4; ++q) {
+      const float4 v = src[q];
+      avs[4 * q] = v.x;
+      avs[4 * q + 1] = v.y;
+      avs[4 * q + 2] = v.z;
+      avs[4 * q + 3] = v.w;
+    }
+  };
+  auto zero = [&] {
+#pragma unroll
+    for (int nt = 0; nt < ONT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  float a1[DK / 4], a2[CH / 4];
+  {
+    const uint4* src = reinterpret_cast<const uint4*>(K + (r0 + lr) * DK + DK / 4 * lk);
+#pragma unroll
+    for (int q = 0; q < DK / 32; ++q) {
+      const uint4 v = src[q];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a1[8 * q + e] = bf2f(lane_of(v, e));
+    }
+  }
+  zero();
+  product(a1, s_l, std::integral_constant<int, DK / 4>{});                         // X = K S
+  row_part(T, CH, a2);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {                     // Y = beta (V - q X)
     const int i = r0 + 4 * lk + r;
     const float be = sc[SC_BETA + i], qs = sc[SC_Q + i];
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-      const int col = 16 * nt + lr;
-      y_l[i * SST + col] = be * (bf2f(V[i * DV + col]) - qs * acc[nt][r]);
-    }
+    const uint2 v = *reinterpret_cast<const uint2*>(V + i * DV + col0 + ONT * lr);
+    *reinterpret_cast<float4*>(y_l + i * SST + ONT * lr) =
+        make_float4(be * (bf_lo(v.x) - qs * acc[0][r]), be * (bf_hi(v.x) - qs * acc[1][r]),
+                    be * (bf_lo(v.y) - qs * acc[2][r]), be * (bf_hi(v.y) - qs * acc[3][r]));
   }
   __syncthreads();
-#pragma unroll
-  for (int nt = 0; nt < 8; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  product([&](int ks) { return T[(r0 + lr) * CH + 4 * ks + lk]; }, y_l,            // v_new = T Y
-          std::integral_constant<int, CH / 4>{});
+  zero();
+  product(a2, y_l, std::integral_constant<int, CH / 4>{});                         // v_new = T Y
   __syncthreads();                                  // every wave has read Y
 #pragma unroll
   for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) y_l[(r0 + 4 * lk + r) * SST + 16 * nt + lr] = acc[nt][r];
+    *reinterpret_cast<float4*>(y_l + (r0 + 4 * lk + r) * SST + ONT * lr) =
+        make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]);
+  row_part(Qd, DK, a1);
+  row_part(Pm, CH, a2);
   __syncthreads();
-#pragma unroll
-  for (int nt = 0; nt < 8; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  product([&](int ks) { return Qd[(r0 + lr) * DK + 4 * ks + lk]; }, s_l,           // O = Qd S ...
-          std::integral_constant<int, DK / 4>{});
-  product([&](int ks) { return Pm[(r0 + lr) * CH + 4 * ks + lk]; }, y_l,           // ... + P v_new
-          std::integral_constant<int, CH / 4>{});
+  zero();
+  product(a1, s_l, std::integral_constant<int, DK / 4>{});                         // O = Qd S ...
+  product(a2, y_l, std::integral_constant<int, CH / 4>{});                         // ... + P v_new
+  const bool wide = a.ldo % 4 == 0 && (reinterpret_cast<uintptr_t>(a.out) & 7u) == 0;     // uniform
   const int64_t p0 = a.p_begin + static_cast<int64_t>(c) * CH;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int64_t p = p0 + r0 + 4 * lk + r;
     if (p >= a.P) continue;
-    uint16_t* dst = a.out + p * a.ldo + static_cast<int64_t>(h) * DV + lr;
+    uint16_t* dst = a.out + p * a.ldo + static_cast<int64_t>(h) * DV + col0 + ONT * lr;
+    if (wide)
+      *reinterpret_cast<uint2*>(dst) = make_uint2(bf16_pair(acc[0][r], acc[1][r]), bf16_pair(acc[2][r], acc[3][r]));
+    else
 #pragma unroll
-    for (int nt = 0; nt < 8; ++nt) dst[16 * nt] = f2bf(acc[nt][r]);
+      for (int nt = 0; nt < ONT; ++nt) dst[nt] = f2bf(acc[nt][r]);
   }
 }
 
@@ -1010,7 +1033,7 @@ int gdn_run(const char* fn, const LayerIO* io, int n, int64_t P, int nk, int nv,
       hipLaunchKernelGGL(k_gdn_scan<true>, dim3(nv * 8), dim3(256), 0, stream, sb);
       if (const int e = check_launch(fn)) return e;
       OutArgs oa{ws, cbytes, sbytes, nk, P, c0 * CH, out, ldo};
-      hipLaunchKernelGGL(k_gdn_out, dim3(nc, nv), dim3(256), 0, stream, oa);
+      hipLaunchKernelGGL(k_gdn_out, dim3(nc, nv, DV / OC), dim3(256), 0, stream, oa);
       if (const int e = check_launch(fn)) return e;
     } else {
       hipLaunchKernelGGL(k_gdn_prep<false>, dim3(nc, nv, n), dim3(256), 0, stream, pb);
