@@ -213,8 +213,9 @@ int rf_row_gather(const uint16_t* x, int64_t ldx, int64_t P, int64_t H, const in
  * over w = [wq (hq d rows); wgate (hq d, present when gate is given); wk; wv (hkv d each)], the norm gain folded in:
  * q [rows, hq d] = the normed queries with q_norm and RoPE (table row j for input row j), gate [rows, hq d] = the
  * normed gate projection, K (k_norm, RoPE) and V into cache slots slot_begin .. Same arithmetic and limits as
- * rf_norm_q, rf_norm_linear and rf_norm_kv_write with a workspace; needs the workspace of rf_gemm_workspace_bytes
- * (rows, all w rows, H), if any. */
+ * rf_norm_q, rf_norm_linear and rf_norm_kv_write with a workspace; needs the workspace of
+ * rf_norm_attn_rows_workspace_bytes(rows, all w rows, H). */
+int rf_norm_attn_rows_workspace_bytes(int64_t rows, int64_t N, int64_t H, size_t* bytes);
 int rf_norm_attn_rows(const uint16_t* x, int64_t ldx, const float* ssq, int64_t rows, int64_t H, float eps,
                       const uint16_t* w, int hq, int hkv, int d, const uint16_t* qnorm, const uint16_t* knorm,
                       int norm_kind, const uint16_t* cs, int rot, uint16_t* q, int64_t ldq, uint16_t* gate, int64_t ldg,

@@ -821,14 +821,18 @@ __device__ __forceinline__ void v_rows(const KvArgs& a, const KvLane& L, const u
   }
 }
 
-// The tile at rows m0 and weight rows w0 .. w0 + 255, which are the epilogue's columns n0 .. (its K or V columns).
-__device__ __forceinline__ void norm_kv_tile(const uint16_t* __restrict__ Xin, int64_t ldx,
-                                             const uint16_t* __restrict__ W, int M, int K, int m0, int w0, int n0,
-                                             const KvArgs& a, uint4* lds) {
+__global__ __launch_bounds__(NTHR) void k_norm_kv(const uint16_t* __restrict__ Xin, int64_t ldx,
+                                                  const uint16_t* __restrict__ W, int M, int N, int K,
+                                                  KvArgs a) {
+  __shared__ uint4 lds[LDS_U4];
   float* rsc = reinterpret_cast<float*>(lds + IMAGE_U4);         // [256] row norm scales
+  const int tiles_n = N / BN;
+  int tm, tn;
+  tile_coords(xcd_tile(blockIdx.x, gridDim.x), (M + BM - 1) / BM, tiles_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
   const float my_rs = row_scale(a.ssq, a.nparts, a.h, a.eps, M, m0);
   f32x16 acc[4][4];
-  mainloop(Xin, ldx, W, K, M, K, m0, w0, lds, acc);
+  mainloop(Xin, ldx, W, K, M, K, m0, n0, lds, acc);
   rsc[threadIdx.x] = my_rs;
   __syncthreads();
 
@@ -860,29 +864,6 @@ __device__ __forceinline__ void norm_kv_tile(const uint16_t* __restrict__ Xin, i
       kv_chunk_row(a, L, [&](int c) { return image_chunk(lds, row, c); }, ch, gm, gm < M, rope_fetch(a, L, gm, gm < M));
     }
   }
-}
-
-__global__ __launch_bounds__(NTHR) void k_norm_kv(const uint16_t* __restrict__ Xin, int64_t ldx,
-                                                  const uint16_t* __restrict__ W, int M, int N, int K,
-                                                  KvArgs a) {
-  __shared__ uint4 lds[LDS_U4];
-  int tm, tn;
-  tile_coords(xcd_tile(blockIdx.x, gridDim.x), (M + BM - 1) / BM, N / BN, tm, tn);
-  norm_kv_tile(Xin, ldx, W, M, K, tm * BM, tn * BN, tn * BN, a, lds);
-}
-
-// Column groups with an epilogue each, as k_norm_attn_reduce: column blocks [0, c1) take a0, [c1, c2) a1, the rest
-// a2. One round of tiles where the products apart leave CUs idle or pay for split planes: 1499 rows at 16 query and 2
-// K / V heads of 256 over width 2048, 216 tiles, 97 us against 138 as three products.
-__global__ __launch_bounds__(NTHR) void k_norm_attn(const uint16_t* __restrict__ Xin, int64_t ldx,
-                                                    const uint16_t* __restrict__ W, int M, int N, int K, KvArgs a0,
-                                                    KvArgs a1, KvArgs a2, int c1, int c2) {
-  __shared__ uint4 lds[LDS_U4];
-  int tm, tn;
-  tile_coords(xcd_tile(blockIdx.x, gridDim.x), (M + BM - 1) / BM, N / BN, tm, tn);
-  const int first = tn < c1 ? 0 : tn < c2 ? c1 : c2;              // block-uniform
-  const KvArgs a = tn < c1 ? a0 : tn < c2 ? a1 : a2;
-  norm_kv_tile(Xin, ldx, W, M, K, tm * BM, tn * BN, (tn - first) * BN, a, lds);
 }
 
 // out = bf16(r_row * (x W^T)) with W's columns carrying the input norm gain (rf_fold_norm) and
@@ -1062,6 +1043,27 @@ __global__ __launch_bounds__(256) void k_norm_attn_reduce(const float* __restric
   if (y < c1) norm_kv_reduce(part, splits, M, N, y, a0);
   else if (y < c2) norm_kv_reduce(part + static_cast<int64_t>(c1) * BN, splits, M, N, y - c1, a1);
   else norm_kv_reduce(part + static_cast<int64_t>(c2) * BN, splits, M, N, y - c2, a2);
+}
+
+// The same epilogues over a normed product x [M, N] (bf16, as rf_norm_linear leaves it) for more rows: the product on
+// whole persistent tiles, then this row pass with every CU's lanes, rather than k_norm_kv's row pass at one wave per
+// SIMD, whose k_norm and RoPE held the tiles for as long as their products. 1499 rows at 16 query and 2 K / V heads of
+// 256 over width 2048 (216 tiles): 61 + 18 us; as tiles with the row pass 97, as three split products 138.
+__device__ __forceinline__ void norm_attn_finish(const uint16_t* __restrict__ x, int M, int N, int first,
+                                                 const KvArgs& a) {
+  const int t = threadIdx.x, r = t >> 5, ch = t & 31, y = blockIdx.y;
+  const int m = blockIdx.x * RED_ROWS + r;
+  const KvLane L(a, (y - first) * BN, ch);
+  const uint4* row = reinterpret_cast<const uint4*>(x + static_cast<int64_t>(min(m, M - 1)) * N + y * BN);
+  const bool ok = m < M;
+  kv_chunk_row(a, L, [&](int c) { return row[c]; }, ch, m, ok, rope_fetch(a, L, m, ok));
+}
+__global__ __launch_bounds__(256) void k_norm_attn_finish(const uint16_t* __restrict__ x, int M, int N, KvArgs a0,
+                                                          KvArgs a1, KvArgs a2, int c1, int c2) {
+  const int y = blockIdx.y;                         // block-uniform; a branch each (a selected argument went through scratch)
+  if (y < c1) norm_attn_finish(x, M, N, 0, a0);
+  else if (y < c2) norm_attn_finish(x, M, N, c1, a1);
+  else norm_attn_finish(x, M, N, c2, a2);
 }
 
 // Adds a run's fp32 sums (acc) into the fp64 accumulator C for the tile at (m0, n0), rows < M. The sums go
@@ -2578,6 +2580,18 @@ extern "C" int rf_norm_qkv_rows(const uint16_t* x, int64_t ldx, const float* ssq
   return check_launch(fn);
 }
 
+static size_t attn_rows_bytes(int64_t rows, int64_t N, int64_t H) {
+  return plan(rows, N, H).split() ? split_bytes(rows, N, H) : static_cast<size_t>(rows) * N * 2;
+}
+
+extern "C" int rf_norm_attn_rows_workspace_bytes(int64_t rows, int64_t N, int64_t H, size_t* bytes) {
+  if (!bytes || rows < 0 || rows > (1 << 16) || N <= 0 || N % BN || H <= 0 || H % BK)
+    return fail(RF_EINVAL_ARG, "rf_norm_attn_rows_workspace_bytes: rows %lld, N %lld (multiple of 256), H %lld (multiple "
+                "of 64)", (long long)rows, (long long)N, (long long)H);
+  *bytes = rows ? attn_rows_bytes(rows, N, H) : 0;
+  return RF_OK;
+}
+
 extern "C" int rf_norm_attn_rows(const uint16_t* x, int64_t ldx, const float* ssq, int64_t rows, int64_t H, float eps,
                                  const uint16_t* w, int hq, int hkv, int d, const uint16_t* qnorm, const uint16_t* knorm,
                                  int norm_kind, const uint16_t* cs, int rot, uint16_t* q, int64_t ldq, uint16_t* gate,
@@ -2611,10 +2625,10 @@ extern "C" int rf_norm_attn_rows(const uint16_t* x, int64_t ldx, const float* ss
   if (rows > ROWS_MAX && grid_of(rows, N) > 256)
     return fail(RF_EINVAL_SHAPE, "%s: %lld rows (at most 512, or one round of 256 tiles)", fn, (long long)rows);
   const Plan pl = plan(rows, N, H);
-  const size_t need = split_bytes(rows, N, H);
+  const size_t need = attn_rows_bytes(rows, N, H);
   if (need && (!workspace || ws_bytes < need))
-    return fail(RF_EINVAL_ARG, "%s: workspace %zu bytes, needs %zu (rf_gemm_workspace_bytes of %lld x %lld x %lld)", fn,
-                ws_bytes, need, (long long)rows, (long long)N, (long long)H);
+    return fail(RF_EINVAL_ARG, "%s: workspace %zu bytes, needs %zu (rf_norm_attn_rows_workspace_bytes of %lld x %lld x "
+                "%lld)", fn, ws_bytes, need, (long long)rows, (long long)N, (long long)H);
   const int nparts = static_cast<int>(H / SSQ_COLS);
   // [queries | gate | K | V] columns: the queries as K columns of hq heads, the gate as V columns (copied)
   const KvArgs aq{ssq, nparts, static_cast<float>(H), eps, hq, d, qnorm, norm_kind, cs, rot, q, q,
@@ -2628,8 +2642,11 @@ extern "C" int rf_norm_attn_rows(const uint16_t* x, int64_t ldx, const float* ss
                    row_stride, slot_begin, nullptr};
   const int c1 = static_cast<int>(NQ / BN), c2 = gate ? 2 * c1 : static_cast<int>(N / BN);
   if (!pl.split()) {                                // one round of tiles
-    hipLaunchKernelGGL(k_norm_attn, dim3(grid_of(rows, N)), dim3(NTHR), 0, stream, x, ldx, w, static_cast<int>(rows),
-                       static_cast<int>(N), static_cast<int>(H), aq, gate ? ag : akv, akv, c1, c2);
+    uint16_t* prod = static_cast<uint16_t*>(workspace);
+    const int rc = rf_norm_linear(x, ldx, ssq, rows, H, eps, w, N, prod, N, nullptr, 0, stream);
+    if (rc != RF_OK) return rc;
+    hipLaunchKernelGGL(k_norm_attn_finish, reduce_grid(rows, N), dim3(256), 0, stream, prod, static_cast<int>(rows),
+                       static_cast<int>(N), aq, gate ? ag : akv, akv, c1, c2);
     return check_launch(fn);
   }
   launch_partials(x, ldx, w, H, rows, N, H, pl, workspace, stream);

@@ -79,6 +79,7 @@ SIGNATURES = {
     "rf_norm_linear_swiglu": [_P, _I64, _P, _I64, _I64, _F32, _P, _I64, _P, _I64, _P, _I64, _P, _SZ, _P],
     "rf_norm_qkv_rows": [_P, _I64, _P, _I64, _I64, _F32, _P, _I32, _I32, _I32, _P, _P, _I32, _P, _I32, _P, _I64, _P,
                          _I64, _P, _P, _I64, _I64, _P, _SZ, _P],
+    "rf_norm_attn_rows_workspace_bytes": [_I64, _I64, _I64, _PSZ],
     "rf_norm_attn_rows": [_P, _I64, _P, _I64, _I64, _F32, _P, _I32, _I32, _I32, _P, _P, _I32, _P, _I32, _P, _I64, _P,
                           _I64, _P, _P, _I64, _I64, _I64, _I64, _P, _SZ, _P],
     "rf_attend_rows": [_P, _I64, _P, _I64, _I32, _I32, _P, _P, _I32, _I64, _I64, _I64, _F32, _P, _I64, _P, _SZ, _P],

@@ -311,12 +311,13 @@ class FillModel:
             self._attn_ws = ws = torch.empty(need, dtype=torch.uint8, device=device)
         return ws
 
-    def gemm_workspace(self, M, N, K, device, role="consume", rows=False):
+    def gemm_workspace(self, M, N, K, device, role="consume", rows=False, size=None):
         """The split-K workspace of an M x N x K product (None when it runs unsplit): one buffer per role,
         shared by every GEMM of that role in stream order -- "consume" for the cache fill and the exact
         rows' and tail's layers, "produce" for the map apply that may run beside them on another stream.
-        rows: size it for norm_kv_rows / norm_qkv_rows over M scattered rows (ops.rows_workspace_bytes)."""
-        need = (ops.rows_workspace_bytes if rows else ops.gemm_workspace_bytes)(M, N, K)
+        rows: size it for norm_kv_rows / norm_qkv_rows over M scattered rows (ops.rows_workspace_bytes); size: by
+        another rule."""
+        need = (size or (ops.rows_workspace_bytes if rows else ops.gemm_workspace_bytes))(M, N, K)
         if need == 0:
             return None
         wss = self.__dict__.setdefault("_gemm_ws", {})
@@ -531,7 +532,8 @@ class FillModel:
             q, gate = ops.norm_attn_rows(h, ssq, self.eps, w["wattn"], self.n_heads, self.n_kv, self.head_dim,
                                          w.get("q_norm"), w.get("k_norm"), self.knorm_kind, cs, c["kbuf"], c["vbuf"],
                                          slot, gate="wgate" in w,
-                                         workspace=self.gemm_workspace(T, w["wattn"].shape[0], H, h.device))
+                                         workspace=self.gemm_workspace(T, w["wattn"].shape[0], H, h.device,
+                                                                       size=ops.norm_attn_rows_workspace_bytes))
         else:
             ops.norm_kv_write(h, ssq, self.eps, w["wkv"], self.n_kv, self.head_dim, w.get("k_norm"), self.knorm_kind,
                               cs, c["kbuf"], c["vbuf"], slot,

@@ -414,6 +414,14 @@ def norm_qkv_rows(x, ssq, eps, wqkv, hq, hkv, d, qnorm, knorm, norm_kind, cs, po
     return out
 
 
+@_size_rule
+def norm_attn_rows_workspace_bytes(rows, n, H):
+    """Bytes of the workspace norm_attn_rows needs for `rows` rows of n weight rows of width H."""
+    b = ctypes.c_size_t(0)
+    _lib.call("rf_norm_attn_rows_workspace_bytes", rows, n, H, ctypes.byref(b))
+    return b.value
+
+
 def attn_rows_ok(rows, n):
     """Whether norm_attn_rows takes `rows` rows of n weight rows: few rows, or at most one tile of 256 x 256 per CU."""
     return rows <= ROWS_MAX or -(-rows // 256) * (n // 256) <= 256
@@ -443,7 +451,7 @@ def norm_attn_rows(x, ssq, eps, w, hq, hkv, d, qnorm, knorm, norm_kind, cs, kbuf
     hs, rs, cap = _cache_args(kbuf, vbuf, hkv, d, slot_begin, rows)
     out = torch.empty(2 if gate else 1, rows, hq * d, dtype=torch.bfloat16, device=x.device)
     q, g = out[0], out[1] if gate else None
-    ws, nb = _ws(workspace, rows, n, H, x.device)
+    ws, nb = _ws(workspace, rows, n, H, x.device, norm_attn_rows_workspace_bytes)
     _lib.call("rf_norm_attn_rows", _ptr(x), x.stride(0), _ptr(ssq), rows, H, float(eps), _ptr(w), hq, hkv, d,
               _ptr(qnorm), _ptr(knorm), int(norm_kind), _ptr(cs), cs.shape[1], _ptr(q), q.stride(0), _ptr(g),
               g.stride(0) if gate else 0, _ptr(kbuf), _ptr(vbuf), hs, rs, int(slot_begin), cap, _ptr(ws), nb, _stream(x))
