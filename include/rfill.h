@@ -526,7 +526,7 @@ int rf_read_cosine(const uint16_t* pred, int64_t ld_pred, const uint16_t* truth,
 
 /* The ridge solve of RidgeFit (code/kva/ridge.py:80-105) in fp64: for each of the nlam values lam (host array
  * lams, each > 0), W_lam = (C + lam scale I)^-1 Cxy with C = cxx [d, d] (row stride ldc; symmetric positive
- * semi-definite, the centred scatter) and Cxy = cxy [d, R] (row stride ldb; the cross statistics of every
+ * semi-definite, its lower triangle is read; the centred scatter) and Cxy = cxy [d, R] (row stride ldb; the cross statistics of every
  * target side by side), written to w + l w_stride as [d, R] (row stride ldw); and, if bias is not NULL,
  * bias + l bias_stride = mean_y - mean_x W_lam ([R]; mean_x [d], mean_y [R] on the device): the unpenalised
  * bias of the centred fit. The inverse of C + lam scale I comes from a block recursion on its Schur

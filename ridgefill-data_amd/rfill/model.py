@@ -204,11 +204,13 @@ class FillModel:
                                   workspace=self.gemm_workspace(P, w["wkv"].shape[0], x.shape[1], x.device))
         else:
             ws = [self._layer(i) for i in ids]
+            n = 2 * self.n_kv * self.head_dim           # (other widths are refused by the launch itself)
+            space = (get_ws(ops.batch_workspace_bytes(len(ids), P, n, xs[0].shape[1]))
+                     if get_ws is not None and n % 256 == 0 else None)
             ops.norm_kv_write_batch(xs, ssqs, self.eps, [w["wkv"] for w in ws], self.n_kv, self.head_dim,
                                     [w.get("k_norm") for w in ws], self.knorm_kind, cs,
                                     [cache[i]["kbuf"] for i in ids], [cache[i]["vbuf"] for i in ids], slots[0],
-                                    None if get_ws is None else get_ws(ops.batch_workspace_bytes(
-                                        len(ids), P, 2 * self.n_kv * self.head_dim, xs[0].shape[1])))
+                                    space)
         for i in ids:
             self.commit(cache[i], P)
 

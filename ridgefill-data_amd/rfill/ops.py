@@ -18,7 +18,7 @@ def _stream(t):
     return ctypes_ptr(torch._C._cuda_getCurrentRawStream(t.get_device()))
 
 
-_size_rule = functools.lru_cache(maxsize=1024)
+_size_rule = functools.lru_cache(maxsize=1024, typed=True)
 
 
 def ctypes_ptr(v):
