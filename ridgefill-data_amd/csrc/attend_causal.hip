@@ -569,17 +569,19 @@ size_t part_bytes(int64_t nq, int hq, int hkv, int d, int splits) {
                     : 0;
 }
 
-// Key-range splits {ns, W}: W key tiles per split block, ns = ceil(key tiles / W) splits, at most 64. The plan takes
-// the ns of the least estimated time. A block alone takes t us a key tile; all of them
-// together run at most R tiles a us (the chip's power limit: beyond about 200 live blocks more of them only slow each
-// other down, also the second block a CU holds at d 64), so a round of B <= 256 live blocks takes W max(t, B / R) and
-// 6 us to start and end; the splits write and read their partials (b us a block) and add the combine launch. Live blocks of query block qb:
-// ceil(ntiles_qb / W) per head block, ntiles_qb exact for consecutive queries (qpos null), else from query positions
-// spread evenly over the keys (the exact rows; a round then counts as 0.85 of the CUs). Fitted to 16 .. 2500 queries over 3000 .. 28672 keys (32 / 8 heads at
-// d 128, 16 / 2 at d 256), 1 to 64 splits; against the rule before it (rounds of 208 blocks, W + 2 tiles each, none
-// from 256 query blocks up), over 28672 keys, consecutive queries (us): d 128, 1021 queries 481 -> 422, 1499 801 -> 684, 2500 1453
-// -> 1071; d 256, 700 445 -> 357, 1499 914 -> 726, 2500 1411 -> 1152; scattered at d 256: 300 230 -> 145, 1021 513 ->
-// 420 (with the XCDs' interleaved splits). Only the time depends on these estimates, not the results.
+// Key-range splits {ns, W}: W key tiles per split block, ns = ceil(key tiles / W) splits, at most 64. The plan
+// takes the ns of the least estimated time. A block alone takes t us a key tile; all of them together run at
+// most R tiles a us (the chip's power limit: beyond about 200 live blocks more of them only slow each other
+// down, also the second block a CU holds at d 64), so a round of B <= 256 live blocks takes W max(t, B / R) and
+// 6 us to start and end; the splits write and read their partials (b us a block) and add the combine launch.
+// Live blocks of query block qb: ceil(ntiles_qb / W) per head block, ntiles_qb exact for consecutive queries
+// (qpos null), else from query positions spread evenly over the keys (the exact rows; a round then counts as
+// 0.85 of the CUs). Fitted to 16 .. 2500 queries over 3000 .. 28672 keys (32 / 8 heads at d 128, 16 / 2 at d
+// 256), 1 to 64 splits; against the rule before it (rounds of 208 blocks, W + 2 tiles each, none from 256 query
+// blocks up), over 28672 keys, consecutive queries (us): d 128, 1021 queries 481 -> 422, 1499 801 -> 684, 2500
+// 1453 -> 1071; d 256, 700 445 -> 357, 1499 914 -> 726, 2500 1411 -> 1152; scattered at d 256: 300 230 -> 145,
+// 1021 513 -> 420 (with the XCDs' interleaved splits). Only the time depends on these estimates, not the
+// results.
 struct Splits {
   int ns, W;
 };
