@@ -268,8 +268,14 @@ int rf_attend_causal(const uint16_t* q, int64_t ldq, int64_t nq, const int64_t* 
                      hipStream_t stream);
 
 /* Workspace bytes rf_attend_causal uses for nq queries over n_keys keys (the full key-range split; 0 when the
- * query blocks alone fill the GPU). Host only. */
+ * query blocks alone fill the GPU), whichever queries they are: the larger of what scattered queries and the last nq
+ * keys' own ask for. Host only. */
 int rf_attend_causal_workspace_bytes(int64_t nq, int hq, int hkv, int d, int64_t n_keys, size_t* bytes);
+
+/* The same for one call's queries: at positions anywhere (scattered; rf_attend_causal with qpos), or at slots
+ * slot0 .. slot0 + nq - 1. Host only. */
+int rf_attend_causal_workspace_bytes_at(int64_t nq, int hq, int hkv, int d, int64_t n_keys, int scattered, int64_t slot0,
+                                        size_t* bytes);
 
 /* out = bf16(x + y) row by row (rows x H) and out's row sum-of-squares partials ssq [rows, H / 256]: the
  * residual adds of layer_rows (code/kva/model.py:274, Model.mlp :114). out may alias x. */

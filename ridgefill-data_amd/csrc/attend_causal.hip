@@ -638,15 +638,31 @@ bool causal_shape_ok(int hq, int hkv, int d) {
 
 using namespace rf;
 
-extern "C" int rf_attend_causal_workspace_bytes(int64_t nq, int hq, int hkv, int d, int64_t n_keys, size_t* bytes) {
-  if (!bytes || nq < 0 || n_keys < 0) return fail(RF_EINVAL_ARG, "rf_attend_causal_workspace_bytes: arguments");
+static int causal_size(const char* fn, int64_t nq, int hq, int hkv, int d, int64_t n_keys, size_t* bytes) {
+  if (!bytes || nq < 0 || n_keys < 0) return fail(RF_EINVAL_ARG, "%s: arguments", fn);
   if (!causal_shape_ok(hq, hkv, d))
-    return fail(RF_EUNSUPPORTED, "rf_attend_causal_workspace_bytes: head_dim %d, %d query heads over %d K / V heads "
-                "(d 64, 128 or 256; a group of 1, 2, 4 or 8, or up to 16 at d 256)", d, hq, hkv);
+    return fail(RF_EUNSUPPORTED, "%s: head_dim %d, %d query heads over %d K / V heads (d 64, 128 or 256; a group of 1, "
+                "2, 4 or 8, or up to 16 at d 256)", fn, d, hq, hkv);
+  return RF_OK;
+}
+
+extern "C" int rf_attend_causal_workspace_bytes(int64_t nq, int hq, int hkv, int d, int64_t n_keys, size_t* bytes) {
+  if (int rc = causal_size("rf_attend_causal_workspace_bytes", nq, hq, hkv, d, n_keys, bytes)) return rc;
   // for queries anywhere and for the last nq keys' own
   const int ns = std::max(causal_plan(nq, hq, hkv, d, n_keys, true, 0).ns,
                           causal_plan(nq, hq, hkv, d, n_keys, false, std::max<int64_t>(0, n_keys - nq)).ns);
   *bytes = part_bytes(nq, hq, hkv, d, ns);
+  return RF_OK;
+}
+
+extern "C" int rf_attend_causal_workspace_bytes_at(int64_t nq, int hq, int hkv, int d, int64_t n_keys, int scattered,
+                                                   int64_t slot0, size_t* bytes) {
+  const char* fn = "rf_attend_causal_workspace_bytes_at";
+  if (int rc = causal_size(fn, nq, hq, hkv, d, n_keys, bytes)) return rc;
+  if (!scattered && (slot0 < 0 || slot0 + nq > n_keys))
+    return fail(RF_EINVAL_SHAPE, "%s: queries at slots [%lld, %lld) past the %lld keys", fn, (long long)slot0,
+                (long long)(slot0 + nq), (long long)n_keys);
+  *bytes = part_bytes(nq, hq, hkv, d, causal_plan(nq, hq, hkv, d, n_keys, scattered != 0, scattered ? 0 : slot0).ns);
   return RF_OK;
 }
 

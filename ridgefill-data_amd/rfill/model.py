@@ -546,7 +546,7 @@ class FillModel:
         self.commit(c, T)
         if self._causal_ok():
             o = ops.attend_causal(q, slot, c["kbuf"], c["vbuf"], c["n"], self.n_heads, self.scale,
-                                  workspace=self._causal_workspace(T, c["n"], h.device))
+                                  workspace=self._causal_workspace(T, c["n"], h.device, slot))
         else:
             o = ops.attend_rows(q, torch.arange(slot, slot + T, device=h.device), c["kbuf"], c["vbuf"], c["n"],
                                 self.n_heads, self.scale, workspace=self._attn_workspace(T, c["n"], h.device))
@@ -586,12 +586,13 @@ class FillModel:
             hook("final", h)
         return (self.logits(h[torch.as_tensor(keep, device=self.device)]) if keep is not None else None), cache
 
-    def _causal_workspace(self, nq, n, device):
-        """rf_attend_causal's workspace (the key-range splits' partials), shared by every layer
-        (stream-ordered reuse)."""
-        need = ops.attend_causal_workspace_bytes(nq, self.n_heads, self.n_kv, self.head_dim, n)
+    def _causal_workspace(self, nq, n, device, slot0=None):
+        """rf_attend_causal's workspace (the key-range splits' partials) for nq queries from slot0 on, or scattered
+        ones, shared by every layer (stream-ordered reuse)."""
+        need = ops.attend_causal_workspace_bytes(nq, self.n_heads, self.n_kv, self.head_dim, n, slot0, slot0 is None)
         ws = getattr(self, "_causal_ws", None)
         if ws is None or ws.numel() < need or ws.device != device:
+            self._causal_ws = ws = None                 # (the old one back before the larger one is taken)
             self._causal_ws = ws = torch.empty(need, dtype=torch.uint8, device=device)
         return ws
 

@@ -573,10 +573,15 @@ CAUSAL_GROUPS_256 = (1, 2, 4, 8, 16)    # and at head_dim 256
 
 
 @_size_rule
-def attend_causal_workspace_bytes(nq, hq, hkv, d, n):
-    """Device bytes attend_causal uses for nq queries over n keys (the key-range splits' partials; may be 0)."""
+def attend_causal_workspace_bytes(nq, hq, hkv, d, n, slot0=None, scattered=False):
+    """Device bytes attend_causal uses for nq queries over n keys (the key-range splits' partials; may be 0): for
+    queries from slot0 on, for scattered ones, or without either the larger of the last nq keys' and scattered ones'."""
     b = ctypes.c_size_t(0)
-    _lib.call("rf_attend_causal_workspace_bytes", nq, hq, hkv, d, n, ctypes.byref(b))
+    if slot0 is None and not scattered:
+        _lib.call("rf_attend_causal_workspace_bytes", nq, hq, hkv, d, n, ctypes.byref(b))
+    else:
+        _lib.call("rf_attend_causal_workspace_bytes_at", nq, hq, hkv, d, n, int(scattered), 0 if scattered else slot0,
+                  ctypes.byref(b))
     return b.value
 
 
@@ -602,7 +607,9 @@ def attend_causal(q, slot0, kbuf, vbuf, n, hq, scale, out=None, workspace=None, 
     out = torch.empty(nq, hq * d, dtype=torch.bfloat16, device=q.device) if out is None else out
     _need(out, "out", torch.bfloat16, 2)
     if workspace is None:
-        workspace = torch.empty(attend_causal_workspace_bytes(nq, hq, hkv, d, n), dtype=torch.uint8, device=q.device)
+        need = (attend_causal_workspace_bytes(nq, hq, hkv, d, n, scattered=True) if qpos is not None else
+                attend_causal_workspace_bytes(nq, hq, hkv, d, n, int(slot0)))
+        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     _need(workspace, "workspace", torch.uint8, 1)
     if workspace.numel() == 0:
         workspace = None

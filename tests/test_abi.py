@@ -123,3 +123,42 @@ def test_gram_upper_workspace_sizes():
     assert ridge.gram_upper_workspace_bytes(0, 4096, 65536, 8192) == 0
     with pytest.raises(ValueError):
         ridge.gram_upper_workspace_bytes(4352, 4096, 65536, 8192)           # M past N
+
+
+def test_attention_workspace_by_kind_of_query():
+    """Host-only size rule of rf_attend_causal's key-range splits, told which queries it serves: a 4096-row tail of a
+    32K prompt runs unsplit and asks for nothing, though as many scattered queries are split (whole key ranges of
+    256-row blocks: 130 or 258 fp32 values a row and split); without the kind it is the larger of the two."""
+    from rfill import ops
+    for hq, hkv, d in ((32, 8, 128), (16, 2, 256)):
+        nq, n = 4096, 32768
+        tail = ops.attend_causal_workspace_bytes(nq, hq, hkv, d, n, n - nq)
+        rows = ops.attend_causal_workspace_bytes(nq, hq, hkv, d, n, scattered=True)
+        assert tail == 0 and rows % (nq * hq * (d + 2) * 4) == 0
+        assert ops.attend_causal_workspace_bytes(nq, hq, hkv, d, n) == max(tail, rows)
+    few = ops.attend_causal_workspace_bytes(37, 32, 8, 128, 3038, 3001)
+    assert few > 0 and few % (64 * 32 * 130 * 4) == 0
+    with pytest.raises(ValueError):
+        ops.attend_causal_workspace_bytes(100, 32, 8, 128, 3038, 2939)      # slots past the keys
+
+
+def test_model_attention_workspace_follows_the_call(monkeypatch):
+    """FillModel keeps no workspace for a tail that runs unsplit, and gives a smaller buffer back before it takes a
+    larger one."""
+    import torch
+    from rfill import model as M
+    m = M.FillModel.__new__(M.FillModel)
+    m.n_heads, m.n_kv, m.head_dim = 32, 8, 128
+    kept = []
+
+    def empty(n, dtype, device):
+        kept.append(getattr(m, "_causal_ws", None))
+        return torch.zeros(1, dtype=dtype).expand(n)
+
+    cpu = torch.device("cpu")
+    monkeypatch.setattr(M.torch, "empty", empty)
+    assert m._causal_workspace(4096, 32768, cpu, 28672).numel() == 0
+    small = m._causal_workspace(37, 3038, cpu, 3001).numel()
+    assert m._causal_workspace(37, 3038, cpu, 3001).numel() == small > 0
+    assert m._causal_workspace(300, 28672, cpu).numel() > small
+    assert len(kept) == 3 and all(w is None for w in kept)
