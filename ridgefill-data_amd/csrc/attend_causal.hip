@@ -291,6 +291,17 @@ __device__ __forceinline__ void tile_step(const char* __restrict__ st, const cha
   }
 }
 
+// The key split that the at-th column of query blocks of a head block takes. With fewer than 8 head blocks several
+// XCDs share one: each takes every xcds-th of its splits (class by class), so that the splits past the early queries,
+// which end at once, are spread over them instead of idling the last.
+__host__ __device__ __forceinline__ int split_of(int at, int ns, int head_blocks) {
+  const int xcds = head_blocks < 8 ? 8 / head_blocks : 1;
+  if (xcds == 1 || ns <= xcds) return at;
+  const int per = ns / xcds, more = ns % xcds, cut = more * (per + 1);
+  const int cls = at < cut ? at / (per + 1) : more + (at - cut) / per;
+  return (at < cut ? at - cls * (per + 1) : (at - cut) - (cls - more) * per) * xcds + cls;
+}
+
 template <int AD>
 __global__ __launch_bounds__(Cfg<AD>::NTHR, 1) void k_attend_causal(CausalArgs a) {
   using L = Layout<AD>;
@@ -306,16 +317,7 @@ __global__ __launch_bounds__(Cfg<AD>::NTHR, 1) void k_attend_causal(CausalArgs a
   const int qbs = gridDim.x, ns = gridDim.z;
   const int u = xcd_tile(blockIdx.x + qbs * (blockIdx.y + gridDim.y * blockIdx.z), qbs * gridDim.y * ns);
   const int qb = u % qbs, hb = u / (qbs * ns);
-  // With fewer than 8 head blocks several XCDs share one: each takes every xcds-th of its splits (class by class),
-  // so that the splits past the early queries, which end at once, are spread over them instead of idling the last.
-  const int xcds = gridDim.y < 8 ? 8 / static_cast<int>(gridDim.y) : 1;
-  int sp = (u / qbs) % ns;
-  if (xcds > 1 && ns > xcds) {
-    const int per = ns / xcds, more = ns % xcds, cut = more * (per + 1);
-    const int cls = sp < cut ? sp / (per + 1) : more + (sp - cut) / per;
-    const int at = sp < cut ? sp - cls * (per + 1) : (sp - cut) - (cls - more) * per;
-    sp = at * xcds + cls;
-  }
+  const int sp = split_of((u / qbs) % ns, ns, static_cast<int>(gridDim.y));
   const int hk = hb / (rep / a.hpb), hoff = (hb % (rep / a.hpb)) * a.hpb;
   const int j0 = qb * qp;
   const int jlast = min(j0 + qp, a.nq) - 1;
@@ -569,57 +571,117 @@ size_t part_bytes(int64_t nq, int hq, int hkv, int d, int splits) {
                     : 0;
 }
 
-// Key-range splits {ns, W}: W key tiles per split block, ns = ceil(key tiles / W) splits, at most 64. The plan
-// takes the ns of the least estimated time. A block alone takes t us a key tile; all of them together run at
-// most R tiles a us (the chip's power limit: beyond about 200 live blocks more of them only slow each other
-// down, also the second block a CU holds at d 64), so a round of B <= 256 live blocks takes W max(t, B / R) and
-// 6 us to start and end; the splits write and read their partials (b us a block) and add the combine launch.
-// Live blocks of query block qb: ceil(ntiles_qb / W) per head block, ntiles_qb exact for consecutive queries
-// (qpos null), else from query positions spread evenly over the keys (the exact rows; a round then counts as
-// 0.85 of the CUs). Fitted to 16 .. 2500 queries over 3000 .. 28672 keys (32 / 8 heads at d 128, 16 / 2 at d
-// 256), 1 to 64 splits; against the rule before it (rounds of 208 blocks, W + 2 tiles each, none from 256 query
-// blocks up), over 28672 keys, consecutive queries (us): d 128, 1021 queries 481 -> 422, 1499 801 -> 684, 2500
-// 1453 -> 1071; d 256, 700 445 -> 357, 1499 914 -> 726, 2500 1411 -> 1152; scattered at d 256: 300 230 -> 145,
-// 1021 513 -> 420 (with the XCDs' interleaved splits). Only the time depends on these estimates, not the
-// results.
+// Key-range splits {ns, W}: W key tiles per split block, ns = ceil(key tiles / W) splits, at most 64: the ns of the
+// least estimated time. The blocks run as the kernel maps them, each XCD an eighth of them in order on 32 CUs, and cost
+// the key tiles they run: a block ends at its last query's tile, so a prompt from slot 0 runs about half of its queries
+// x keys, and a split past an early query nothing. Tiles of query block qb: exact for consecutive queries (qpos null),
+// else for positions spread evenly over the keys (real ones are uneven: 0.85 to 0.92 of the CUs are counted then).
+// A block alone takes t us a key tile, all of them together run at most R tiles a us (beyond that more blocks only slow
+// each other down, also the second one a CU holds at d 64), a block takes 6 us to start and end. Live blocks that fit
+// an XCD's CUs take as long as the longest of them; more of them go in rounds if they are of one length, and fill each
+// other's gaps if they are not: all tiles at the full rate, and 0.3 of the longest block for the uneven end; between the
+// two by how far the lengths differ. Splits write and read their partials (b us a block) and add the merge launch; they
+// are taken where they gain 4 %.
+// Fitted to 16 .. 6000 queries behind 3000 .. 28672 keys, scattered ones, and prompts of 700 .. 16384 from slot 0 (32 /
+// 8 heads at d 64 and 128, 16 / 2 at d 256, 4 / 2 at d 64, 8 / 1 at d 128) at 1 to 64 splits: the choice takes 1.4 %
+// more than the best count on average. Two rules it is better than (us): each block at the W tiles that its split may
+// have, which is the same for tails behind a long prefix, split prompts from slot 0 three ways (d 128, 32 / 8 heads,
+// 4096 rows 200, now 171; 8192 634, now 572; d 256, 4096 306, now 249); rounds of 208 blocks of W + 2 tiles, none from
+// 256 query blocks on: over 28672 keys d 128, 1021 queries 481 -> 422, 2500 1453 -> 1071; d 256, 1499 914 -> 717,
+// scattered 1021 557 -> 350. Only the time depends on these estimates, not the results.
 struct Splits {
   int ns, W;
 };
 
 constexpr size_t PART_MAX = 512u << 20;    // bytes of partials that a plan may ask for
+constexpr int PLAN_BLOCKS = 2048;          // from this many query blocks (x head blocks) on, unsplit
+
+// Tiles of the query blocks, and what part of the blocks runs under a split.
+struct PlanBlocks {
+  int QB;
+  int tiles[PLAN_BLOCKS];                  // of query block qb, not falling
+  int64_t sum[PLAN_BLOCKS + 1];            // of the query blocks before qb
+};
+
+struct PlanLoad {
+  int64_t live = 0, work = 0;              // blocks that run, their tiles
+  int longest = 0;
+};
 
 Splits causal_plan(int64_t nq, int hq, int hkv, int d, int64_t n_keys, bool scattered, int64_t slot0) {
-  const int64_t T = key_tiles(n_keys, d), QB = query_blocks(nq, hq, hkv, d), qp = queries_per_block(hq, hkv, d);
-  const int64_t HB = head_blocks(hq, hkv, d), KT = kt_of(d), slots = 256;
-  if (T <= 1 || QB * HB >= 8 * slots) return Splits{1, static_cast<int>(std::max<int64_t>(T, 1))};
+  const int64_t T = key_tiles(n_keys, d), qp = queries_per_block(hq, hkv, d), KT = kt_of(d);
+  const int64_t HB = head_blocks(hq, hkv, d);
+  if (T <= 1 || nq <= 0 || query_blocks(nq, hq, hkv, d) * HB >= PLAN_BLOCKS)
+    return Splits{1, static_cast<int>(std::max<int64_t>(T, 1))};
   const double t = d == 256 ? 1.7 : d == 128 ? 1.45 : 1.24, R = d == 256 ? 124 : d == 128 ? 135 : 190;
-  const double b = d == 256 ? 0.06 : d == 128 ? 0.03 : 0.015, cap = scattered ? 0.85 * slots : slots;
-  auto tiles_of = [&](int64_t qb) {
-    if (scattered) return std::max<int64_t>(1, (T * (qb + 1) + QB - 1) / QB);
-    const int64_t last = slot0 + std::min<int64_t>((qb + 1) * qp, nq) - 1;
-    return std::min<int64_t>(T, last / KT + 1);
-  };
+  const double b = d == 256 ? 0.06 : d == 128 ? 0.03 : 0.015, start = 6;
+  const double slots = 32 * (!scattered ? 1.0 : d == 64 ? 0.85 : 0.92), t_full = std::max(t, 256 / R);
+  PlanBlocks pb;
+  const int QB = pb.QB = static_cast<int>(query_blocks(nq, hq, hkv, d));
+  pb.sum[0] = 0;
+  for (int qb = 0; qb < QB; ++qb) {
+    const int64_t n = scattered ? std::max<int64_t>(1, (T * (qb + 1) + QB - 1) / QB)
+                                : std::min<int64_t>(T, (slot0 + std::min<int64_t>((qb + 1) * qp, nq) - 1) / KT + 1);
+    pb.tiles[qb] = static_cast<int>(n);
+    pb.sum[qb + 1] = pb.sum[qb] + n;
+  }
   Splits best{1, static_cast<int>(T)};
   double best_us = 0;
-  for (int64_t ns = 1, W = T + 1; ns <= 64; ++ns) {
-    if ((T + ns - 1) / ns == W) continue;
-    W = (T + ns - 1) / ns;
-    if (ns > 1 && (W < 2 || part_bytes(nq, hq, hkv, d, static_cast<int>((T + W - 1) / W)) > PART_MAX)) break;
-    int64_t live = 0;
-    for (int64_t qb = 0; qb < QB; ++qb) live += (tiles_of(qb) + W - 1) / W;
-    live *= HB;
-    const int64_t real = (T + W - 1) / W;
-    if (HB < 8 && real % (8 / HB)) {              // the XCDs' shares of the splits are unequal
-      if (scattered && ns > 1) continue;
-      live = QB * HB * real;
+  int from[64], full[64], order[64];       // first query block that reaches split s, and that reaches past it
+  int64_t W = T + 1;
+  for (int64_t want = 1; want <= 64; want += want < 16 ? 1 : want < 32 ? 4 : 8) {
+    if ((T + want - 1) / want == W) continue;
+    W = (T + want - 1) / want;
+    const int ns = static_cast<int>((T + W - 1) / W);
+    if (ns > 1 && (W < 2 || part_bytes(nq, hq, hkv, d, ns) > PART_MAX)) break;
+    for (int s = 0, i = 0, j = 0; s < ns; ++s) {
+      while (i < QB && pb.tiles[i] <= s * W) ++i;
+      while (j < QB && pb.tiles[j] < (s + 1) * W) ++j;
+      from[s] = i;
+      full[s] = j;
+      order[s] = split_of(s, ns, static_cast<int>(HB));
     }
-    const double whole = static_cast<double>(static_cast<int64_t>(live / cap)), rest = live - whole * cap;
-    double us = whole * (W * std::max(t, slots / R) + 6);
-    if (rest > 0) us += W * std::max(t, rest / R) + 6;
-    if (ns > 1) us += live * b + 0.1 * ns + 6;
+    // an XCD's blocks: a run of whole and part columns (head block, split) of QB query blocks; one XCD for all of them
+    // where they are alike
+    const int64_t blocks = HB * ns * QB;
+    // (too few blocks for one to wait for another or slow it down: the longest is all that counts)
+    const bool few = blocks / 8 + 1 <= std::min(slots, t * R / 8);
+    const int xcds = few ? 0 : HB % 8 == 0 ? 1 : 8;
+    double us = few ? std::min<int64_t>(W, pb.tiles[QB - 1]) * t + start : 0;
+    int64_t live = 0;
+    for (int s = 0; few && s < ns; ++s) live += HB * (QB - from[s]);
+    int at = 0, lo = 0;                    // the next block: column at of its head block, query block lo
+    for (int x = 0; x < xcds; ++x) {
+      PlanLoad l;
+      for (int64_t left = blocks / 8 + (x < blocks % 8 ? 1 : 0); left > 0;) {
+        const int hi = static_cast<int>(std::min<int64_t>(QB, lo + left)), s = order[at];
+        const int f = std::min(std::max(lo, from[s]), hi), g = std::min(std::max(f, full[s]), hi);
+        left -= hi - lo;
+        lo = hi == QB ? 0 : hi;
+        if (lo == 0) at = at + 1 == ns ? 0 : at + 1;
+        if (f == hi) continue;
+        l.live += hi - f;
+        l.work += pb.sum[g] - pb.sum[f] - (g - f) * s * W + (hi - g) * W;
+        l.longest = std::max(l.longest, static_cast<int>(g < hi ? W : pb.tiles[hi - 1] - s * W));
+      }
+      live += l.live;
+      if (l.live == 0) continue;
+      const double n = static_cast<double>(l.live), whole = static_cast<double>(static_cast<int64_t>(n / slots));
+      const double rest = n - whole * slots;
+      double v = l.longest * std::max(t, n * 8 / R) + start;
+      if (n > slots) {
+        const double mean = l.work / n;
+        const double even = whole * (mean * t_full + start) + (rest > 0 ? l.longest * std::max(t, rest * 8 / R) + start : 0);
+        const double uneven = l.work / slots * t_full + start * (whole + 1) + 0.3 * l.longest * t;
+        v = even + (uneven - even) * std::min(1.0, 2 * (l.longest - mean) / mean);
+      }
+      us = std::max(us, v);
+    }
+    if (xcds == 1) live *= 8;
+    if (ns > 1) us = 1.04 * (us + live * b + 0.1 * ns + 6);
     if (ns == 1 || us < best_us) {
       best_us = us;
-      best = Splits{static_cast<int>((T + W - 1) / W), static_cast<int>(W)};
+      best = Splits{ns, static_cast<int>(W)};
     }
   }
   return best;

@@ -162,3 +162,16 @@ def test_model_attention_workspace_follows_the_call(monkeypatch):
     assert m._causal_workspace(37, 3038, cpu, 3001).numel() == small > 0
     assert m._causal_workspace(300, 28672, cpu).numel() > small
     assert len(kept) == 3 and all(w is None for w in kept)
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (32, 8, 64), (16, 2, 256)])
+def test_prompts_from_slot_0_are_not_split(hq, hkv, d):
+    """A prompt's own attention from slot 0: half its (queries x keys) is masked, so a block per query block keeps every
+    CU as busy as key splits would, without their partials; no workspace from 4096 rows on, as on a tail of as many rows
+    behind a prefix. Few queries behind a long prefix are split."""
+    from rfill import ops
+    for n in (4096, 8192, 12288, 16384):
+        assert ops.attend_causal_workspace_bytes(n, hq, hkv, d, n, 0) == 0, n
+    assert ops.attend_causal_workspace_bytes(4096, hq, hkv, d, 8192, 4096) == 0
+    assert ops.attend_causal_workspace_bytes(300, hq, hkv, d, 28672, 28372) > 0
+    assert ops.attend_causal_workspace_bytes(300, hq, hkv, d, 28672, scattered=True) > 0
