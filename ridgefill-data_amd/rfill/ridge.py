@@ -313,10 +313,15 @@ class RidgeStats:
             self._sq = torch.empty_like(self._part)
         return self._xt, self._yt, self._part
 
-    def _gram(self, a, ea, b, db, eb, c, block, upper=False, init=False):
-        """gram_centred of X^T (a: dim main and ea extra rows) with a workspace kept between calls."""
+    def _gram(self, a, ea, b, db, eb, c, block, upper=False):
+        """gram_centred of X^T (a: dim main and ea extra rows) into the sums c, with a workspace kept between calls;
+        returns c. c None: the first product, stored in new sums (the caller has them only once it was launched, so a
+        call that failed leaves none behind)."""
         need = gram_centred_workspace_bytes(self.dim, ea, db, eb, a.shape[1], block, upper)
-        gram_centred(a, self.dim, ea, b, db, eb, c, block, upper, init, self._workspace(need))
+        init = c is None
+        if init:
+            c = torch.empty(self.dim + ea, db + (LO_ROWS if eb else 0), dtype=torch.float64, device=self.device)
+        return gram_centred(a, self.dim, ea, b, db, eb, c, block, upper, init, self._workspace(need))
 
     def _workspace(self, need):
         ws = getattr(self, "_gws", None)
@@ -367,11 +372,7 @@ class RidgeStats:
             rows = self._x_piece(r, True)
             kp = (rows + 63) // 64 * 64
             xt, e = self._xt[:, :kp], 2 * cx.s
-            init = self.sxx is None                     # the first product is stored, not added to zeros
-            if init:
-                self.sxx = torch.empty(d + e, d + cx.lo_rows, dtype=torch.float64, device=self.device)
-                self._sxx_upper = True
-            self._gram(xt, e, xt, d, e, self.sxx, block, upper=True, init=init)
+            self.sxx = self._gram(xt, e, xt, d, e, self.sxx, block, upper=True)
 
     @torch.no_grad()
     def add_layer(self, i, y):
@@ -402,10 +403,7 @@ class RidgeStats:
             py = tiles_view(part, kp // 64, o)
             transpose_centred(y[r:r + rows], yt[:o, :kp], yt[o:, :kp], cy.shift, cy.lo_row, py, n_centred=cy.s)
             _colsum_fold(py, self.s1y[i])
-            init = i not in self.sxy
-            if init:
-                self.sxy[i] = torch.empty(d + 2 * cx.s, o + cy.lo_rows, dtype=torch.float64, device=self.device)
-            self._gram(xt[:, :kp], 2 * cx.s, yt[:, :kp], o, 2 * cy.s, self.sxy[i], block, init=init)
+            self.sxy[i] = self._gram(xt[:, :kp], 2 * cx.s, yt[:, :kp], o, 2 * cy.s, self.sxy.get(i), block)
 
     def add(self, x, ys, block=8192, w=None):
         """x [n, d] and ys {layer: [n, d_out]}: bf16 rows on the GPU (the same rows, in order)
@@ -413,6 +411,12 @@ class RidgeStats:
         self.begin(x, block, w)
         for i in self.layers:
             self.add_layer(i, ys[i])
+
+    def _sums(self, c, cols, cen=None):
+        """The sums c, or zeros if no product was added into them (the call that began them failed)."""
+        cen = self.cen_x if cen is None else cen
+        return torch.zeros(self.dim + 2 * self.cen_x.s, cols + 2 * cen.s, dtype=torch.float64,
+                           device=self.device) if c is None else c
 
     def state(self, device="cpu"):
         """RidgeStats.state() (code/kva/ridge.py:70-74): shifted sums about cx / cy, fp64."""
@@ -424,7 +428,7 @@ class RidgeStats:
         d, o, cx = self.dim, self.out_dim, self.cen_x
         dx = cx.delta
         # X^T X is accumulated on its block-upper tiles only
-        sxx = centred_state(self.sxx, d, cx, d, cx, self.s1x, self.s1x, n, upper=getattr(self, "_sxx_upper", False))
+        sxx = centred_state(self._sums(self.sxx, d), d, cx, d, cx, self.s1x, self.s1x, n, upper=True)
         cy, sy, sxy = {}, {}, {}
         for i in self.layers:
             if i not in self.cen_y:                 # no rows of this layer yet: zero sums, no shift (ridge.py:73)
@@ -436,7 +440,7 @@ class RidgeStats:
             c = self.cen_y[i]
             cy[i] = c.c
             sy[i] = self.s1y[i] - n * c.delta
-            sxy[i] = centred_state(self.sxy[i], d, cx, o, c, self.s1x, self.s1y[i], n)
+            sxy[i] = centred_state(self._sums(self.sxy.get(i), o, c), d, cx, o, c, self.s1x, self.s1y[i], n)
         mine = dict(split=self.split, layers=self.layers, dim=self.dim, n=self.n, cx=cx.c, cy=cy,
                     sx=self.s1x - n * dx, sxx=sxx, sy=sy, sxy=sxy)
         return _to(combine(self.base, mine, 1) if self.base is not None else mine, device)

@@ -4,6 +4,7 @@ operand rows, the augmented Gram products), combined and moved onto the referenc
 the reference's state -- with centring on and off, and when a saved state is resumed; residual / combine agree
 with the oracle's. (The device accumulation and the solve, rf_ridge_solve, are tested on the GPU in
 test_gpu_fit.py and test_gpu_fit_c5.py.)"""
+import pytest
 import torch
 
 from oracle import ridge as oridge
@@ -140,3 +141,44 @@ def test_residual_and_combine_agree_with_the_oracle():
     assert torch.equal(mine["sxy"][7], ref["sxy"][7]) and mine["n"] == ref["n"]
     r1, r2 = ridge.residual(sa), oridge.residual(sa)
     assert torch.equal(r1["sxy"][7], r2["sxy"][7]) and torch.equal(r1["cy"][7], r2["cy"][7])
+
+
+def test_a_failed_first_product_leaves_no_sums_behind(monkeypatch):
+    """The first product of X^T X and of each X^T Y is stored into fresh (uninitialised) sums. If it fails (no memory
+    for its workspace), nothing of them stays: state() has zeros there, and the next call stores again."""
+    d, n = 256, 320
+    g = torch.Generator().manual_seed(8)
+    x, y = [torch.randn(n, d, generator=g).to(torch.bfloat16) for _ in range(2)]
+    fail = [True]
+
+    def transpose(x, dst, dst_lo, shift, lo_row, partial, partial_sq=None, n_centred=0):
+        dst.copy_(x.T)
+
+    def gram(a, da, ea, b, db, eb, c, fold_rows=0, upper=False, init=False, workspace=None):
+        if fail[0]:
+            c.fill_(float("nan"))                       # what the memory held
+            raise MemoryError
+        prod = a[:da].double() @ b[:db].double().T
+        c.copy_(prod if init else c + prod)
+        return c
+
+    monkeypatch.setattr(ridge, "_need", lambda *a: None)
+    monkeypatch.setattr(ridge, "transpose_centred", transpose)
+    monkeypatch.setattr(ridge, "_colsum_fold", lambda partial, sums: None)
+    monkeypatch.setattr(ridge, "gram_centred", gram)
+    monkeypatch.setattr(ridge.Centring, "of_rows", classmethod(lambda cls, r, *a: _centring(r, None, 0)))
+    st = ridge.RidgeStats(3, [7], d, device="cpu", centre_max=0)
+    with pytest.raises(MemoryError):
+        st.begin(x, block=64)
+    with pytest.raises(MemoryError):
+        st.add_layer(7, y)
+    st.cen_x.delta.zero_()                              # (the sums alone, about no shift)
+    st.cen_y[7].delta.zero_()
+    none = st.state()
+    assert not none["sxx"].any() and not none["sxy"][7].any()
+    fail[0] = False
+    for _ in range(2):
+        st.add(x, {7: y}, block=64)
+    got = st.state()
+    assert torch.equal(got["sxx"], 2 * (x.double().T @ x.double()))
+    assert torch.equal(got["sxy"][7], 2 * (x.double().T @ y.double()))
