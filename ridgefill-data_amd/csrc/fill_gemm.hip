@@ -500,10 +500,11 @@ __device__ __forceinline__ void split_sums(const float* __restrict__ part, int s
 }
 
 // Sum of a row's nparts statistics partials q, in order. Up to 16 partials, a multiple of 4 (H 1024 .. 4096 and
-// H % 1024 == 0): all loaded before the first is added (loads past the end repeat the last).
+// H % 1024 == 0) and 16-byte aligned (no caller has to see to that): all loaded before the first is added (loads past
+// the end repeat the last).
 __device__ __forceinline__ float parts_total(const float* __restrict__ q, int nparts) {
   float s = 0.f;
-  if (nparts % 4 == 0 && nparts <= 16) {            // uniform
+  if (nparts % 4 == 0 && nparts <= 16 && (reinterpret_cast<uintptr_t>(q) & 15u) == 0) {     // the same for every row
     float4 v[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const float4*>(q + 4 * min(k, nparts / 4 - 1));

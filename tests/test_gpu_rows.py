@@ -522,3 +522,32 @@ def test_last_tile_rows_as_few_rows(dev, M):
     for a, b in pairs:
         assert torch.equal(a[:1280], b[:1280])
         assert rel_err(a[1280:], b[1280:]) < 5e-3
+
+
+@pytest.mark.parametrize("H", [1024, 1280, 4096])
+def test_row_statistics_at_any_alignment(dev, H):
+    """The row statistics need no more than a float's alignment: results with them 4, 8 and 12 bytes past a 16-byte
+    boundary are bit for bit those with aligned ones, in every epilogue of the few-rows products."""
+    from rfill import ops
+    R, hq, hkv, d, slot = 33, 4, 2, 128, 5
+    g = torch.Generator(device=dev).manual_seed(H)
+    x = torch.randn(R, H, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(2 * (hq + 2 * hkv) * d, H, generator=g, device=dev) / H ** 0.5).to(torch.bfloat16)
+    cs = ops.rope_table(torch.arange(slot, slot + R, device=dev), ops.inv_freq_default(1e6, d).to(dev))
+    ssq = ops.row_ssq(x)
+    n = (hq + 2 * hkv) * d
+
+    def run(s):
+        kb, vb = (torch.zeros(hkv, R + slot, d, dtype=torch.bfloat16, device=dev) for _ in range(2))
+        q, _ = ops.norm_attn_rows(x, s, 1e-6, w[:n], hq, hkv, d, None, None, 0, cs, kb, vb, slot)
+        return [q, kb, vb, ops.norm_linear(x, s, 1e-6, w, workspace="auto"),
+                ops.norm_linear_swiglu(x, s, 1e-6, w, workspace="auto")]
+
+    want = run(ssq)
+    for off in (1, 2, 3):
+        buf = torch.empty(ssq.numel() + 4, dtype=torch.float32, device=dev)
+        s = buf[off:off + ssq.numel()].view(ssq.shape)
+        s.copy_(ssq)
+        assert s.data_ptr() % 16 == 4 * off
+        for a, b in zip(run(s), want):
+            assert torch.equal(a, b)
