@@ -70,6 +70,13 @@ def _colsum_fold(partial, sums):
     _lib.call("rf_colsum_fold", _ptr(partial), partial.shape[0], partial.shape[1], _ptr(sums), _stream(sums))
 
 
+def _vector(t, name, dtype, n, device):
+    """A vector of n values on `device` that a kernel reads or writes as they lie."""
+    _need(t, name, dtype, 1)
+    if t.numel() != n or t.device != device:
+        raise ValueError(f"{name}: {t.numel()} values on {t.device}, expected {n} on {device}")
+
+
 def gram_workspace_bytes(M, N, K, fold_rows=0):
     """Bytes of rf_gram_accumulate's run-split workspace for this shape (0: it uses none)."""
     nb = ctypes.c_size_t(0)
@@ -156,6 +163,10 @@ def gram_centred(a, da, ea, b, db, eb, c, fold_rows=0, upper=False, init=False, 
     if b.shape[1] != K or a.shape[0] < da + ea or b.shape[0] < db + eb or c.shape[0] < da + ea or c.shape[1] < db + eb:
         raise ValueError(f"gram_centred shapes a {tuple(a.shape)}, b {tuple(b.shape)}, c {tuple(c.shape)} for "
                          f"{da} + {ea} by {db} + {eb} rows")
+    if workspace is not None:
+        _need(workspace, "workspace", torch.uint8, 1)
+    if any(t.device != a.device for t in (b, c, workspace) if t is not None):
+        raise ValueError("gram_centred: operands on several devices")
     need = gram_centred_workspace_bytes(da, ea, db, eb, K, fold_rows, upper)
     if need and (workspace is None or workspace.numel() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=c.device)
@@ -197,6 +208,9 @@ class Centring:
         """The same choice on the GPU in one launch (rf_centre_select); the count is read back once."""
         cols, dev = s1.numel(), s1.device
         cap = max(0, min(cap, cols))
+        s1, s2 = s1.to(torch.float64).contiguous(), s2.to(torch.float64).contiguous()
+        for name, t in (("s1", s1), ("s2", s2)) + ((("c", c),) if c is not None else ()):
+            _vector(t, name, torch.float64, cols, dev)
         f64 = torch.empty(3, cols, dtype=torch.float64, device=dev)
         self.c, self.delta, scratch = f64
         self.shift = torch.empty(cols, dtype=torch.float32, device=dev)
@@ -213,6 +227,11 @@ class Centring:
     @classmethod
     def of_rows(cls, x, part, part_sq, c=None, cap=SHIFT_MAX):
         """The centring chosen from rows x [n, cols] (part / part_sq: room for their per-64-row sums)."""
+        for name, t in (("part", part), ("part_sq", part_sq)):
+            _need(t, name, torch.float32)
+            if t.device != x.device:
+                raise ValueError(f"{name}: on {t.device}, x on {x.device}")
+        _need(x, "x", torch.bfloat16, 2)
         n, cols = x.shape
         tiles = (n + 63) // 64
         s1, s2 = torch.zeros(2, cols, dtype=torch.float64, device=x.device)
@@ -257,8 +276,14 @@ def centred_state(G, ca, A, cb, B, s1a, s1b, n, upper=False):
     if not G.is_cuda:
         return recentre(centred_products(mirror_block_upper(G) if upper else G, ca, A, cb, B), s1a, s1b, A.delta,
                         B.delta, n)
-    if G.stride(1) != 1:
-        raise ValueError("centred_state: G must be row-major")
+    _need(G, "G", torch.float64, 2)
+    if G.shape[0] < ca + 2 * A.s or G.shape[1] < cb + 2 * B.s or (upper and A is not B):
+        raise ValueError(f"centred_state: G {tuple(G.shape)} for {ca} + 2 x {A.s} by {cb} + 2 x {B.s} rows"
+                         + (", upper needs one operand" if upper else ""))
+    for name, t, dtype, k in (("s1a", s1a, torch.float64, ca), ("s1b", s1b, torch.float64, cb),
+                              ("A.delta", A.delta, torch.float64, ca), ("B.delta", B.delta, torch.float64, cb),
+                              ("A.lo_row", A.lo_row, torch.int32, ca), ("B.lo_row", B.lo_row, torch.int32, cb)):
+        _vector(t, name, dtype, k, G.device)
     out = torch.empty(ca, cb, dtype=torch.float64, device=G.device)
     _lib.call("rf_gram_state", _ptr(G), G.stride(0), ca, A.s, _ptr(A.lo_row), cb, B.s, _ptr(B.lo_row), int(upper),
               _ptr(s1a), _ptr(s1b), _ptr(A.delta), _ptr(B.delta), float(n), _ptr(out), out.stride(0), _stream(G))

@@ -327,3 +327,35 @@ def test_centring_and_state_on_the_gpu_match_the_host_path(dev, cols, cap, given
         out = ridge.centred_state(dG, ca, Ag, cols, got, s1a.to(dev), s1b.to(dev), float(n), upper)
         big = n * float((A.delta.abs().max() * want.delta.abs().max())) + 10
         assert float((out.cpu() - ref).abs().max()) < 1e-14 * big * 8, (upper, float((out.cpu() - ref).abs().max()))
+
+
+def test_gram_and_state_refuse_what_the_kernels_do_not_check(dev):
+    """Operands whose type, size or device the kernels take on trust: refused before a launch."""
+    from rfill import ridge
+    f64, d = torch.float64, 256
+    a = torch.zeros(d + 8, 128, dtype=torch.bfloat16, device=dev)
+    c = torch.zeros(d + 4, d + 8, dtype=f64, device=dev)
+    for ws in (torch.empty(1 << 20, dtype=torch.float32, device=dev), torch.empty(1 << 20, dtype=torch.uint8)):
+        with pytest.raises(ValueError):
+            ridge.gram_centred(a, d, 4, a, d, 4, c, workspace=ws)
+    sums = torch.full((d,), 100.0, dtype=f64, device=dev)
+    sums[3] = 10000.0
+    A = ridge.Centring(sums, sums * 120, 100, None, 2)
+    cpu = ridge.Centring(sums.cpu(), sums.cpu() * 120, 100, None, 2)
+    assert A.s == cpu.s == 1
+    G = torch.zeros(d + 2, d + 2, dtype=f64, device=dev)
+    assert ridge.centred_state(G, d, A, d, A, sums, sums, 100, True).shape == (d, d)
+    for bad in ((G[:d + 1], A, sums, sums), (G[:, :d + 1], A, sums, sums), (G.float(), A, sums, sums),
+                (G, cpu, sums, sums), (G, A, sums[:-1], sums), (G, A, sums, sums.float()), (G, A, sums.cpu(), sums)):
+        g, op, s1a, s1b = bad
+        with pytest.raises(ValueError):
+            ridge.centred_state(g, d, op, d, op, s1a, s1b, 100)
+    with pytest.raises(ValueError):
+        ridge.Centring(sums, sums[1:], 100)
+    with pytest.raises(ValueError):
+        ridge.Centring(sums, sums, 100, torch.zeros(1, dtype=f64))
+    # sums in another type or stride are read as the values they are
+    wide = torch.stack((sums, sums * 120)).t().contiguous()
+    B = ridge.Centring(wide[:, 0], wide[:, 1].float(), 100, None, 2)
+    for name in ("c", "shift", "lo_row", "idx", "delta"):
+        assert torch.equal(getattr(A, name), getattr(B, name))
