@@ -593,7 +593,7 @@ extern "C" int rf_ridge_solve_wt(const double* cxx, int64_t ldc, int64_t d, cons
                                  size_t ws_bytes, hipStream_t stream) {
   const char* fn = "rf_ridge_solve_wt";
   if (!wt) return fail(RF_EINVAL_ARG, "%s: null pointer", fn);
-  if (targets <= 0 || width <= 0 || width % 2 || width * targets > (1ll << 30) || width > (1ll << 24))
+  if (targets <= 0 || width <= 0 || width % 2 || width > (1ll << 24) || width * targets > (1ll << 30))
     return fail(RF_EINVAL_SHAPE, "%s: %d targets of width %lld (even)", fn, targets, (long long)width);
   for (int j = 0; j < targets; ++j)
     if (!wt[j]) return fail(RF_EINVAL_ARG, "%s: null pointer for target %d", fn, j);
