@@ -141,9 +141,11 @@ __global__ __launch_bounds__(256) void k_colsum_fold(const float* __restrict__ p
 // rounded to fp32, or `given`), the channels with c^2 > variance (at most cap of them, largest c^2 / variance
 // first, lower index first among equals) with their fp32 shift, their row among the centred channels in
 // channel order, and what is left of c for the others. One block: thread t takes the per = ceil(cols / 1024)
-// channels from t * per on, so a block scan of the threads' counts gives the channel order; when more than cap
-// channels qualify, each one's rank is counted against every ratio, staged 1024 at a time in LDS. It takes 16 us
-// at 4096 channels and replaces about twenty launches of sorts and index operations (their gaps: 150 us).
+// channels from t * per on, so a block scan of the threads' counts gives the channel order. When more than cap
+// channels qualify, the cap-th largest ratio is found digit by digit (a positive double's bits order as its value):
+// eight passes over the ratios with a 256-bin histogram each; its equals are taken in channel order. At 4096
+// channels it takes 13 us with at most cap qualifying and 29 with more (each ratio counted against every other: 1300),
+// at 16384 72 and 117 (20 ms), and replaces about twenty launches of sorts and index operations (180 us, mostly gaps).
 constexpr int SEL_THREADS = 1024;
 struct CentreArgs {
   const double *s1, *s2, *given;
@@ -157,14 +159,33 @@ struct CentreArgs {
   int* count;
   double* ratio;          // [cols] scratch: c^2 / variance of a qualifying channel, else -1
 };
+
+// Sum over the block's threads of the values of the threads before this one; the whole sum in *total.
+__device__ __forceinline__ int block_before(int mine, int (&scan)[SEL_THREADS], int* total) {
+  const int t = threadIdx.x;
+  __syncthreads();                                  // scan's last use
+  scan[t] = mine;
+  __syncthreads();
+  for (int h = 1; h < SEL_THREADS; h <<= 1) {
+    const int v = t >= h ? scan[t - h] : 0;
+    __syncthreads();
+    scan[t] += v;
+    __syncthreads();
+  }
+  *total = scan[SEL_THREADS - 1];
+  return scan[t] - mine;
+}
+
 __global__ __launch_bounds__(SEL_THREADS) void k_centre_select(CentreArgs a) {
 #pragma clang fp contract(off)
-  __shared__ double stage[SEL_THREADS];
   __shared__ int scan[SEL_THREADS];
+  __shared__ int hist[256];
+  __shared__ int pick[2];
   const int t = threadIdx.x, per = (a.cols + SEL_THREADS - 1) / SEL_THREADS;
-  const int lo = min(t * per, a.cols), hi = min(lo + per, a.cols);
+  const int lo = static_cast<int>(min(static_cast<int64_t>(t) * per, static_cast<int64_t>(a.cols)));
+  const int hi = min(lo + per, a.cols);
   int mine = 0;
-  for (int k = lo; k < hi; ++k) {
+  for (int k = t; k < a.cols; k += SEL_THREADS) {   // (any order serves here and for the histograms)
     const double mean = a.s1[k] / a.n;
     double var = a.s2[k] / a.n - mean * mean;
     var = var < 0.0 ? 0.0 : var;                    // (a NaN stays one and qualifies nothing)
@@ -175,51 +196,73 @@ __global__ __launch_bounds__(SEL_THREADS) void k_centre_select(CentreArgs a) {
     a.ratio[k] = big ? c2 / fmax(var, 1e-300) : -1.0;
     mine += big ? 1 : 0;
   }
-  scan[t] = mine;
-  __syncthreads();
-  for (int h = SEL_THREADS / 2; h >= 1; h >>= 1) {
-    if (t < h) scan[t] += scan[t + h];
-    __syncthreads();
-  }
-  const int nbig = scan[0];
-  __syncthreads();
-  // selected channels of this thread: a.lo_row holds the rank until the row is known
-  for (int k = lo; k < hi; ++k) a.lo_row[k] = 0;
+  int nbig;
+  block_before(mine, scan, &nbig);
+  // the least ratio taken (as bits), and how many channels of exactly that ratio
+  uint64_t least = 0;
+  int ties = nbig;
   if (nbig > a.cap) {
-    for (int j0 = 0; j0 < a.cols; j0 += SEL_THREADS) {
+    int left = a.cap;                               // still to find at or below the digits known so far
+    uint64_t known = 0;
+    for (int sh = 56; sh >= 0 && left > 0; sh -= 8) {
+      if (t < 256) hist[t] = 0;
       __syncthreads();
-      stage[t] = j0 + t < a.cols ? a.ratio[j0 + t] : -1.0;
-      __syncthreads();
-      for (int k = lo; k < hi; ++k) {
+      for (int k = t; k < a.cols; k += SEL_THREADS) {
         const double r = a.ratio[k];
-        if (r < 0.0) continue;
-        int above = 0;
-        for (int j = 0; j < SEL_THREADS; ++j) above += (stage[j] > r || (stage[j] == r && j0 + j < k)) ? 1 : 0;
-        a.lo_row[k] += above;
+        const uint64_t u = static_cast<uint64_t>(__double_as_longlong(r));
+        if (r >= 0.0 && ((u ^ least) & known) == 0) atomicAdd(&hist[(u >> sh) & 255], 1);
       }
+      __syncthreads();
+      if (t < 64) {                                 // lane l: the bins 255 - 4 l .. 252 - 4 l, from the largest down
+        int n[4], sum = 0;
+        for (int i = 0; i < 4; ++i) sum += n[i] = hist[255 - 4 * t - i];
+        int above = sum;
+        for (int h = 1; h < 64; h <<= 1) {
+          const int v = __shfl_up(above, h, 64);
+          if (t >= h) above += v;
+        }
+        above -= sum;                               // channels in larger bins than this lane's
+        for (int i = 0; i < 4; ++i) {
+          if (above < left && left <= above + n[i]) {       // one bin of one lane
+            pick[0] = 255 - 4 * t - i;
+            pick[1] = left - above;
+          }
+          above += n[i];
+        }
+      }
+      __syncthreads();
+      least |= static_cast<uint64_t>(pick[0]) << sh;
+      known |= 255ull << sh;
+      left = pick[1];
+      __syncthreads();                              // (pick and hist are written again)
     }
+    ties = left;
   }
+  // in reach of the count: larger ratios all, of the equals the first `ties` in channel order
+  auto bits = [&](int k) { return static_cast<uint64_t>(__double_as_longlong(a.ratio[k])); };
+  const bool ranked = nbig > a.cap;
+  int equal = 0, total;
+  for (int k = lo; k < hi; ++k) equal += ranked && a.ratio[k] >= 0.0 && bits(k) == least ? 1 : 0;
+  const int before = block_before(equal, scan, &total);
+  auto taken = [&](int k, int& eq) {
+    if (!(a.ratio[k] >= 0.0) || (ranked && a.cap == 0)) return false;
+    if (!ranked || bits(k) > least) return true;
+    return bits(k) == least && eq++ < ties;
+  };
+  int eq = before;
   mine = 0;
-  for (int k = lo; k < hi; ++k) mine += (a.ratio[k] >= 0.0 && a.lo_row[k] < a.cap) ? 1 : 0;
-  __syncthreads();
-  scan[t] = mine;
-  __syncthreads();
-  for (int h = 1; h < SEL_THREADS; h <<= 1) {       // inclusive scan
-    const int v = t >= h ? scan[t - h] : 0;
-    __syncthreads();
-    scan[t] += v;
-    __syncthreads();
-  }
-  int row = scan[t] - mine;
+  for (int k = lo; k < hi; ++k) mine += taken(k, eq) ? 1 : 0;
+  int row = block_before(mine, scan, &total);
+  eq = before;
   for (int k = lo; k < hi; ++k) {
-    const bool sel = a.ratio[k] >= 0.0 && a.lo_row[k] < a.cap;
+    const bool sel = taken(k, eq);
     const float sh = sel ? static_cast<float>(a.c[k]) : 0.f;
     a.shift[k] = sh;
     a.delta[k] = a.c[k] - static_cast<double>(sh);
     a.lo_row[k] = sel ? row : -1;
     if (sel) a.idx[row++] = k;
   }
-  if (t == SEL_THREADS - 1) *a.count = scan[t];
+  if (t == 0) *a.count = total;
 }
 
 // One product of the fit's state from its augmented Gram G: D[r, c] = the sum of the parts of the centred
