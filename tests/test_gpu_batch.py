@@ -2,10 +2,11 @@
 K / V fills of several late layers in one launch each, on persistent tiles) and of fill_late's grouped
 schedule.
 
-Bar: bitwise. Every layer's x, row statistics and K / V cache equal the per-layer launches' without a
-split-K workspace (the same tiles, the same MFMA order, the same epilogue arithmetic); cache slots outside
-the written rows keep their contents. The per-layer launches themselves are pinned to the oracle in
-test_gpu_fill.py."""
+Bar: bitwise for launches without a workspace and for rows in whole rounds of tiles. Every layer's x, row
+statistics and K / V cache equal the per-layer launches' without a split-K workspace (the same tiles, the same
+MFMA order, the same epilogue arithmetic); cache slots outside the written rows keep their contents. Rows left
+over by whole rounds, which a workspace lets run as products of few rows with K split, are held to the rounding of
+one bf16 value. The per-layer launches themselves are pinned to the oracle in test_gpu_fill.py."""
 import pytest
 import torch
 
@@ -150,7 +151,8 @@ def test_batch_c2_shape(dev):
 
 def test_fill_late_groups_equal_per_layer(dev):
     """fill_late's grouped schedule (ATTN_GROUP attention layers per map launch and K / V launch) gives every
-    layer the caches of per-layer unsplit launches, bitwise, with given exact-row inputs scattered in."""
+    layer the caches of per-layer unsplit launches, bitwise, with given exact-row inputs scattered in (a width of
+    512: the rows' sums are never split)."""
     from rfill import ops
     from rfill.kva import ATTN_GROUP, Arm, Projector, fill_late
     from rfill.model import FillModel
@@ -188,7 +190,7 @@ def test_fill_late_hybrid_groups_equal_per_layer(dev):
     """A hybrid late stack (GDN, GDN, GDN, attention, GDN, GDN) at width 1024 filled by fill_late's grouped
     schedule (one map launch per group, paired GDN fills with one in-projection launch, batched attention
     fills) against per-layer unsplit launches: every GDN conv and recurrent state and the attention layer's K
-    / V bitwise equal."""
+    / V bitwise equal (2500 rows: no launch leaves rows over)."""
     from fill_cases import hybrid_config, hybrid_tensors
     from rfill import ops
     from rfill.kva import Arm, Projector, fill_late
@@ -302,3 +304,109 @@ def test_batch_rows_left_over(dev, name, P):
         assert torch.allclose(a, r, rtol=2e-2)          # sums of 256 squares of bf16 values, each within 2^-8
     for a in got[2] + got[3]:
         assert bool((a[:, :slot0] == -7).all()) and bool((a[:, slot0 + P:] == -7).all())
+
+
+def _near(a, r):
+    """One bf16 rounding apart, of the few values whose sums' order changed (test_batch_rows_left_over's bar)."""
+    a, r = a.float(), r.float()
+    assert float((a - r).norm()) <= 1e-3 * float(r.norm())
+    assert bool(((a - r).abs() <= 2.0 ** -7 * r.abs().amax(-1, keepdim=True)).all())
+
+
+def test_fill_late_with_rows_left_over(dev):
+    """fill_late at a width and prompt whose launches leave rows over (33 tile rows, the last of 20 rows: K split two
+    ways, the split count following the layers in the launch), in a group of four layers and one of two that share the
+    call's workspace, against per-layer unsplit launches: rows of the whole rounds bitwise, the rest to one rounding."""
+    from rfill import ops
+    from rfill.kva import Arm, Projector, fill_late
+    from rfill.model import FillModel
+    L, split, tail = 8, 2, 100
+    whole = 32 * 256
+    P = whole + 20
+    cfg, t = _case("w1024_qwen3_knorm", L)
+    H, hkv, d = cfg["hidden_size"], cfg["num_key_value_heads"], cfg["head_dim"]
+    for nl in (4, 2):
+        assert ops.batch_workspace_bytes(nl, P, H, H) >= 2 * nl * 20 * H * 4
+    assert ops.batch_workspace_bytes(4, P, 2 * hkv * d, H) >= 2 * 4 * 20 * 2 * hkv * d * 4
+    late = list(range(split, L))
+    Wl, Bl = _maps(H, late, 45)
+    W, B = dict(zip(late, Wl)), dict(zip(late, Bl))
+    h = inputs(P + tail, H, seed=46).to(dev)
+    m = FillModel(cfg, t, dev)
+    cache, got_p = fill_late(m, h, Arm("ridgefill", split=split, tail=tail, fill="proj", projector=Projector(split, W, B)))
+    torch.cuda.synchronize()
+    assert got_p == P
+    cs = m.rope_table(torch.arange(P, device=dev))
+    for i in late:
+        x, s = ops.map_apply(h[:P], W[i].to(dev), B[i].to(dev))
+        w = m.W[i]
+        kb = torch.zeros(hkv, P + 64, d, dtype=torch.bfloat16, device=dev)
+        vb = kb.clone()
+        ops.norm_kv_write(x, s, m.eps, w["wkv"], m.n_kv, m.head_dim, w.get("k_norm"), m.knorm_kind, cs, kb, vb, 0)
+        for got, want in ((cache[i]["k"], kb), (cache[i]["v"], vb)):
+            assert torch.equal(got[:, :whole], want[:, :whole]), f"layer {i}"
+            _near(got[:, whole:P], want[:, whole:P])
+
+
+def test_fill_late_hybrid_with_rows_left_over(dev):
+    """The hybrid's grouped schedule with rows left over in its map launch and in the GDN pairs' in-projections, which
+    share the call's workspace: the attention layer's K / V as above; a GDN layer's states sum over all rows, of which
+    the last 30 carry the changed roundings: 1e-3 of their norm."""
+    from fill_cases import hybrid_config, hybrid_tensors
+    from rfill import ops
+    from rfill.kva import Arm, Projector, fill_late
+    from rfill.model import FillModel
+    kinds = ["gdn", "gdn", "gdn", "attn", "gdn", "gdn"]
+    cfg = hybrid_config(kinds, hidden=1024)
+    H, tail, whole = cfg["hidden_size"], 100, 32 * 256
+    P = whole + 30
+    late = list(range(len(kinds)))
+    Wl, Bl = _maps(H, late, 50)
+    W, B = dict(zip(late, Wl)), dict(zip(late, Bl))
+    h = inputs(P + tail, H, seed=51).to(dev)
+    m = FillModel(cfg, hybrid_tensors(cfg, seed=52), dev)
+    m._layer(0, "gdn")
+    n_in = m.W[0]["w_in"].shape[0] - m.nk * m.dk
+    assert ops.batch_workspace_bytes(len(kinds), P, H, H) > 0
+    assert ops.norm_linear_batch_workspace_bytes([P, 3, P, 3], [n_in, m.nk * m.dk] * 2, H) > 0
+    cache, _ = fill_late(m, h, Arm("ridgefill", split=0, tail=tail, fill="proj", projector=Projector(0, W, B)))
+    torch.cuda.synchronize()
+    ref, pos = m.new_cache(), torch.arange(P, device=dev)
+    for i in late:
+        x, s = ops.map_apply(h[:P], W[i].to(dev), B[i].to(dev))
+        if kinds[i] == "attn":
+            w = m.W[i]
+            kb = torch.zeros(m.n_kv, P + 64, m.head_dim, dtype=torch.bfloat16, device=dev)
+            vb = kb.clone()
+            ops.norm_kv_write(x, s, m.eps, w["wkv"], m.n_kv, m.head_dim, w.get("k_norm"), m.knorm_kind,
+                              m.rope_table(pos), kb, vb, 0)
+            _near(cache[i]["k"][:, :P], kb[:, :P])
+            _near(cache[i]["v"][:, :P], vb[:, :P])
+        else:
+            m.fill(i, x, pos, ref, ssq=s)
+            for part in ("conv", "rec"):
+                assert rel_err(cache[i][part], ref[i][part]) < 1e-3, f"layer {i}: {part}"
+
+
+@pytest.mark.parametrize("small", [1, 161, 200, 256])
+def test_norm_linear_batch_small_entry_taller_than_the_rows_left(dev, small):
+    """A small entry (at most 256 rows, all of them as few rows) beside 30 rows left over by the large one: its row
+    blocks are taller than the plan's, one or two of them."""
+    from rfill import ops
+    P, H, n = 32 * 256 + 30, 1024, 2048
+    g = torch.Generator().manual_seed(small)
+    x = inputs(P, H, seed=53).to(dev)
+    ssq = ops.row_ssq(x)
+    w = [(torch.randn(k, H, generator=g) / H ** 0.5).to(torch.bfloat16).to(dev) for k in (n, 512)]
+    need = ops.norm_linear_batch_workspace_bytes([P, small], [n, 512], H)
+    assert need > 0 and need % (30 * n * 4 + small * 512 * 4) == 0
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    outs = [[torch.full((P + 1, n), 3.0, dtype=torch.bfloat16, device=dev) for _ in range(2)] for _ in range(2)]
+    for o, space in zip(outs, (ws, None)):
+        ops.norm_linear_batch([x, x[:small]], [ssq, ssq[:small]], 1e-6, w, [o[0][:P], o[1][:small, :512]], space)
+    torch.cuda.synchronize()
+    (a, b), (ra, rb) = outs
+    assert torch.equal(a[:32 * 256], ra[:32 * 256])
+    _near(a[32 * 256:P], ra[32 * 256:P])
+    _near(b[:small, :512], rb[:small, :512])
+    assert bool((a[P:] == 3.0).all()) and bool((b[small:] == 3.0).all()) and bool((b[:small, 512:] == 3.0).all())
