@@ -390,3 +390,11 @@ def test_centring_past_its_cap(dev, cols, cap):
     for name in ("c", "shift", "lo_row", "idx", "delta"):
         assert torch.equal(getattr(got, name).cpu(), getattr(want, name)), name
     assert took < 5e-3
+
+
+@pytest.mark.parametrize("init", [False, True])
+@pytest.mark.parametrize("da,ea,db,eb,K,upper", [(256, 130, 256, 160, 1088, False), (512, 160, 512, 160, 640, True),
+                                                 (256, 132, 256, 2, 2048, False)])
+def test_gram_centred_with_one_tall_row_block(dev, da, ea, db, eb, K, upper, init):
+    """130 to 160 extra rows (their count is even): one row block of five row tiles."""
+    test_gram_centred_is_the_augmented_product(dev, da, ea, db, eb, K, 512, upper, init)
