@@ -551,3 +551,29 @@ def test_row_statistics_at_any_alignment(dev, H):
         assert s.data_ptr() % 16 == 4 * off
         for a, b in zip(run(s), want):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("hq,hkv,d,nq,n", [(16, 2, 256, 300, 9000), (16, 2, 256, 37, 20000), (4, 2, 64, 500, 9000),
+                                           (8, 1, 128, 64, 8000), (2, 2, 256, 16, 12000), (24, 6, 128, 90, 6000)])
+def test_split_queries_at_positions_over_few_head_blocks(dev, hq, hkv, d, nq, n):
+    """Scattered queries with fewer than eight head blocks (2, 1, 2 and 6 of them): several XCDs share a head block and
+    take its splits interleaved. Every split count from the plan's down (a smaller workspace gives fewer splits, also
+    counts that the XCDs do not share evenly) against one pass: fp32 sums in another order before one bf16 rounding of
+    the probabilities' product (4e-3 of the norm, as above)."""
+    from rfill import ops
+    g = torch.Generator().manual_seed(nq + n)
+    q = torch.randn(nq, hq * d, generator=g).to(torch.bfloat16).to(dev)
+    kb, vb = (torch.randn(hkv, n + 3, d, generator=g).to(torch.bfloat16).to(dev) for _ in range(2))
+    qpos = torch.randperm(n, generator=g)[:nq].sort().values
+    qpos[0] = 0
+    qpos = qpos.to(dev)
+    need = ops.attend_causal_workspace_bytes(nq, hq, hkv, d, n, scattered=True)
+    one = ops.attend_causal(q, 0, kb, vb, n, hq, d ** -0.5, qpos=qpos, workspace=torch.empty(16, dtype=torch.uint8, device=dev))
+    unit = 256 * (d + 2) * 4                            # one block's partials
+    blocks = -(-nq // (256 // min(hq // hkv, 8))) * (hq // min(hq // hkv, 8))
+    ns = need // (unit * blocks)
+    assert need == ns * unit * blocks and ns > 2
+    for k in sorted({ns, ns - 1, 7, 5, 3, 2} & set(range(2, ns + 1))):
+        ws = torch.full((k * unit * blocks,), 0xFF, dtype=torch.uint8, device=dev)
+        got = ops.attend_causal(q, 0, kb, vb, n, hq, d ** -0.5, qpos=qpos, workspace=ws)
+        assert rel_err(got, one) < 4e-3, k
