@@ -203,3 +203,25 @@ def test_fill_checkpoints(dev):
     assert torch.equal(mc[0]["rec"], plain[0]["rec"]) and torch.equal(mc[0]["conv"], plain[0]["conv"])
     with pytest.raises(ValueError, match="multiple"):
         m.fill(0, x[:64].to(dev), torch.arange(64, device=dev), m.new_cache(), checkpoint_every=100)
+
+
+@pytest.mark.parametrize("off,pad", [(1, 0), (2, 8), (4, 8)])
+def test_forward_outputs_at_any_alignment(dev, off, pad):
+    """The delta rule's outputs 2, 4 and 8 bytes past a 16-byte boundary (the stores of 8 bytes need the last), in rows
+    as long as the outputs or longer: the aligned call's bits, and nothing beside them written."""
+    from rfill import ops
+    cfg = gdn_config()
+    om = OM.OracleModel(cfg, gdn_tensors(cfg, seed=8), dtype=torch.bfloat16)
+    P, n = 150, 4 * 128
+    rows = _pre_rows(om, inputs(P, cfg["hidden_size"], seed=26)).to(dev)
+    w = om.W[0]
+    args = (w["conv"].to(dev).contiguous(), None, w["A_log"].to(dev), w["dt_bias"].to(dev))
+    state = [torch.zeros(4, 128, 128, dtype=torch.float32, device=dev) for _ in range(2)]
+    want, _ = ops.gdn_forward(rows, 2, 4, 128, 128, *args, state[0])
+    buf = torch.full((off + P * (n + pad) + 8,), 3.0, dtype=torch.bfloat16, device=dev)
+    out = buf[off:off + P * (n + pad)].view(P, n + pad)[:, :n]
+    ops.gdn_forward(rows, 2, 4, 128, 128, *args, state[1], out=out)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and torch.equal(state[0], state[1])
+    assert bool((buf[:off] == 3.0).all()) and bool((buf[off + P * (n + pad):] == 3.0).all())
+    assert bool((buf[off:off + P * (n + pad)].view(P, n + pad)[:, n:] == 3.0).all())
