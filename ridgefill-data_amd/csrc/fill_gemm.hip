@@ -2085,10 +2085,18 @@ int split_count(int64_t M, int64_t N, int64_t K) {
 
 // How a batched launch of nl products, each M x N x K, runs: rows [0, m_fused) of every entry as 256 x 256 tiles,
 // the rest (at most BATCH_ROWS rows, rblocks row blocks of at most 160 each) as products of few rows with K split
-// `splits` ways. A round of tiles on the 256 CUs costs the same whether all of them have one or only a few do, and a
-// tile row is a whole one however few of its rows exist; the few-rows products cost what their rows do. The times
-// compared, in us (measured at K 2048 and 4096): a round 1.45 per 64-deep step + 8; a round of few-rows blocks
-// 0.55 + 0.1 per 32 rows a step + 4, 6 for the second launch, and the split planes written and read at 4 TB/s.
+// `splits` ways. A round of tiles on the 256 CUs costs about the same whether all of them have one or only a few do,
+// and a tile row is a whole one however few of its rows exist; the few-rows products cost what their rows do.
+// The times compared (us; steps of K / 64; fitted to 800 shapes of maps, norm + linear and K / V launches, K 1024 to
+// 4096, 100 to 9000 rows, 2 to 24 thousand columns in all, each as tiles and with up to five row counts split off):
+//   tiles: 10 to launch; a full round 1.16 a step + 6; a last round of at most 128 tiles 0.96 a step + 4 (fewer CUs
+//     clock higher), linearly more up to a full one's; a round more by 2 for norm + linear, and by 18 for the row
+//     pass of K / V (from 16 column blocks on half of that past the first: a block's tiles are K and V columns by turns).
+//   rows: a round of blocks 0.65 a step of its split + 7, and 0.08 a step, row tile and 256 blocks; 2 for the second
+//     launch; the split planes written and read 0.072 a MB; K / V's row pass 0.1 a MB of one plane written and read.
+// The choice takes 0.2 % more than the best of the measured ones on average. A round at 1.45 a step + 8 however few its
+// tiles, as it was priced before, took few rows too often: 769 x 24576 x 4096 178 us, now 159 as tiles; maps of three
+// layers of 2000 rows at 4096 197, now 172; and for K / V launches, whose rounds it took for cheaper, not often enough.
 // 6160 rows of four 8B layers: the 64 map tiles (32 K / V tiles) that held the last 16 rows took a seventh (fourth)
 // round, 743 (507) us in all; now 685 (401) for whole rounds and 32 (22) for the rows, product and epilogue.
 struct BatchPlan {
@@ -2098,31 +2106,49 @@ struct BatchPlan {
 };
 constexpr int64_t BATCH_ROWS = 1024;
 
+// What an epilogue adds to the map's: us a round of tiles (or two rounds, by turns), and us a MB of one plane of few
+// rows.
+struct Epilogue {
+  double round, plane;
+  bool turns;
+};
+constexpr Epilogue EP_MAP{0, 0, false}, EP_LINEAR{2, 0, false};
+Epilogue ep_kv(int64_t N) { return Epilogue{18, 0.1, N >= 16 * BN}; }
+
+// us of `tiles` tiles of K, without the launch.
+double tiles_us(int64_t tiles, int64_t K, const Epilogue& e) {
+  const double steps = static_cast<double>(K / BK), full = 1.16 * steps + 6, part = 0.96 * steps + 4;
+  const int64_t last = tiles % 256, rounds = (tiles + 255) / 256;
+  const double fill = std::max(0.0, (last - 128) / 128.0);
+  return tiles / 256 * full + (last ? part + (full - part) * fill : 0) +
+         (e.turns && rounds ? std::max<int64_t>(rounds, 2) * 0.5 : static_cast<double>(rounds)) * e.round;
+}
+constexpr double LAUNCH_US = 10;
+
 struct RowShape {
   int splits, rt, rblocks;
   double us;
 };
 // cblocks: the column blocks of every entry together, for m rows each.
-RowShape batch_rows_shape(int64_t cblocks, int64_t m, int64_t K) {
+RowShape batch_rows_shape(int64_t cblocks, int64_t m, int64_t K, const Epilogue& e) {
   const int64_t rb = (m + 159) / 160, rt = ((m + rb - 1) / rb + 31) / 32, blocks = rb * cblocks;
   const int64_t s = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / blocks, K / 512), 16));
   const double rounds = static_cast<double>((blocks * s + 255) / 256), steps = static_cast<double>(K / BK) / s;
-  const double planes = static_cast<double>(cblocks) * RN * m * 4 * 2 * s;
+  const double plane = static_cast<double>(cblocks) * RN * m * 4 * 2 * 1e-6;
   return RowShape{static_cast<int>(s), static_cast<int>(rt), static_cast<int>(rb),
-                  rounds * (steps * (0.55 + 0.1 * rt) + 4) + 6 + planes / 4e6};
+                  rounds * (0.65 * steps + 7) + 0.08 * steps * rt * blocks * s / 256 + 2 + 0.072 * plane * s +
+                      e.plane * plane};
 }
 
-BatchPlan batch_plan(int64_t cblocks, int64_t M, int64_t K) {
+BatchPlan batch_plan(int64_t cblocks, int64_t M, int64_t K, const Epilogue& e) {
   BatchPlan best;
   best.m_fused = M;
   if (K < 1024 || M <= 0) return best;
-  const double round = 1.45 * static_cast<double>(K / BK) + 8;
-  auto rounds = [&](int64_t trows) { return static_cast<double>((trows * cblocks + 255) / 256); };
   const int64_t trows = (M + BM - 1) / BM;
-  double cost = rounds(trows) * round - 5;           // 5 us: what a plan has to gain at least
+  double cost = tiles_us(trows * cblocks, K, e) - 3.6;      // what a plan has to gain at least
   for (int64_t fr = trows - 1; fr >= 0 && M - fr * BM <= BATCH_ROWS; --fr) {
-    const RowShape r = batch_rows_shape(cblocks, M - fr * BM, K);
-    const double c = rounds(fr) * round + r.us;
+    const RowShape r = batch_rows_shape(cblocks, M - fr * BM, K, e);
+    const double c = tiles_us(fr * cblocks, K, e) + r.us;
     if (c < cost) {
       cost = c;
       best = BatchPlan{fr * BM, r.splits, r.rt, r.rblocks};
@@ -2137,8 +2163,8 @@ BatchPlan batch_plan(int64_t cblocks, int64_t M, int64_t K) {
 // most half full, its tile rows are split, so that wave takes a fraction of a tile's time.
 // Products of at most ROWS_MAX rows take k_rows_partial (rt row tiles per row block, rblocks row blocks)
 // for every row, split so that about one block runs per CU, then the reduce epilogue. So do the last rows of other
-// widths where batch_plan says so: 1499 x 12288 x 2048 (288 tiles) 102 us in two rounds, 93 as one
-// round and 219 rows.
+// widths where batch_plan says so (with the map's epilogue, the cheapest): 1499 x 12288 x 2048 (288 tiles) 102 us in
+// two rounds, 93 as one round and 219 rows.
 struct Plan {
   int64_t m_fused;
   int splits;
@@ -2168,7 +2194,7 @@ Plan plan(int64_t M, int64_t N, int64_t K) {
     return Plan{M, 1};
   }
   // tile rows that do not divide a round: the rows past the whole rounds as products of few rows, where that is less
-  const BatchPlan b = batch_plan(tiles_n, M, K);
+  const BatchPlan b = batch_plan(tiles_n, M, K, EP_MAP);
   return b.rows() ? Plan{b.m_fused, b.splits, b.rt, b.rblocks} : Plan{M, 1};
 }
 
@@ -2223,16 +2249,23 @@ void launch_partials(const uint16_t* X, int64_t ldx, const uint16_t* W, int64_t 
 // Three layers of 1792 x 256 x 256: 93 us as three launches of 7 tiles, 18 as one product and one epilogue launch.
 bool small_kv(int64_t nl, int64_t M, int64_t N, int64_t K, RowShape* r) {
   if (K >= 1024 || M <= 0 || M > 4096) return false;
-  *r = batch_rows_shape(nl * (N / BN), M, K);
+  *r = batch_rows_shape(nl * (N / BN), M, K, ep_kv(N));
   const double tiles = static_cast<double>(nl) * ((grid_of(M, N) + 255) / 256) * (1.45 * (K / BK) + 25);
-  return r->splits == 1 && r->us < tiles;
+  return r->splits == 1 && LAUNCH_US + r->us < tiles;
 }
 
+// Bytes of the split planes of nl entries under plan p.
+size_t batch_planes(int64_t nl, const BatchPlan& p, int64_t M, int64_t N) {
+  return p.rows() ? static_cast<size_t>(nl) * p.splits * (M - p.m_fused) * N * 4 : 0;
+}
+
+// What the map or the K / V launch of this shape asks for, whichever is more.
 size_t batch_bytes(int64_t nl, int64_t M, int64_t N, int64_t K) {
   RowShape r{};
   if (small_kv(nl, M, N, K, &r)) return static_cast<size_t>(nl) * M * N * 4;
-  const BatchPlan p = batch_plan(nl * (N / BN), M, K);
-  return p.rows() ? static_cast<size_t>(nl) * p.splits * (M - p.m_fused) * N * 4 : 0;
+  const int64_t cb = nl * (N / BN);
+  return std::max(batch_planes(nl, batch_plan(cb, M, K, EP_MAP), M, N),
+                  batch_planes(nl, batch_plan(cb, M, K, ep_kv(N)), M, N));
 }
 
 // The few-rows products of `nl` entries filled into j (x, w, m, n): block and plane offsets, then one launch.
@@ -2272,7 +2305,7 @@ BatchPlan lin_plan(int nl, const int64_t* rows, const int64_t* n, int64_t H, int
     cb += n[l] / BN;
   }
   *m_large = M;
-  return M && persistent_lin_ok(H) ? batch_plan(cb, M, H) : BatchPlan{M};
+  return M && persistent_lin_ok(H) ? batch_plan(cb, M, H, EP_LINEAR) : BatchPlan{M};
 }
 
 size_t lin_bytes(int nl, const int64_t* rows, const int64_t* n, int64_t H) {
@@ -2979,8 +3012,8 @@ extern "C" int rf_map_apply_batch_ws(int nl, const uint16_t* b, int64_t ldb, con
   if (!aligned16(b)) return fail(RF_EINVAL_SHAPE, "rf_map_apply_batch: b must be 16-byte aligned");
   if (workspace && !aligned16(workspace)) return fail(RF_EINVAL_SHAPE, "rf_map_apply_batch: workspace alignment");
   if (P == 0) return RF_OK;
-  BatchPlan pl = batch_plan(nl * (h_out / BN), P, h_in);
-  if (pl.rows() && (!workspace || ws_bytes < batch_bytes(nl, P, h_out, h_in))) pl = BatchPlan{P};
+  BatchPlan pl = batch_plan(nl * (h_out / BN), P, h_in, EP_MAP);
+  if (pl.rows() && (!workspace || ws_bytes < batch_planes(nl, pl, P, h_out))) pl = BatchPlan{P};
   const int64_t mf = pl.m_fused;
   if (mf > 0)
     hipLaunchKernelGGL(k_map_apply_p<false>, dim3(persistent_grid(nl * static_cast<int64_t>(grid_of(mf, h_out)))),
@@ -3066,8 +3099,9 @@ extern "C" int rf_norm_kv_write_batch_ws(int nl, const uint16_t* const* x, int64
   const bool tiled = persistent_kv_ok(H, rot, P);
   const bool small = !tiled && workspace && ws_bytes >= batch_bytes(nl, P, N, H) && small_kv(nl, P, N, H, &few);
   if (tiled || small) {
-    BatchPlan pl = small ? BatchPlan{0, few.splits, few.rt, few.rblocks} : batch_plan(nl * (N / BN), P, H);
-    if (pl.rows() && !small && (!workspace || ws_bytes < batch_bytes(nl, P, N, H))) pl = BatchPlan{P};
+    BatchPlan pl = small ? BatchPlan{0, few.splits, few.rt, few.rblocks}
+                         : batch_plan(nl * (N / BN), P, H, ep_kv(N));
+    if (pl.rows() && !small && (!workspace || ws_bytes < batch_planes(nl, pl, P, N))) pl = BatchPlan{P};
     const int64_t mf = pl.m_fused;
     if (mf > 0) launch_norm_kv_p(kl, nl, ldx, mf, N, H, a, stream);
     if (pl.rows()) {

@@ -175,3 +175,14 @@ def test_prompts_from_slot_0_are_not_split(hq, hkv, d):
     assert ops.attend_causal_workspace_bytes(4096, hq, hkv, d, 8192, 4096) == 0
     assert ops.attend_causal_workspace_bytes(300, hq, hkv, d, 28672, 28372) > 0
     assert ops.attend_causal_workspace_bytes(300, hq, hkv, d, 28672, scattered=True) > 0
+
+
+def test_rows_left_over_only_where_they_gain():
+    """Host-only plans of the rows past whole rounds of tiles: few rows past a round run apart; a last round that is half
+    full, whose tiles run faster than a full one's, is left as it is."""
+    from rfill import ops
+    assert ops.gemm_workspace_bytes(1499, 12288, 2048) > 0                  # 240 tiles and 219 rows
+    assert ops.batch_workspace_bytes(4, 6160, 4096, 4096) > 0               # six rounds and 16 rows
+    assert ops.gemm_workspace_bytes(1600, 12288, 4096) > 0                  # 240 tiles and 320 rows: 152 us against 166
+    for M, N in ((769, 24576), (2000, 12288)):                              # 384 tiles: 160, 171 us against 186, 193
+        assert ops.gemm_workspace_bytes(M, N, 4096) == 0
