@@ -291,17 +291,6 @@ __device__ __forceinline__ void tile_step(const char* __restrict__ st, const cha
   }
 }
 
-// The key split that the at-th column of query blocks of a head block takes. With fewer than 8 head blocks several
-// XCDs share one: each takes every xcds-th of its splits (class by class), so that the splits past the early queries,
-// which end at once, are spread over them instead of idling the last.
-__host__ __device__ __forceinline__ int split_of(int at, int ns, int head_blocks) {
-  const int xcds = head_blocks < 8 ? 8 / head_blocks : 1;
-  if (xcds == 1 || ns <= xcds) return at;
-  const int per = ns / xcds, more = ns % xcds, cut = more * (per + 1);
-  const int cls = at < cut ? at / (per + 1) : more + (at - cut) / per;
-  return (at < cut ? at - cls * (per + 1) : (at - cut) - (cls - more) * per) * xcds + cls;
-}
-
 template <int AD>
 __global__ __launch_bounds__(Cfg<AD>::NTHR, 1) void k_attend_causal(CausalArgs a) {
   using L = Layout<AD>;
@@ -317,7 +306,16 @@ __global__ __launch_bounds__(Cfg<AD>::NTHR, 1) void k_attend_causal(CausalArgs a
   const int qbs = gridDim.x, ns = gridDim.z;
   const int u = xcd_tile(blockIdx.x + qbs * (blockIdx.y + gridDim.y * blockIdx.z), qbs * gridDim.y * ns);
   const int qb = u % qbs, hb = u / (qbs * ns);
-  const int sp = split_of((u / qbs) % ns, ns, static_cast<int>(gridDim.y));
+  // With fewer than 8 head blocks several XCDs share one: each takes every xcds-th of its splits (class by class),
+  // so that the splits past the early queries, which end at once, are spread over them instead of idling the last.
+  const int xcds = gridDim.y < 8 ? 8 / static_cast<int>(gridDim.y) : 1;
+  int sp = (u / qbs) % ns;
+  if (xcds > 1 && ns > xcds) {
+    const int per = ns / xcds, more = ns % xcds, cut = more * (per + 1);
+    const int cls = sp < cut ? sp / (per + 1) : more + (sp - cut) / per;
+    const int at = sp < cut ? sp - cls * (per + 1) : (sp - cut) - (cls - more) * per;
+    sp = at * xcds + cls;
+  }
   const int hk = hb / (rep / a.hpb), hoff = (hb % (rep / a.hpb)) * a.hpb;
   const int j0 = qb * qp;
   const int jlast = min(j0 + qp, a.nq) - 1;
@@ -602,6 +600,16 @@ struct PlanBlocks {
   int tiles[PLAN_BLOCKS];                  // of query block qb, not falling
   int64_t sum[PLAN_BLOCKS + 1];            // of the query blocks before qb
 };
+
+// The split that the at-th column of query blocks of a head block takes, as k_attend_causal maps them. (Shared with the
+// kernel, this compiles to another loop head there, 0.5 to 1 % slower.)
+int split_of(int at, int ns, int head_blocks) {
+  const int xcds = head_blocks < 8 ? 8 / head_blocks : 1;
+  if (xcds == 1 || ns <= xcds) return at;
+  const int per = ns / xcds, more = ns % xcds, cut = more * (per + 1);
+  const int cls = at < cut ? at / (per + 1) : more + (at - cut) / per;
+  return (at < cut ? at - cls * (per + 1) : (at - cut) - (cls - more) * per) * xcds + cls;
+}
 
 struct PlanLoad {
   int64_t live = 0, work = 0;              // blocks that run, their tiles
