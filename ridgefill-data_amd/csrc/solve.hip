@@ -15,12 +15,12 @@
 //   the inverse   of an n x n SPD matrix (n a multiple of 128, its lower triangle) by block recursion on
 //                 [A11 .; A21 A22]: X11 = A11^-1, T = A21 X11, S = A22 - T A21^T (the Schur complement, SPD),
 //                 X22 = S^-1, X21 = -X22 T, X11 -= T^T X21, X12 = X21^T. Symmetric results are computed on their
-//                 lower tiles only; the product that forms X21 stores X12 too. d 4096, three lambdas: 8.0 ms for
-//                 the inverses (19.7 with 64 x 64 leaves, every product in full and separate copies and
-//                 transposes), one lambda 4.5 (15.8), d 1024 0.7 (3.1).
+//                 lower tiles only; the product that forms X21 stores X12 too. d 4096, three lambdas: 6.7 ms of
+//                 kernels for the inverses (18.6 with 64 x 64 leaves, every product in full and separate copies and
+//                 transposes), one lambda 4.0 (15.2), d 1024 0.65 (2.9).
 //   k_gemv_rows   out = init + alpha v M, rows summed by 4 waves in order (the bias's vector products).
 //   rf_ridge_solve  per lambda: A = C + lam s I padded to a multiple of 128 with an identity block, X = A^-1,
-//                 W = X[:d, :d] Cxy (k_dgemm, or k_solve_wt's W^T; the dominant 2 d^2 R flops, 26.6 ms for four
+//                 W = X[:d, :d] Cxy (k_dgemm, or k_solve_wt's W^T; the dominant 2 d^2 R flops, 26.4 ms for four
 //                 targets of 4096 and three lambdas, 79 % of the fp64 MFMA peak), bias = mean_y - (mean_x X) Cxy
 //                 (= mean_y - mean_x W; one pass over Cxy for every lambda). Up to 8 lambdas go together:
 //                 every launch of the recursion carries all of them in its grid.

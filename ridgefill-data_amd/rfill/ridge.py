@@ -3,17 +3,17 @@ statistics accumulated by librfill's MFMA Gram kernel.
 
 begin(x) / add_layer(i, y) (code/kva/ridge.py:34-62): up to PIECE rows at a time are transposed into the
 K-contiguous operands X^T, Y_i^T (rf_transpose_centred, which also yields the column sums), then one
-rf_gram_accumulate launch per operand pair adds X^T X or X^T Y_i: bf16 products summed in fp32 over runs of
-at most `block` rows (default 8192, the reference's block), each run added into fp64 -- as the reference's
-per-block fp32 GEMM (code/kva/ridge.py:47, :62) is. X^T is built once per piece and serves every layer.
+rf_gram_centred call per operand pair adds X^T X (its block-upper tiles) or X^T Y_i: bf16 products summed in
+fp32 over runs of at most `block` rows (default 8192, the reference's block), each run added into fp64 -- as the
+reference's per-block fp32 GEMM (code/kva/ridge.py:47, :62) is. X^T is built once per piece and serves every layer.
 
 Centring. The reference subtracts its shifts (the first block's means, code/kva/ridge.py:37-38, :56-57)
 before each block's fp32 GEMM, which keeps the fp32 sums at the size of the centred values. Here the
 channels whose first-block mean exceeds their spread (mean^2 > variance; at most SHIFT_MAX per operand,
 largest ratio first) are centred in the transpose: their fp32 values x - shift go into the operand as three
-bf16 rows whose sum is exact (hi in the main rows; mid and lo in the rows after them). One Gram product over
-[main rows; mid and lo rows] then carries every centred product. The other channels, whose
-raw sums are at most twice their centred size, are summed raw. state() combines the lo rows' products in
+bf16 rows whose sum is exact (hi in the main rows; mid and lo in the rows after them). The Gram product over
+[main rows; mid and lo rows], the extra rows as products of few rows, then carries every centred product. The
+other channels, whose raw sums are at most twice their centred size, are summed raw. state() combines the lo rows' products in
 fp64 and moves every sum onto the reference's shifts by exact fp64 algebra, so the state dict has the
 reference's layout and meaning.
 
