@@ -1,6 +1,6 @@
 """GPU parity of the closed-form fit at the 8B width of the fit configuration (d 4096, 16 targets,
 Student-t(5) rows with 4 outlier channels x 20, Y_l = X T_l + N(0, 0.1), bf16 storage): the device's
-sufficient statistics against fp64 products of the same bf16 rows (torch fp64 on the GPU, the checker), and
+sufficient statistics against fp64 products of the same bf16 rows (torch fp64 on the GPU, the oracle), and
 the maps RidgeFit solves from them against the oracle's fp64 eigendecomposition solve (code/kva/ridge.py:
 80-105) of those fp64 statistics, at lambda in {1e-4, 1e-3, 1e-2} x mean(diag C). A second workload adds 8
 channels whose mean is 60x their spread (real hidden states carry such channels): the transpose centres them

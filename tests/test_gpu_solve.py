@@ -1,6 +1,6 @@
 """GPU parity of the ridge solve (rf_ridge_solve: the inverse of C + lam s I by block recursion on Schur
 complements over a 128 x 128 Gauss-Jordan base, fp64 MFMA products) against torch.linalg.solve in fp64 on the
-same device (the checker), for sizes on and off the 128-multiple grid (the padded identity block), several
+same device (the oracle), for sizes on and off the 128-multiple grid (the padded identity block), several
 right-hand-side widths and lambdas, and the bias mean_y - mean_x W. Bar: 1e-10 relative Frobenius (fp64
 arithmetic on matrices of condition number up to ~1e4)."""
 import pytest
